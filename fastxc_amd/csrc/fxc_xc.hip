@@ -12,7 +12,8 @@
 // each workgroup computes one tile for 16 consecutive bins, reading every
 // station spectrum once per tile instead of once per pair-window.  Three
 // arithmetic forms share the tiling:
-//   FP32    plain fp32 FMA on the vector ALU (the parity path);
+//   FP32    fp32 products and sums on the fp32 matrix instructions (the parity
+//           path);
 //   BF16X3  spectra split into bf16 hi+lo, three MFMA products
 //           (hi*hi + hi*lo + lo*hi) with fp32 accumulation;
 //   FP16    one fp16 MFMA product with a power-of-two scale per station;
@@ -229,11 +230,13 @@ split_segments_kernel(const float2 *__restrict__ spec, const unsigned char *__re
 // ---------------------------------------------------------------------------
 // Tile descriptors: tile t covers src stations [src_base, +32) and rec
 // stations [rec_base, +32); rows[t][i][j] is the workspace row of pair
-// (src_base+i, rec_base+j) or -1.
+// (src_base+i, rec_base+j) or -1.  Bit 2 si + sj of blocks: some pair of the
+// 16 x 16 block (source half si, receiver half sj) is listed.
 // ---------------------------------------------------------------------------
 struct TileDesc {
   int src_base;
   int rec_base;
+  int blocks;
 };
 
 // Streaming store of one complex value: the cross-spectra are written once
@@ -251,105 +254,38 @@ __device__ __forceinline__ void store_stream2(float2 *dst, float2 a, float2 b) {
   __builtin_nontemporal_store(v, (u64x2 *)dst);
 }
 
-// Work item -> (tile, bin chunk) of the FP32 contraction.  Workgroups are
-// dispatched round-robin over the 8 XCDs, so 8 consecutive items take 8
-// consecutive bin chunks of one tile: each XCD's L2 then serves one chunk of
-// every station's spectra, and each pair row receives 8 x 128 contiguous
-// bytes at once.  (The MFMA contraction keeps the same chunk-per-XCD rule
-// with its own order of tiles; see contract_mfma_kernel.)
+// Bin chunks are taken in groups of 8, one per XCD (see ItemWalk).
 constexpr int kChunkGroup = 8;
 
-__device__ __forceinline__ bool tile_chunk_of(long long item, int ntiles, int nchunks, int &tile,
-                                              int &chunk) {
-  const long long per_group = (long long)ntiles * kChunkGroup;
-  const int g = (int)(item / per_group);
-  const int r = (int)(item - g * per_group);
-  tile = r / kChunkGroup;
-  chunk = g * kChunkGroup + (r - tile * kChunkGroup);
-  return chunk < nchunks;
-}
-__device__ __forceinline__ bool tile_chunk(int ntiles, int nchunks, int &tile, int &chunk) {
-  return tile_chunk_of(blockIdx.x, ntiles, nchunks, tile, chunk);
-}
-
-// FP32 contraction: thread = (bin, 8x8 micro-tile of pairs).
-__global__ void __launch_bounds__(256)
-contract_fp32_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int nspec,
-                     const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
-                     float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
-                     int chunk0, int nchunks) {
-  __shared__ int rows[kTilePairs];
-  __shared__ int active[16];
-  int tile, chunk;
-  if (!tile_chunk(ntiles, nchunks, tile, chunk)) return;
-  chunk += chunk0;
-  const int tid = threadIdx.x;
-  const int *trow = tile_rows + (size_t)tile * kTilePairs;
-  for (int i = tid; i < kTilePairs; i += blockDim.x) rows[i] = trow[i];
-  if (tid < 16) active[tid] = 0;
-  __syncthreads();
-  for (int i = tid; i < kTilePairs; i += blockDim.x) {
-    if (rows[i] >= 0) {
-      const int mi = (i >> 5) >> 3, mj = (i & 31) >> 3;
-      active[mi * 4 + mj] = 1;
+// Item order of the persistent contractions.  Workgroups are dispatched
+// round-robin over the 8 XCDs, so workgroup w runs on XCD x = w mod 8 and
+// takes chunks 8 g + x only: each XCD's L2 then serves one chunk of every
+// station's spectra at a time.  Within an XCD's stream j = 0, 1, ... (tile
+// j mod ntiles of chunk group j / ntiles) the U = gridDim.x / 8 workgroups of
+// the XCD take runs of kRun consecutive j, so a workgroup's consecutive items
+// are mostly neighbouring tiles of one tile row at one chunk, which share
+// their source stations.  (gridDim.x is a multiple of 8.)
+struct ItemWalk {
+  static constexpr int kRun = 8;
+  int ntiles, nchunks, xcd, wu, nu;
+  long long nj;
+  __device__ __forceinline__ ItemWalk(int ntiles_, int nchunks_)
+      : ntiles(ntiles_), nchunks(nchunks_), xcd(blockIdx.x & 7), wu(blockIdx.x >> 3),
+        nu(gridDim.x >> 3),
+        nj((long long)ntiles_ * ((nchunks_ + kChunkGroup - 1) / kChunkGroup)) {}
+  // next valid item at or after this workgroup's k-th (items whose chunk is
+  // past the end are skipped); -1 when none is left
+  __device__ __forceinline__ long long next(long long k, int &tile, int &chunk) const {
+    for (;; ++k) {
+      const long long j = (k / kRun) * nu * kRun + (long long)wu * kRun + k % kRun;
+      if (j >= nj) return -1;
+      const long long g = j / ntiles;
+      tile = (int)(j - g * ntiles);
+      chunk = (int)(g * kChunkGroup) + xcd;
+      if (chunk < nchunks) return k;
     }
   }
-  __syncthreads();
-  const int b = tid & 15;
-  const int g = tid >> 4;
-  const int mi = g >> 2, mj = g & 3;
-  const int k = chunk * kBinChunk + b;
-  if (k >= nspec || !active[g]) return;
-  const TileDesc td = tiles[tile];
-  const int s0 = td.src_base + mi * 8;
-  const int r0 = td.rec_base + mj * 8;
-  float2 acc[8][8];
-#pragma unroll
-  for (int a = 0; a < 8; ++a)
-#pragma unroll
-    for (int c = 0; c < 8; ++c) acc[a][c] = make_float2(0.f, 0.f);
-  // software pipeline: loads of window w+1 are in flight while window w is
-  // accumulated
-  const size_t wstride = (size_t)nsta * nspec;
-  float2 sv[8], rv[8], sn[8], rn[8];
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
-    sv[a] = (s0 + a < nsta) ? spec[(size_t)(s0 + a) * nspec + k] : make_float2(0.f, 0.f);
-    rv[a] = (r0 + a < nsta) ? spec[(size_t)(r0 + a) * nspec + k] : make_float2(0.f, 0.f);
-  }
-  for (int w = 0; w < nstep; ++w) {
-    if (w + 1 < nstep) {
-      const float2 *base = spec + (size_t)(w + 1) * wstride + k;
-#pragma unroll
-      for (int a = 0; a < 8; ++a) {
-        sn[a] = (s0 + a < nsta) ? base[(size_t)(s0 + a) * nspec] : make_float2(0.f, 0.f);
-        rn[a] = (r0 + a < nsta) ? base[(size_t)(r0 + a) * nspec] : make_float2(0.f, 0.f);
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        // conj(s) * r
-        acc[a][c].x += sv[a].x * rv[c].x + sv[a].y * rv[c].y;
-        acc[a][c].y += sv[a].x * rv[c].y - sv[a].y * rv[c].x;
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      sv[a] = sn[a];
-      rv[a] = rn[a];
-    }
-  }
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int row = rows[(mi * 8 + a) * kTile + mj * 8 + c];
-      if (row >= 0) store_stream(xspec + (size_t)row * xpitch + k, cscale(acc[a][c], scale));
-    }
-  }
-}
+};
 
 // MFMA contraction.  Per bin: Cr = A.B1, Ci = A.B2 with a_s = [Re | Im] and
 // b2_s = [Im | -Re], so conj(a)*b = Cr + i Ci.  Results are staged in LDS as
@@ -474,6 +410,32 @@ __device__ __forceinline__ void mfma_bin(const SrcFrag<NK16> &x, const RecFrag<N
 // pairs, and a 16-thread group still reads one pair's 16 bins as a
 // permutation of one 128-byte row.
 __device__ __forceinline__ int stage_index(int p, int b) { return p * kBinChunk + (b ^ (p & 15)); }
+
+// The store phase of a contraction item: rows of the staged tile to the
+// workspace, 16 bins from k0.  8 consecutive threads write one pair's 16 bins
+// (128 bytes), two adjacent bins (16 bytes) each.  The swizzle keeps bins 2c
+// and 2c+1 in one 16-byte slot, (2c) ^ (p & 14), in swapped order when p is
+// odd.
+__device__ __forceinline__ void store_tile(const float2 *stage, const int *rows, int k0, int nspec,
+                                           float2 *__restrict__ xspec, long long xpitch) {
+  const int tid = threadIdx.x;
+  const int b = (tid & 7) * 2;
+  const int k = k0 + b;
+  if (k >= nspec) return;
+  for (int p = tid >> 3; p < kTilePairs; p += blockDim.x >> 3) {
+    const int row = rows[p];
+    if (row < 0) continue;
+    const float4 v = *(const float4 *)(stage + p * kBinChunk + (b ^ (p & 14)));
+    const bool sw = (p & 1) != 0;
+    const float2 v0 = sw ? make_float2(v.z, v.w) : make_float2(v.x, v.y);
+    const float2 v1 = sw ? make_float2(v.x, v.y) : make_float2(v.z, v.w);
+    float2 *dst = xspec + (size_t)row * xpitch + k;
+    if (k + 1 < nspec)
+      store_stream2(dst, v0, v1);
+    else
+      store_stream(dst, v0);
+  }
+}
 
 // Operands of one bin for the whole 32x32 tile: two 16-station source blocks
 // and two 16-station receiver blocks, hi (and lo for the split form).
@@ -700,8 +662,7 @@ __device__ __forceinline__ void compute_tile_bin_chunked(const unsigned short *_
 // One work item = one 32x32 station tile x 16 bins; 8 waves, each computing
 // the whole tile (four 16x16 MFMA blocks) for two of the 16 bins, so every
 // station fragment is read once per workgroup.  Persistent: a workgroup walks
-// runs of neighbouring tiles at one bin chunk (the order is set out at the
-// top of the kernel), and each wave keeps the source operands of its two
+// runs of neighbouring tiles at one bin chunk (ItemWalk), and each wave keeps the source operands of its two
 // bins in registers while consecutive tiles share their source stations.
 // With small K each wave software-pipelines its bins: the receiver operands
 // of the next bin -- of this item or of the next one -- are loaded before the
@@ -728,31 +689,9 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
   constexpr bool kPipe = NK16 * (kSplit ? 2 : 1) <= 8;
   constexpr int kBins = kBinChunk / 8;  // bins per wave and item
   static_assert(kBins == 2, "two bins per wave and item");
-  // Item order.  Workgroups are dispatched round-robin over the 8 XCDs, so
-  // workgroup w runs on XCD x = w mod 8 and takes chunks 8 g + x only: each
-  // XCD's L2 then serves one chunk of every station's spectra at a time.
-  // Within an XCD's stream j = 0, 1, ... (tile j mod ntiles of chunk group
-  // j / ntiles) the U = gridDim.x / 8 workgroups of the XCD take runs of
-  // kRun consecutive j, so a workgroup's consecutive items are mostly
-  // neighbouring tiles of one tile row at one chunk, which share their
-  // source stations.  (gridDim.x is a multiple of 8.)
-  constexpr int kRun = 8;
-  const int xcd = blockIdx.x & 7, wu = blockIdx.x >> 3, nu = gridDim.x >> 3;
-  const long long nj = (long long)ntiles * ((nchunks + kChunkGroup - 1) / kChunkGroup);
-  // next valid item at or after this workgroup's k-th (items whose chunk is
-  // past the end are skipped); -1 when none is left
-  auto next_item = [&](long long k, int &tile, int &chunk) -> long long {
-    for (;; ++k) {
-      const long long j = (k / kRun) * nu * kRun + (long long)wu * kRun + k % kRun;
-      if (j >= nj) return -1;
-      const long long g = j / ntiles;
-      tile = (int)(j - g * ntiles);
-      chunk = (int)(g * kChunkGroup) + xcd;
-      if (chunk < nchunks) return k;
-    }
-  };
+  const ItemWalk walk(ntiles, nchunks);
   int tile = 0, chunk = 0;
-  long long item = next_item(0, tile, chunk);
+  long long item = walk.next(0, tile, chunk);
   if (item < 0) return;
   ItemAddr ia;
   item_addr<kMode>(tiles[tile], chunk0 + chunk, nsta, lane_r, lane_g, scale, sta_scale, ia);
@@ -783,7 +722,7 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
     rows[tid] = rreg0;
     rows[tid + 512] = rreg1;
     int ntile = 0, nchunk = 0;
-    const long long nitem = next_item(item + 1, ntile, nchunk);
+    const long long nitem = walk.next(item + 1, ntile, nchunk);
     ItemAddr na = ia;
     bool same_src = false;
     if (nitem >= 0) {
@@ -853,30 +792,239 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
       }
     }
     __syncthreads();
-    // 8 consecutive threads write one pair's 16 bins (128 bytes), two
-    // adjacent bins (16 bytes) each.  The swizzle keeps bins 2c and 2c+1 in
-    // one 16-byte slot, (2c) ^ (p & 14), in swapped order when p is odd.
-    const int b = (tid & 7) * 2;
-    const int k = ia.k0 + b;
-    if (k < nspec) {
-      for (int p = tid >> 3; p < kTilePairs; p += blockDim.x >> 3) {
-        const int row = rows[p];
-        if (row < 0) continue;
-        const float4 v = *(const float4 *)(stage + p * kBinChunk + (b ^ (p & 14)));
-        const bool sw = (p & 1) != 0;
-        const float2 v0 = sw ? make_float2(v.z, v.w) : make_float2(v.x, v.y);
-        const float2 v1 = sw ? make_float2(v.x, v.y) : make_float2(v.z, v.w);
-        float2 *dst = xspec + (size_t)row * xpitch + k;
-        if (k + 1 < nspec)
-          store_stream2(dst, v0, v1);
-        else
-          store_stream(dst, v0);
-      }
-    }
+    store_tile(stage, rows, ia.k0, nspec, xspec, xpitch);
     item = nitem;
     tile = ntile;
     chunk = nchunk;
     ia = na;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// FP32 contraction on the fp32 matrix instructions.
+//
+// Operand: the spectra as [bin][window][station] complex64, windows padded
+// with zeros to a multiple of 4, so the 16 lanes that hold one window of 16
+// stations in a v_mfma_f32_16x16x4 operand read 128 contiguous bytes.  The
+// transposed copy costs one read and one write of the spectra.
+//
+// Per bin and 4 windows of a 16x16 station block (A, B: source, receiver):
+//   Re += Ar Br + Ai Bi,   Im += Ar Bi + (-Ai) Br,
+// four instructions whose lane reads one window (lane / 16) of one station
+// (lane mod 16), both parts of a complex value from one 8-byte load.  Products
+// and sums are fp32, as the vector form's.
+//
+// Bound: fp32 matrix issue (8 x bins x windows x pairs flops at the ~147
+// TFLOP/s a large fp32 product reaches), then the 8-byte-per-bin result
+// writes.  The vector-ALU form it replaces issued the same flops at half that
+// rate and re-read station rows with 8 x 8 pairs per thread: 600 stations x
+// 47 windows x 18523 bins 33.7 ms; 8 stations x 24 windows 85 us.
+// ---------------------------------------------------------------------------
+constexpr int kF32Group = 4;     // windows per matrix step
+constexpr int kF32TrSta = 64;    // stations per transpose workgroup
+constexpr int kF32TrThreads = 256;
+
+// Bins [bin0, bin0 + 16 gridDim.x) of spec [nstep][nsta][nspec] into out
+// [bin - bin0][kF32Group * gridDim.z][nsta]; windows >= nstep are zero.
+__global__ void __launch_bounds__(kF32TrThreads)
+f32_transpose_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int nspec, int bin0,
+                     float2 *__restrict__ out) {
+  __shared__ float2 tile[kF32Group][kF32TrSta][kBinChunk + 1];
+  constexpr int kLoads = kF32Group * kF32TrSta * kBinChunk / kF32TrThreads;
+  const int tid = threadIdx.x;
+  const int k0 = bin0 + blockIdx.x * kBinChunk, s0 = blockIdx.y * kF32TrSta;
+  const int w0 = blockIdx.z * kF32Group, wpad = gridDim.z * kF32Group;
+  // 16 lanes read one station's 16 bins; all loads issued before the first use
+  float2 z[kLoads];
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const int i = tid + j * kF32TrThreads;
+    const int k = k0 + i % kBinChunk, s = s0 + (i / kBinChunk) % kF32TrSta;
+    const int w = w0 + i / (kBinChunk * kF32TrSta);
+    z[j] = make_float2(0.f, 0.f);
+    if (w < nstep && s < nsta && k < nspec) z[j] = spec[((size_t)w * nsta + s) * nspec + k];
+  }
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const int i = tid + j * kF32TrThreads;
+    tile[i / (kBinChunk * kF32TrSta)][(i / kBinChunk) % kF32TrSta][i % kBinChunk] = z[j];
+  }
+  __syncthreads();
+  // 64 lanes write one window's 64 stations of one bin (512 bytes)
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const int i = tid + j * kF32TrThreads;
+    const int s = i % kF32TrSta, k = (i / kF32TrSta) % kBinChunk, w = i / (kF32TrSta * kBinChunk);
+    if (s0 + s < nsta && k0 + k < nspec)
+      out[((size_t)(blockIdx.x * kBinChunk + k) * wpad + w0 + w) * nsta + s0 + s] = tile[w][s][k];
+  }
+}
+
+// Operands of two matrix steps (8 windows) of one bin: source and receiver
+// halves of the tile.
+struct F32Ops {
+  float2 s[2][2], r[2][2];
+};
+
+// Steps st and st + 1 of the bin whose window 0 starts at p; a step past the
+// last one repeats it (never used).  Offsets: the lane's window and station.
+__device__ __forceinline__ void f32_load(F32Ops &o, const float2 *__restrict__ p, int st, int steps,
+                                         size_t step_elems, const unsigned (&so)[2],
+                                         const unsigned (&ro)[2]) {
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const float2 *q = p + (size_t)(st + u < steps ? st + u : steps - 1) * step_elems;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      o.s[u][h] = q[so[h]];
+      o.r[u][h] = q[ro[h]];
+    }
+  }
+}
+
+template <bool kAll>
+__device__ __forceinline__ void f32_step(const F32Ops &o, int u, int blocks, f32x4_t (&cr)[2][2],
+                                         f32x4_t (&ci)[2][2]) {
+  // all four instructions of every block interleaved, so that no instruction
+  // waits for the accumulator of the one before it
+  auto on = [&](int si, int sj) { return kAll || ((blocks >> (2 * si + sj)) & 1); };
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+#pragma unroll
+    for (int sj = 0; sj < 2; ++sj)
+      if (on(si, sj)) {
+        cr[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].x, o.r[u][sj].x, cr[si][sj], 0, 0, 0);
+        ci[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].x, o.r[u][sj].y, ci[si][sj], 0, 0, 0);
+      }
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+#pragma unroll
+    for (int sj = 0; sj < 2; ++sj)
+      if (on(si, sj)) {
+        cr[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].y, o.r[u][sj].y, cr[si][sj], 0, 0, 0);
+        ci[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(-o.s[u][si].y, o.r[u][sj].x, ci[si][sj], 0, 0, 0);
+      }
+}
+
+// One bin of the tile, staged in LDS.  cur holds steps 0 and 1 on entry; on
+// return it holds steps 0 and 1 of the next bin (next_p, next offsets).
+template <bool kAll>
+__device__ __forceinline__ void f32_bin(F32Ops &cur, const float2 *__restrict__ p, int steps,
+                                        size_t step_elems, const unsigned (&so)[2],
+                                        const unsigned (&ro)[2], const float2 *__restrict__ next_p,
+                                        const unsigned (&nso)[2], const unsigned (&nro)[2],
+                                        int blocks, float scale, int b, int lane_r, int lane_g,
+                                        float2 *stage) {
+  f32x4_t cr[2][2], ci[2][2];
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+#pragma unroll
+    for (int sj = 0; sj < 2; ++sj) cr[si][sj] = ci[si][sj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int st = 0; st < steps; st += 2) {
+    F32Ops nxt;
+    if (st + 2 < steps)
+      f32_load(nxt, p, st + 2, steps, step_elems, so, ro);
+    else
+      f32_load(nxt, next_p, 0, steps, step_elems, nso, nro);
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
+    f32_step<kAll>(cur, 0, blocks, cr, ci);
+    if (st + 1 < steps) f32_step<kAll>(cur, 1, blocks, cr, ci);
+    cur = nxt;
+  }
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+#pragma unroll
+    for (int sj = 0; sj < 2; ++sj) {
+      if (!kAll && !((blocks >> (2 * si + sj)) & 1)) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int a = si * 16 + 4 * lane_g + r, c = sj * 16 + lane_r;
+        stage[stage_index(a * kTile + c, b)] =
+            make_float2(cr[si][sj][r] * scale, ci[si][sj][r] * scale);
+      }
+    }
+}
+
+// Work items, order and staging as contract_mfma_kernel: a 32x32 station tile
+// x 16 bins per item, 8 waves computing two bins each.  Operands of the next
+// 8 windows (or of the next bin) load while the current ones multiply.  op
+// holds bins [16 slab0, ...): the chunks of this launch are slab0 ..
+// slab0 + nchunks - 1.  16 x 16 blocks without listed pairs are skipped.
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int steps,
+                    const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
+                    float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
+                    int slab0, int nchunks) {
+  extern __shared__ __align__(16) float2 stage[];  // [kTilePairs][kBinChunk], swizzled
+  __shared__ int rows[kTilePairs];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int lane_r = lane & 15, lane_g = lane >> 4;
+  const size_t step_elems = (size_t)kF32Group * nsta;
+  const size_t bin_elems = step_elems * steps;
+  const ItemWalk walk(ntiles, nchunks);
+  int tile = 0, chunk = 0;
+  long long item = walk.next(0, tile, chunk);
+  if (item < 0) return;
+  // stations past the array end load a valid station; their pairs are never
+  // stored (nor are bins past the last one)
+  auto offsets = [&](const TileDesc &td, unsigned (&so)[2], unsigned (&ro)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int s = td.src_base + h * 16 + lane_r, r = td.rec_base + h * 16 + lane_r;
+      so[h] = (unsigned)(lane_g * nsta + (s < nsta ? s : nsta - 1));
+      ro[h] = (unsigned)(lane_g * nsta + (r < nsta ? r : nsta - 1));
+    }
+  };
+  auto bin_ptr = [&](int c, int b) {
+    const int k = c * kBinChunk + b, last = nspec - 1 - slab0 * kBinChunk;
+    return op + (size_t)(k < last ? k : last) * bin_elems;
+  };
+  TileDesc td = tiles[tile];
+  unsigned so[2], ro[2];
+  offsets(td, so, ro);
+  F32Ops cur;
+  f32_load(cur, bin_ptr(chunk, wave), 0, steps, step_elems, so, ro);
+  int rreg0 = tile_rows[(size_t)tile * kTilePairs + tid];
+  int rreg1 = tile_rows[(size_t)tile * kTilePairs + tid + 512];
+  while (item >= 0) {
+    __syncthreads();  // the previous item's store phase is done with rows/stage
+    rows[tid] = rreg0;
+    rows[tid + 512] = rreg1;
+    int ntile = tile, nchunk = chunk;
+    const long long nitem = walk.next(item + 1, ntile, nchunk);
+    TileDesc ntd = td;
+    unsigned nso[2] = {so[0], so[1]}, nro[2] = {ro[0], ro[1]};
+    const float2 *np = bin_ptr(chunk, wave);  // no next item: any valid bin
+    if (nitem >= 0) {
+      ntd = tiles[ntile];
+      offsets(ntd, nso, nro);
+      np = bin_ptr(nchunk, wave);
+      rreg0 = tile_rows[(size_t)ntile * kTilePairs + tid];
+      rreg1 = tile_rows[(size_t)ntile * kTilePairs + tid + 512];
+    }
+    const float2 *p0 = bin_ptr(chunk, wave), *p1 = bin_ptr(chunk, wave + 8);
+    if (td.blocks == 15) {
+      f32_bin<true>(cur, p0, steps, step_elems, so, ro, p1, so, ro, 15, scale, wave, lane_r, lane_g,
+                    stage);
+      f32_bin<true>(cur, p1, steps, step_elems, so, ro, np, nso, nro, 15, scale, wave + 8, lane_r,
+                    lane_g, stage);
+    } else {
+      f32_bin<false>(cur, p0, steps, step_elems, so, ro, p1, so, ro, td.blocks, scale, wave, lane_r,
+                     lane_g, stage);
+      f32_bin<false>(cur, p1, steps, step_elems, so, ro, np, nso, nro, td.blocks, scale, wave + 8,
+                     lane_r, lane_g, stage);
+    }
+    __syncthreads();
+    store_tile(stage, rows, (slab0 + chunk) * kBinChunk, nspec, xspec, xpitch);
+    item = nitem;
+    tile = ntile;
+    chunk = nchunk;
+    td = ntd;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      so[h] = nso[h];
+      ro[h] = nro[h];
+    }
   }
 }
 
@@ -1402,6 +1550,11 @@ struct fxc_xc_plan {
   unsigned short *d_hi = nullptr, *d_lo = nullptr;
   size_t split_elems = 0;
   bool ws_shared = false;
+  // FP32 form: transposed spectra of slab_chunks 16-bin chunks at a time
+  // (every chunk when the memory allows)
+  float2 *d_f32 = nullptr;
+  size_t f32_elems = 0;
+  int f32_slab = 0;
   unsigned int *d_amax = nullptr;
   float *d_inv_scale = nullptr, *d_scale = nullptr;
   int scale_cap = 0;
@@ -1579,6 +1732,7 @@ extern "C" int fxc_xc_plan_destroy(fxc_xc_plan *p) {
     dfree(p->d_hi);
     dfree(p->d_lo);
   }
+  dfree(p->d_f32);
   dfree(p->d_amax);
   dfree(p->d_inv_scale);
   dfree(p->d_scale);
@@ -1652,6 +1806,9 @@ int xc_set_pairs_on(fxc_xc_plan *p, int nsta, const int *h_src, const int *h_rec
       TileDesc td;
       td.src_base = (int)(kv.first / nblk) * kTile;
       td.rec_base = (int)(kv.first % nblk) * kTile;
+      td.blocks = 0;
+      for (auto &e : cp)
+        td.blocks |= 1 << (2 * (e.first / kTile / 16) + e.first % kTile / 16);
       p->h_tiles.push_back(td);
       const size_t off = rows.size();
       rows.resize(off + kTilePairs, -1);
@@ -1776,9 +1933,61 @@ static int xc_band_prepare(fxc_xc_plan *p, hipStream_t st) {
   return FXC_OK;
 }
 
-// Split pass for the MFMA forms (no-op for FP32).
+// Bin chunks the contraction covers: [first, first + count).
+static void xc_chunks(const fxc_xc_plan *p, int *first, int *count) {
+  const bool band = p->band_c1 >= 0 && p->precision != FXC_PREC_PLAIN;
+  *first = band ? p->band_c0 : 0;
+  *count = band ? p->band_c1 - p->band_c0 : ceil_div(p->nspec, kBinChunk);
+}
+
+// Transposed operand of the FP32 form for chunks [c0, c0 + n).
+static int xc_f32_transpose(fxc_xc_plan *p, const float2 *d_spec, int c0, int n, hipStream_t st) {
+  FXC_TRY(xc_mark(p, kTimeSplit, true, st));
+  const unsigned steps = (unsigned)ceil_div(p->nstep, kF32Group);
+  hipLaunchKernelGGL(f32_transpose_kernel,
+                     dim3((unsigned)n, (unsigned)ceil_div(p->nsta, kF32TrSta), steps),
+                     dim3(kF32TrThreads), 0, st, d_spec, p->nstep, p->nsta, p->nspec,
+                     c0 * kBinChunk, p->d_f32);
+  FXC_HIP(hipGetLastError());
+  return xc_mark(p, kTimeSplit, false, st);
+}
+
+// Workspace of the transposed operand: every chunk of the band, or, where the
+// device has no room for that, as many as fit (then each slab of chunks is
+// transposed and contracted in turn).
+static int xc_f32_workspace(fxc_xc_plan *p) {
+  int c0 = 0, n = 0;
+  xc_chunks(p, &c0, &n);
+  const size_t chunk = (size_t)kBinChunk * p->nsta * ceil_div(p->nstep, kF32Group) * kF32Group;
+  if (chunk * n > p->f32_elems && !(p->f32_slab > 0 && p->f32_elems >= chunk * kChunkGroup)) {
+    dfree(p->d_f32);
+    p->d_f32 = nullptr;
+    p->f32_elems = 0;
+    for (int m = n;; m = std::max(kChunkGroup, m / 2)) {
+      const int rc = dmalloc((void **)&p->d_f32, chunk * m * sizeof(float2));
+      if (rc == FXC_OK) {
+        p->f32_elems = chunk * m;
+        break;
+      }
+      (void)hipGetLastError();  // out of memory: a smaller slab
+      if (m <= kChunkGroup) return rc;
+    }
+  }
+  const size_t fit = p->f32_elems / chunk;
+  p->f32_slab = fit >= (size_t)n ? 0 : (int)(fit / kChunkGroup) * kChunkGroup;
+  return FXC_OK;
+}
+
+// Operands of the contraction from the spectra (no-op for PLAIN).
 static int xc_prepare_spectra(fxc_xc_plan *p, const float2 *d_spec, hipStream_t st) {
-  if (p->precision == FXC_PREC_FP32 || p->precision == FXC_PREC_PLAIN) return FXC_OK;
+  if (p->precision == FXC_PREC_PLAIN) return FXC_OK;
+  if (p->precision == FXC_PREC_FP32) {
+    FXC_TRY(xc_f32_workspace(p));
+    if (p->f32_slab > 0) return FXC_OK;  // transposed slab by slab
+    int c0 = 0, n = 0;
+    xc_chunks(p, &c0, &n);
+    return xc_f32_transpose(p, d_spec, c0, n, st);
+  }
   FXC_TRY(xc_mark(p, kTimeSplit, true, st));
   // spec mode: only the band's chunks (kSplitBins == kBinChunk)
   static_assert(kSplitBins == kBinChunk, "split blocks are contraction chunks");
@@ -1807,19 +2016,26 @@ static int xc_prepare_spectra(fxc_xc_plan *p, const float2 *d_spec, hipStream_t 
   return FXC_OK;
 }
 
+// Grid of the persistent contractions: a multiple of 8 workgroups (one per
+// CU, LDS-bound).
+static int xc_persistent_grid(unsigned *grid) {
+  int dev = 0, ncu = 0;
+  FXC_HIP(hipGetDevice(&dev));
+  FXC_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  *grid = (unsigned)std::max(8, ncu / 8 * 8);
+  if (const char *env = getenv("FXC_XC_MFMA_GRID"))
+    *grid = (unsigned)std::max(8, atoi(env) / 8 * 8);
+  return FXC_OK;
+}
+
 template <int kMode, int KH, bool kChunked = false>
 static int launch_mfma_kh(dim3 grid, size_t lds, hipStream_t st, const unsigned short *hi,
                           const unsigned short *lo, int nsta, int nspec, const float *sc,
                           const TileDesc *tiles, const int *trows, float2 *dst, long long xpitch,
                           float scale, int kchunks, int chunk0, int nchunks) {
   auto kern = contract_mfma_kernel<kMode, KH / 8, kChunked>;
-  // persistent grid: a multiple of 8 workgroups (one per CU, LDS-bound),
-  // capped by the number of work items
-  int dev = 0, ncu = 0;
-  FXC_HIP(hipGetDevice(&dev));
-  FXC_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  unsigned g = (unsigned)std::max(8, ncu / 8 * 8);
-  if (const char *env = getenv("FXC_XC_MFMA_GRID")) g = (unsigned)std::max(8, atoi(env) / 8 * 8);
+  unsigned g = 0;  // capped by the number of work items
+  FXC_TRY(xc_persistent_grid(&g));
   const dim3 grid1(std::min(g, grid.x));
   // the kernel's item order gives each XCD (blockIdx.x mod 8) its own chunks
   // and covers every item only when the grid is a multiple of 8
@@ -1874,17 +2090,14 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
                              hipStream_t st) {
   const long long t0 = p->chunk_tile_begin[c], t1 = p->chunk_tile_begin[c + 1];
   const unsigned ntl = (unsigned)(t1 - t0);
-  int c0 = 0, nbc = ceil_div(p->nspec, kBinChunk);
-  if (p->band_c1 >= 0 && p->precision != FXC_PREC_PLAIN) {
-    c0 = p->band_c0;
-    nbc = p->band_c1 - p->band_c0;
-  }
+  int c0 = 0, nbc = 0;
+  xc_chunks(p, &c0, &nbc);
   // 1-D grid covering ntl tiles x nbc chunks in groups of kChunkGroup chunks
   const unsigned nwg = ntl * (unsigned)(ceil_div(nbc, kChunkGroup) * kChunkGroup);
   const float scale = 1.0f / (float)p->nstep;
   const TileDesc *tiles = p->d_tiles + t0;
   const int *trows = p->d_tile_rows + t0 * kTilePairs;
-  FXC_TRY(xc_mark(p, kTimeContract, true, st));
+  if (p->precision != FXC_PREC_FP32) FXC_TRY(xc_mark(p, kTimeContract, true, st));
   if (p->precision == FXC_PREC_PLAIN) {
     const long long r0 = p->chunk_row_begin[c], nrows = p->chunk_row_begin[c + 1] - r0;
     const int nbk = ceil_div(p->nspec, 256);
@@ -1896,8 +2109,24 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
                          d_spec + w * win, p->nspec, p->d_row_src + r0, p->d_row_rec + r0, nrows,
                          dst, p->xpitch, nbk, scale);
   } else if (p->precision == FXC_PREC_FP32) {
-    hipLaunchKernelGGL(contract_fp32_kernel, dim3(nwg), dim3(256), 0, st, d_spec, p->nstep,
-                       p->nsta, p->nspec, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0, nbc);
+    const size_t lds = (size_t)kTilePairs * kBinChunk * sizeof(float2);
+    FXC_HIP(hipFuncSetAttribute((const void *)contract_f32_kernel,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    unsigned grid = 0;
+    FXC_TRY(xc_persistent_grid(&grid));
+    const int slab = p->f32_slab > 0 ? p->f32_slab : nbc;
+    for (int b = 0; b < nbc; b += slab) {
+      const int n = std::min(slab, nbc - b);
+      if (p->f32_slab > 0) FXC_TRY(xc_f32_transpose(p, d_spec, c0 + b, n, st));
+      FXC_TRY(xc_mark(p, kTimeContract, true, st));
+      const unsigned items = ntl * (unsigned)(ceil_div(n, kChunkGroup) * kChunkGroup);
+      hipLaunchKernelGGL(contract_f32_kernel, dim3(std::min(grid, items)), dim3(512), lds, st,
+                         p->d_f32, p->nsta, p->nspec, (int)ceil_div(p->nstep, kF32Group), tiles,
+                         trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n);
+      FXC_HIP(hipGetLastError());
+      FXC_TRY(xc_mark(p, kTimeContract, false, st));
+    }
+    return FXC_OK;
   } else {
     const size_t lds = (size_t)kTilePairs * kBinChunk * sizeof(float2);
     // grid.y carries the tile count to the launcher (the launch itself is 1-D)

@@ -640,7 +640,9 @@ int run(const Args &a) {
       }
       // workspace rows that fit the remaining budget (the plan chunks the rest)
       const size_t used = d_spec_elems * 8 + d_cc_elems * 4 +
-                          (prec == FXC_PREC_BF16X3 || prec == FXC_PREC_FP16 ? nl * (size_t)work->nspec * 256 : 0);
+                          (prec == FXC_PREC_BF16X3 || prec == FXC_PREC_FP16 ? nl * (size_t)work->nspec * 256 : 0) +
+                          // transposed spectra, windows in fours
+                          (prec == FXC_PREC_FP32 ? nl * (size_t)work->nspec * (((size_t)work->nstep + 3) / 4) * 32 : 0);
       const size_t pitch = ((size_t)work->nspec + 15) / 16 * 16 * 8;
       long long chunk = 0;
       if (budget > used + (256ull << 20)) chunk = (long long)((budget - used - (256ull << 20)) / pitch);

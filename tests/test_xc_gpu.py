@@ -320,3 +320,28 @@ def test_band_rejects_bad_ranges(gpu):
         plain.set_band(10, 500)
     plain.set_band()  # parity is always accepted
     plain.close()
+
+
+@pytest.mark.parametrize("nsta,nstep", [(2, 1), (9, 4), (16, 5), (17, 7), (33, 8), (48, 13), (65, 3)])
+def test_fp32_matrix_tiles(gpu, nsta, nstep):
+    """Edges of the FP32 contraction: window counts around its steps of 4 and 8, station counts
+    around its 16- and 32-station blocks, pairs in either order and listed twice, a last bin chunk
+    that is not full.  fp32 sums of 2 nstep products: relative error below 2 nstep 2^-24 of
+    sum |a||b|, here against the FP64 stack."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    nspec = 73
+    rng = np.random.default_rng(nsta * 100 + nstep)
+    spec = (rng.standard_normal((nstep, nsta, nspec)) +
+            1j * rng.standard_normal((nstep, nsta, nspec))).astype(np.complex64)
+    a, b = np.nonzero(rng.random((nsta, nsta)) < 0.6)
+    src = np.concatenate([[0], a, a[:5]]).astype(np.int32)
+    rec = np.concatenate([[nsta - 1], b, b[:5]]).astype(np.int32)
+    plan = XcPlan(nspec, nstep, 0.1, 20, "fp32")
+    plan.set_pairs(nsta, src, rec)
+    got = plan.cross_spectra(torch.from_numpy(spec).to(gpu)).cpu().numpy()
+    z = spec.astype(np.complex128)
+    want = (z[:, src].conj() * z[:, rec]).mean(axis=0)
+    bound = (np.abs(z[:, src]) * np.abs(z[:, rec])).mean(axis=0) * (2 * nstep + 2) * 2.0 ** -24
+    assert (np.abs(got - want) <= 2 * bound).all()
