@@ -36,6 +36,7 @@
 #include <climits>
 #include <map>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace fxc {
@@ -815,216 +816,316 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
 // and sums are fp32, as the vector form's.
 //
 // Bound: fp32 matrix issue (8 x bins x windows x pairs flops at the ~147
-// TFLOP/s a large fp32 product reaches), then the 8-byte-per-bin result
-// writes.  The vector-ALU form it replaces issued the same flops at half that
-// rate and re-read station rows with 8 x 8 pairs per thread: 600 stations x
-// 47 windows x 18523 bins 33.7 ms; 8 stations x 24 windows 85 us.
+// TFLOP/s a large fp32 product reaches), then operand reads that miss an XCD's
+// L2 (600 stations x 47 windows: 3.7 MB per 16-bin chunk, 22 GB read per call)
+// and the 8-byte-per-bin result writes.  600 x 47 x 18523 bins: transpose 1.8
+// ms + contraction 14.7 ms (matrix pipe busy 65 %) against 33.7 ms for the
+// vector-ALU form it replaced, which issued the same flops at half the rate
+// and re-read station rows with 8 x 8 pairs per thread; 8 stations x 24
+// windows 17 + 37 us against 85 us.
 // ---------------------------------------------------------------------------
 constexpr int kF32Group = 4;     // windows per matrix step
-constexpr int kF32TrSta = 64;    // stations per transpose workgroup
 constexpr int kF32TrThreads = 256;
 
 // Bins [bin0, bin0 + 16 gridDim.x) of spec [nstep][nsta][nspec] into out
-// [bin - bin0][kF32Group * gridDim.z][nsta]; windows >= nstep are zero.
+// [bin - bin0][wpad][nsta]; windows >= nstep are zero.  A workgroup takes kSta
+// stations x 256 / kSta windows: 64 x 4, or 16 x 16 for arrays of at most 16
+// stations, whose lanes and launches would mostly be idle at 64 x 4 (8
+// stations x 24 windows: 26 us).
+template <int kSta>
 __global__ void __launch_bounds__(kF32TrThreads)
 f32_transpose_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int nspec, int bin0,
-                     float2 *__restrict__ out) {
-  __shared__ float2 tile[kF32Group][kF32TrSta][kBinChunk + 1];
-  constexpr int kLoads = kF32Group * kF32TrSta * kBinChunk / kF32TrThreads;
+                     int wpad, float2 *__restrict__ out) {
+  constexpr int kWin = 256 / kSta;
+  __shared__ float2 tile[kWin][kSta][kBinChunk + 1];
+  constexpr int kLoads = kWin * kSta * kBinChunk / kF32TrThreads;
   const int tid = threadIdx.x;
-  const int k0 = bin0 + blockIdx.x * kBinChunk, s0 = blockIdx.y * kF32TrSta;
-  const int w0 = blockIdx.z * kF32Group, wpad = gridDim.z * kF32Group;
+  const int k0 = bin0 + blockIdx.x * kBinChunk, s0 = blockIdx.y * kSta;
+  const int w0 = blockIdx.z * kWin;
   // 16 lanes read one station's 16 bins; all loads issued before the first use
   float2 z[kLoads];
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) {
     const int i = tid + j * kF32TrThreads;
-    const int k = k0 + i % kBinChunk, s = s0 + (i / kBinChunk) % kF32TrSta;
-    const int w = w0 + i / (kBinChunk * kF32TrSta);
+    const int k = k0 + i % kBinChunk, s = s0 + (i / kBinChunk) % kSta;
+    const int w = w0 + i / (kBinChunk * kSta);
     z[j] = make_float2(0.f, 0.f);
     if (w < nstep && s < nsta && k < nspec) z[j] = spec[((size_t)w * nsta + s) * nspec + k];
   }
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) {
     const int i = tid + j * kF32TrThreads;
-    tile[i / (kBinChunk * kF32TrSta)][(i / kBinChunk) % kF32TrSta][i % kBinChunk] = z[j];
+    tile[i / (kBinChunk * kSta)][(i / kBinChunk) % kSta][i % kBinChunk] = z[j];
   }
   __syncthreads();
-  // 64 lanes write one window's 64 stations of one bin (512 bytes)
+  // kSta lanes write one window's stations of one bin
 #pragma unroll
   for (int j = 0; j < kLoads; ++j) {
     const int i = tid + j * kF32TrThreads;
-    const int s = i % kF32TrSta, k = (i / kF32TrSta) % kBinChunk, w = i / (kF32TrSta * kBinChunk);
-    if (s0 + s < nsta && k0 + k < nspec)
+    const int s = i % kSta, k = (i / kSta) % kBinChunk, w = i / (kSta * kBinChunk);
+    if (s0 + s < nsta && k0 + k < nspec && w0 + w < wpad)
       out[((size_t)(blockIdx.x * kBinChunk + k) * wpad + w0 + w) * nsta + s0 + s] = tile[w][s][k];
   }
 }
 
-// Operands of two matrix steps (8 windows) of one bin: source and receiver
-// halves of the tile.
-struct F32Ops {
-  float2 s[2][2], r[2][2];
+// One matrix step (4 windows) of 32 source stations x 16 receivers (bit si of
+// kMask: source half si is listed).  The instructions of the two blocks are
+// interleaved, so that none waits for the accumulator of the one before it.
+template <int kMask>
+__device__ __forceinline__ void f32_step(const float2 (&s)[2], float2 r, f32x4_t (&cr)[2],
+                                         f32x4_t (&ci)[2]) {
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+    if ((kMask >> si) & 1) {
+      cr[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.x, cr[si], 0, 0, 0);
+      ci[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.y, ci[si], 0, 0, 0);
+    }
+#pragma unroll
+  for (int si = 0; si < 2; ++si)
+    if ((kMask >> si) & 1) {
+      cr[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].y, r.y, cr[si], 0, 0, 0);
+      ci[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(-s[si].y, r.x, ci[si], 0, 0, 0);
+    }
+}
+
+// Steps loaded ahead of their use (fewer where the sources fill the registers).
+constexpr int kF32Ahead = 6;
+constexpr int f32_ahead(int steps) {
+  return steps > 11 ? 3 : steps > 8 ? 4 : steps > kF32Ahead ? kF32Ahead : steps < 1 ? 1 : steps;
+}
+
+// Position of a wave's next receiver loads: bin start, the lane's offset.
+struct F32Rec {
+  const float2 *p;
+  unsigned off;
 };
 
-// Steps st and st + 1 of the bin whose window 0 starts at p; a step past the
-// last one repeats it (never used).  Offsets: the lane's window and station.
-__device__ __forceinline__ void f32_load(F32Ops &o, const float2 *__restrict__ p, int st, int steps,
-                                         size_t step_elems, const unsigned (&so)[2],
-                                         const unsigned (&ro)[2]) {
+// One bin of a phase: 32 sources x 16 receivers, summed over the depth and
+// staged as [32 sources][16 receivers][16 bins].  kSteps > 0: the sources are
+// in src and ring holds receiver steps 0 .. ahead-1 on entry, those of the
+// next bin on return.  kSteps 0 (any depth): sources load with the receivers
+// and nothing is ahead across bins.
+template <int kSteps, int kMask>
+__device__ __forceinline__ void f32_bin(const float2 (&src)[kSteps > 0 ? kSteps : 1][2],
+                                        float2 (&ring)[kF32Ahead], F32Rec cur, F32Rec nxt,
+                                        const float2 *__restrict__ sp, const unsigned (&so)[2],
+                                        int steps, size_t step_elems, float scale, int b,
+                                        int lane_r, int lane_g, float2 *stage) {
+  f32x4_t cr[2], ci[2];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const float2 *q = p + (size_t)(st + u < steps ? st + u : steps - 1) * step_elems;
+  for (int si = 0; si < 2; ++si) cr[si] = ci[si] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if constexpr (kSteps > 0) {
+    constexpr int kD = f32_ahead(kSteps);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      o.s[u][h] = q[so[h]];
-      o.r[u][h] = q[ro[h]];
+    for (int s = 0; s < kSteps; ++s) {
+      const float2 r = ring[s % kD];
+      ring[s % kD] = s + kD < kSteps ? (cur.p + (s + kD) * step_elems)[cur.off]
+                                     : (nxt.p + (s + kD - kSteps) * step_elems)[nxt.off];
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
+      f32_step<kMask>(src[s], r, cr, ci);
     }
+    // the next bin's step i sits at (kSteps + i) % kD
+    float2 t[kD];
+#pragma unroll
+    for (int i = 0; i < kD; ++i) t[i] = ring[(kSteps + i) % kD];
+#pragma unroll
+    for (int i = 0; i < kD; ++i) ring[i] = t[i];
+  } else {
+    constexpr int kD = 4;
+    float2 a[kD][2], r[kD];
+    auto load = [&](int i, int s) {  // a step past the last one repeats it (never used)
+      const size_t o = (size_t)(s < steps ? s : steps - 1) * step_elems;
+      a[i][0] = (sp + o)[so[0]];
+      a[i][1] = (sp + o)[so[1]];
+      r[i] = (cur.p + o)[cur.off];
+    };
+#pragma unroll
+    for (int i = 0; i < kD; ++i) load(i, i);
+#pragma unroll 1
+    for (int s0 = 0; s0 < steps; s0 += kD) {
+#pragma unroll
+      for (int i = 0; i < kD; ++i) {
+        const float2 ai[2] = {a[i][0], a[i][1]}, ri = r[i];
+        load(i, s0 + kD + i);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s0 + i < steps) f32_step<kMask>(ai, ri, cr, ci);
+      }
+    }
+  }
+  // pair (16 si + 4 lane_g + r, lane_r), whose low four bits are lane_r
+  float2 *o = stage + stage_index(4 * lane_g * 16 + lane_r, b);
+#pragma unroll
+  for (int si = 0; si < 2; ++si) {
+    if (!((kMask >> si) & 1)) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      o[(16 * si + r) * 16 * kBinChunk] = make_float2(cr[si][r] * scale, ci[si][r] * scale);
   }
 }
 
-template <bool kAll>
-__device__ __forceinline__ void f32_step(const F32Ops &o, int u, int blocks, f32x4_t (&cr)[2][2],
-                                         f32x4_t (&ci)[2][2]) {
-  // all four instructions of every block interleaved, so that no instruction
-  // waits for the accumulator of the one before it
-  auto on = [&](int si, int sj) { return kAll || ((blocks >> (2 * si + sj)) & 1); };
-#pragma unroll
-  for (int si = 0; si < 2; ++si)
-#pragma unroll
-    for (int sj = 0; sj < 2; ++sj)
-      if (on(si, sj)) {
-        cr[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].x, o.r[u][sj].x, cr[si][sj], 0, 0, 0);
-        ci[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].x, o.r[u][sj].y, ci[si][sj], 0, 0, 0);
-      }
-#pragma unroll
-  for (int si = 0; si < 2; ++si)
-#pragma unroll
-    for (int sj = 0; sj < 2; ++sj)
-      if (on(si, sj)) {
-        cr[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.s[u][si].y, o.r[u][sj].y, cr[si][sj], 0, 0, 0);
-        ci[si][sj] = __builtin_amdgcn_mfma_f32_16x16x4f32(-o.s[u][si].y, o.r[u][sj].x, ci[si][sj], 0, 0, 0);
-      }
-}
+// Work items and order as contract_mfma_kernel: a 32 x 32 station tile x 16
+// bins, in two phases of 16 receivers each.  8 waves multiply, two bins per
+// wave; 4 more waves write the finished phase's rows from its 64 KB LDS buffer
+// while the next phase fills the other one.  Vector-memory counters retire
+// loads and stores in order, so a wave that did both would wait for its rows
+// to drain before its next operands (600 stations x 47 windows: 14.7 ms; 14.9
+// with the same waves writing; 16.7 so and without held sources; 19.3 in half
+// tiles with two workgroups per CU, which read half as much again per pair).  One barrier per
+// phase; both kinds of waves pass the same number of them.
+// op holds bins [16 slab0, ...): the chunks of this launch are slab0 ..
+// slab0 + nchunks - 1.  Blocks of 16 x 16 stations without listed pairs are
+// skipped.
+// kSteps > 0 (up to kF32HeldSteps): the depth in steps; the sources of the
+// wave's two bins stay in registers while consecutive items share them.
+constexpr int kF32HeldSteps = 12;  // three waves per SIMD leave 168 registers
+constexpr int kF32Compute = 512, kF32Store = 256;
+constexpr int kF32PhasePairs = kTile * 16;
 
-// One bin of the tile, staged in LDS.  cur holds steps 0 and 1 on entry; on
-// return it holds steps 0 and 1 of the next bin (next_p, next offsets).
-template <bool kAll>
-__device__ __forceinline__ void f32_bin(F32Ops &cur, const float2 *__restrict__ p, int steps,
-                                        size_t step_elems, const unsigned (&so)[2],
-                                        const unsigned (&ro)[2], const float2 *__restrict__ next_p,
-                                        const unsigned (&nso)[2], const unsigned (&nro)[2],
-                                        int blocks, float scale, int b, int lane_r, int lane_g,
-                                        float2 *stage) {
-  f32x4_t cr[2][2], ci[2][2];
-#pragma unroll
-  for (int si = 0; si < 2; ++si)
-#pragma unroll
-    for (int sj = 0; sj < 2; ++sj) cr[si][sj] = ci[si][sj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int st = 0; st < steps; st += 2) {
-    F32Ops nxt;
-    if (st + 2 < steps)
-      f32_load(nxt, p, st + 2, steps, step_elems, so, ro);
-    else
-      f32_load(nxt, next_p, 0, steps, step_elems, nso, nro);
-    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
-    f32_step<kAll>(cur, 0, blocks, cr, ci);
-    if (st + 1 < steps) f32_step<kAll>(cur, 1, blocks, cr, ci);
-    cur = nxt;
-  }
-#pragma unroll
-  for (int si = 0; si < 2; ++si)
-#pragma unroll
-    for (int sj = 0; sj < 2; ++sj) {
-      if (!kAll && !((blocks >> (2 * si + sj)) & 1)) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int a = si * 16 + 4 * lane_g + r, c = sj * 16 + lane_r;
-        stage[stage_index(a * kTile + c, b)] =
-            make_float2(cr[si][sj][r] * scale, ci[si][sj][r] * scale);
-      }
-    }
-}
-
-// Work items, order and staging as contract_mfma_kernel: a 32x32 station tile
-// x 16 bins per item, 8 waves computing two bins each.  Operands of the next
-// 8 windows (or of the next bin) load while the current ones multiply.  op
-// holds bins [16 slab0, ...): the chunks of this launch are slab0 ..
-// slab0 + nchunks - 1.  16 x 16 blocks without listed pairs are skipped.
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int kSteps>
+__global__ void __launch_bounds__(kF32Compute + kF32Store) __attribute__((amdgpu_waves_per_eu(3, 3)))
 contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int steps,
                     const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
                     float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
                     int slab0, int nchunks) {
-  extern __shared__ __align__(16) float2 stage[];  // [kTilePairs][kBinChunk], swizzled
-  __shared__ int rows[kTilePairs];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int lane_r = lane & 15, lane_g = lane >> 4;
-  const size_t step_elems = (size_t)kF32Group * nsta;
-  const size_t bin_elems = step_elems * steps;
+  extern __shared__ __align__(16) float2 stage[];  // [2][kF32PhasePairs][kBinChunk], swizzled
+  const int tid = threadIdx.x;
   const ItemWalk walk(ntiles, nchunks);
   int tile = 0, chunk = 0;
   long long item = walk.next(0, tile, chunk);
-  if (item < 0) return;
-  // stations past the array end load a valid station; their pairs are never
-  // stored (nor are bins past the last one)
-  auto offsets = [&](const TileDesc &td, unsigned (&so)[2], unsigned (&ro)[2]) {
+  if (item < 0) return;  // the whole workgroup
+
+  if (__builtin_amdgcn_readfirstlane(tid) >= kF32Compute) {  // whole waves
+    // Row writers: thread t takes bins 2 (t & 7), +1 of pairs (t >> 3) + 32 i:
+    // 8 threads write one pair's 16 bins (128 bytes).  The rows of the next
+    // phase load before this phase's stores.
+    constexpr int kPer = kF32PhasePairs / (kF32Store / 8);
+    const int t = tid - kF32Compute, b = (t & 7) * 2, p0 = t >> 3;
+    int rows[kPer];
+    auto load_rows = [&](int tl, int h) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int s = td.src_base + h * 16 + lane_r, r = td.rec_base + h * 16 + lane_r;
-      so[h] = (unsigned)(lane_g * nsta + (s < nsta ? s : nsta - 1));
-      ro[h] = (unsigned)(lane_g * nsta + (r < nsta ? r : nsta - 1));
+      for (int i = 0; i < kPer; ++i) {
+        const int p = p0 + 32 * i;  // source p / 16, receiver 16 h + p % 16
+        rows[i] = tile_rows[(size_t)tl * kTilePairs + (p >> 4) * kTile + 16 * h + (p & 15)];
+      }
+    };
+    load_rows(tile, 0);
+    while (item >= 0) {
+      int ntile = tile, nchunk = chunk;
+      const long long nitem = walk.next(item + 1, ntile, nchunk);
+      const int k = (slab0 + chunk) * kBinChunk + b;
+#pragma unroll 1
+      for (int h = 0; h < 2; ++h) {
+        int cur[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) cur[i] = rows[i];
+        load_rows(h == 0 || nitem < 0 ? tile : ntile, h == 0);
+        __syncthreads();  // the phase is staged
+        const float2 *buf = stage + h * (kF32PhasePairs * kBinChunk);
+        if (k < nspec) {
+#pragma unroll
+          for (int i = 0; i < kPer; ++i) {
+            const int p = p0 + 32 * i;
+            if (cur[i] < 0) continue;
+            // bins 2c and 2c+1 share a 16-byte slot, swapped when p is odd
+            const float4 v = *(const float4 *)(buf + p * kBinChunk + (b ^ (p & 14)));
+            const bool sw = (p & 1) != 0;
+            const float2 v0 = sw ? make_float2(v.z, v.w) : make_float2(v.x, v.y);
+            const float2 v1 = sw ? make_float2(v.x, v.y) : make_float2(v.z, v.w);
+            float2 *dst = xspec + (size_t)cur[i] * xpitch + k;
+            if (k + 1 < nspec)
+              store_stream2(dst, v0, v1);
+            else
+              store_stream(dst, v0);
+          }
+        }
+      }
+      item = nitem;
+      tile = ntile;
+      chunk = nchunk;
     }
+    return;
+  }
+
+  constexpr bool kHeld = kSteps > 0;
+  constexpr int kS = kHeld ? kSteps : 1;
+  constexpr int kD = f32_ahead(kS);
+  // (a uniform wave index keeps the operand pointers in scalar registers)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lane_r = lane & 15, lane_g = lane >> 4;
+  const size_t step_elems = (size_t)kF32Group * nsta;
+  const size_t bin_elems = step_elems * (kHeld ? kSteps : steps);
+  // the lane's window and station; stations past the array end load a valid
+  // one (their pairs are never stored, nor are bins past the last one)
+  auto offset = [&](int base) {
+    const int s = base + lane_r;
+    return (unsigned)(lane_g * nsta + (s < nsta ? s : nsta - 1));
   };
   auto bin_ptr = [&](int c, int b) {
     const int k = c * kBinChunk + b, last = nspec - 1 - slab0 * kBinChunk;
     return op + (size_t)(k < last ? k : last) * bin_elems;
   };
+  // source halves listed with receiver half h (0: the phase has no pairs)
+  auto mask_of = [](const TileDesc &t, int h) {
+    return ((t.blocks >> h) & 1) | (((t.blocks >> (2 + h)) & 1) << 1);
+  };
+  // lane offset of an item's first phase with pairs
+  auto first_off = [&](const TileDesc &t) { return offset(t.rec_base + (mask_of(t, 0) ? 0 : 16)); };
   TileDesc td = tiles[tile];
-  unsigned so[2], ro[2];
-  offsets(td, so, ro);
-  F32Ops cur;
-  f32_load(cur, bin_ptr(chunk, wave), 0, steps, step_elems, so, ro);
-  int rreg0 = tile_rows[(size_t)tile * kTilePairs + tid];
-  int rreg1 = tile_rows[(size_t)tile * kTilePairs + tid + 512];
+  float2 src[2][kS][2], ring[kF32Ahead];
+  if constexpr (kHeld) {
+    const F32Rec r{bin_ptr(chunk, wave), first_off(td)};
+#pragma unroll
+    for (int i = 0; i < kD; ++i) ring[i] = (r.p + i * step_elems)[r.off];
+  }
+  bool stale = true;  // src does not hold this item's sources yet
   while (item >= 0) {
-    __syncthreads();  // the previous item's store phase is done with rows/stage
-    rows[tid] = rreg0;
-    rows[tid + 512] = rreg1;
+    const unsigned so[2] = {offset(td.src_base), offset(td.src_base + 16)};
+    const float2 *bp[2] = {bin_ptr(chunk, wave), bin_ptr(chunk, wave + 8)};
+    if (kHeld && stale) {
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+        for (int s = 0; s < kS; ++s) {
+          src[bi][s][0] = (bp[bi] + s * step_elems)[so[0]];
+          src[bi][s][1] = (bp[bi] + s * step_elems)[so[1]];
+        }
+    }
     int ntile = tile, nchunk = chunk;
     const long long nitem = walk.next(item + 1, ntile, nchunk);
-    TileDesc ntd = td;
-    unsigned nso[2] = {so[0], so[1]}, nro[2] = {ro[0], ro[1]};
-    const float2 *np = bin_ptr(chunk, wave);  // no next item: any valid bin
-    if (nitem >= 0) {
-      ntd = tiles[ntile];
-      offsets(ntd, nso, nro);
-      np = bin_ptr(nchunk, wave);
-      rreg0 = tile_rows[(size_t)ntile * kTilePairs + tid];
-      rreg1 = tile_rows[(size_t)ntile * kTilePairs + tid + 512];
+    if (nitem < 0) {
+      ntile = tile;  // the loads ahead of a next item stay on this one
+      nchunk = chunk;
     }
-    const float2 *p0 = bin_ptr(chunk, wave), *p1 = bin_ptr(chunk, wave + 8);
-    if (td.blocks == 15) {
-      f32_bin<true>(cur, p0, steps, step_elems, so, ro, p1, so, ro, 15, scale, wave, lane_r, lane_g,
-                    stage);
-      f32_bin<true>(cur, p1, steps, step_elems, so, ro, np, nso, nro, 15, scale, wave + 8, lane_r,
-                    lane_g, stage);
-    } else {
-      f32_bin<false>(cur, p0, steps, step_elems, so, ro, p1, so, ro, td.blocks, scale, wave, lane_r,
-                     lane_g, stage);
-      f32_bin<false>(cur, p1, steps, step_elems, so, ro, np, nso, nro, td.blocks, scale, wave + 8,
-                     lane_r, lane_g, stage);
+    const TileDesc ntd = tiles[ntile];
+    const unsigned ro[2] = {offset(td.rec_base), offset(td.rec_base + 16)};
+    const F32Rec next_item{bin_ptr(nchunk, wave), first_off(ntd)};
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+      float2 *buf = stage + h * (kF32PhasePairs * kBinChunk);
+      const unsigned off = h ? ro[1] : ro[0];
+      const F32Rec r0{bp[0], off}, r1{bp[1], off};
+      const F32Rec r2 = h == 0 && mask_of(td, 1) ? F32Rec{bp[0], ro[1]} : next_item;
+      auto bins = [&](auto m) {
+        constexpr int kMask = decltype(m)::value;
+        f32_bin<kSteps, kMask>(src[0], ring, r0, r1, bp[0], so, steps, step_elems, scale, wave,
+                               lane_r, lane_g, buf);
+        f32_bin<kSteps, kMask>(src[1], ring, r1, r2, bp[1], so, steps, step_elems, scale, wave + 8,
+                               lane_r, lane_g, buf);
+      };
+      const int mask = mask_of(td, h);
+      if (mask == 3)
+        bins(std::integral_constant<int, 3>{});
+      else if (mask == 2)
+        bins(std::integral_constant<int, 2>{});
+      else if (mask == 1)
+        bins(std::integral_constant<int, 1>{});
+      __syncthreads();  // staged; the writers are done with the other buffer
     }
-    __syncthreads();
-    store_tile(stage, rows, (slab0 + chunk) * kBinChunk, nspec, xspec, xpitch);
+    stale = nchunk != chunk || ntd.src_base != td.src_base;
     item = nitem;
     tile = ntile;
     chunk = nchunk;
     td = ntd;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      so[h] = nso[h];
-      ro[h] = nro[h];
-    }
   }
 }
 
@@ -1943,11 +2044,14 @@ static void xc_chunks(const fxc_xc_plan *p, int *first, int *count) {
 // Transposed operand of the FP32 form for chunks [c0, c0 + n).
 static int xc_f32_transpose(fxc_xc_plan *p, const float2 *d_spec, int c0, int n, hipStream_t st) {
   FXC_TRY(xc_mark(p, kTimeSplit, true, st));
-  const unsigned steps = (unsigned)ceil_div(p->nstep, kF32Group);
-  hipLaunchKernelGGL(f32_transpose_kernel,
-                     dim3((unsigned)n, (unsigned)ceil_div(p->nsta, kF32TrSta), steps),
+  const int wpad = (int)ceil_div(p->nstep, kF32Group) * kF32Group;
+  const int sta = p->nsta <= 16 ? 16 : 64;
+  auto kern = sta == 16 ? f32_transpose_kernel<16> : f32_transpose_kernel<64>;
+  hipLaunchKernelGGL(kern,
+                     dim3((unsigned)n, (unsigned)ceil_div(p->nsta, sta),
+                          (unsigned)ceil_div(wpad, 256 / sta)),
                      dim3(kF32TrThreads), 0, st, d_spec, p->nstep, p->nsta, p->nspec,
-                     c0 * kBinChunk, p->d_f32);
+                     c0 * kBinChunk, wpad, p->d_f32);
   FXC_HIP(hipGetLastError());
   return xc_mark(p, kTimeSplit, false, st);
 }
@@ -2086,6 +2190,19 @@ static int launch_mfma_contract(int precision, int kh, dim3 grid, size_t lds, hi
                                          dst, xpitch, scale, chunk0, nchunks);
 }
 
+// The FP32 contraction for a depth in steps: sources held up to
+// kF32HeldSteps, whose registers two bins' sources still fit (8 per step).
+typedef decltype(&contract_f32_kernel<0>) F32Kernel;
+template <int kSteps>
+static F32Kernel f32_kernel_from(int steps) {
+  if constexpr (kSteps > 0) {
+    if (steps == kSteps) return contract_f32_kernel<kSteps>;
+    return f32_kernel_from<kSteps - 1>(steps);
+  }
+  return contract_f32_kernel<0>;
+}
+static F32Kernel f32_kernel_of(int steps) { return f32_kernel_from<kF32HeldSteps>(steps); }
+
 static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, float2 *dst,
                              hipStream_t st) {
   const long long t0 = p->chunk_tile_begin[c], t1 = p->chunk_tile_begin[c + 1];
@@ -2110,8 +2227,10 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
                          dst, p->xpitch, nbk, scale);
   } else if (p->precision == FXC_PREC_FP32) {
     const size_t lds = (size_t)kTilePairs * kBinChunk * sizeof(float2);
-    FXC_HIP(hipFuncSetAttribute((const void *)contract_f32_kernel,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int steps = (int)ceil_div(p->nstep, kF32Group);
+    auto kern = f32_kernel_of(steps);
+    FXC_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds));
     unsigned grid = 0;
     FXC_TRY(xc_persistent_grid(&grid));
     const int slab = p->f32_slab > 0 ? p->f32_slab : nbc;
@@ -2120,9 +2239,8 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
       if (p->f32_slab > 0) FXC_TRY(xc_f32_transpose(p, d_spec, c0 + b, n, st));
       FXC_TRY(xc_mark(p, kTimeContract, true, st));
       const unsigned items = ntl * (unsigned)(ceil_div(n, kChunkGroup) * kChunkGroup);
-      hipLaunchKernelGGL(contract_f32_kernel, dim3(std::min(grid, items)), dim3(512), lds, st,
-                         p->d_f32, p->nsta, p->nspec, (int)ceil_div(p->nstep, kF32Group), tiles,
-                         trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n);
+      hipLaunchKernelGGL(kern, dim3(std::min(grid, items)), dim3(kF32Compute + kF32Store), lds, st,
+                         p->d_f32, p->nsta, p->nspec, steps, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n);
       FXC_HIP(hipGetLastError());
       FXC_TRY(xc_mark(p, kTimeContract, false, st));
     }
