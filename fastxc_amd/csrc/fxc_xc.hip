@@ -1150,74 +1150,127 @@ constexpr unsigned kRadixLag8 = (1u << 2) | (1u << 3) | (1u << 4) | (1u << 5) | 
 constexpr unsigned kRadixLag9 = kRadixLag8 | (1u << 9);
 constexpr int kLagRegs = (kLdsComplexCapacity + kLagThreads - 1) / kLagThreads;
 
+// Bins of one lag transform into registers: X[k], or (kHalf) every second bin
+// X[2 k + part], count of them.  kProd: X is formed as conj(X) Y of two
+// station spectra as it is read.
+template <bool kHalf = false, bool kProd = false>
 __device__ __forceinline__ void lag_prefetch(float2 (&pre)[kLagRegs], const float2 *__restrict__ X,
-                                             int nspec) {
+                                             int count, const float2 *__restrict__ Y = nullptr,
+                                             int part = 0) {
 #pragma unroll
   for (int i = 0; i < kLagRegs; ++i) {
     const int k = threadIdx.x + i * kLagThreads;
-    if (k < nspec) pre[i] = X[k];
+    if (k < count) {
+      const int at = kHalf ? 2 * k + part : k;
+      if constexpr (kProd) {
+        const float2 u = X[at], v = Y[at];
+        pre[i] = make_float2(u.x * v.x + u.y * v.y, u.x * v.y - u.y * v.x);
+      } else {
+        pre[i] = X[at];
+      }
+    }
+    // a product's factors: a few loads in flight at a time, as both spectra
+    // of every bin would not fit the registers
+    if (kProd && i % 5 == 4) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-template <unsigned kRadixLag>
+// kHalf: nfft/2 = 2 M complex values do not fit the LDS, so the transform of
+// the folded spectrum Z runs as two transforms of M, over its even and its odd
+// bins, one after the other in the same LDS:
+//   z[n] = F_0[n mod M] + exp(2 pi i n / 2M) F_1[n mod M].
+// Each half is closed under the fold's mirror (k <-> 2M - k): bin 2 i pairs
+// with 2 (M - i), bin 2 i + 1 with 2 (M - 1 - i) + 1.  The kept lags' F_0 wait
+// in the output row.  A row is read twice (its lines' other halves come from
+// the Infinity Cache) and its 2H+1 lags written; the four-step transform it
+// replaces moved each row about eight times through HBM: 120 stations at
+// 20 Hz (7140 rows, nfft 74088, 4001 lags) 7.2 ms.
+// kProd (with kHalf): the one-window stack conj(S[src]) S[rec] formed from the
+// spectra as they are read.
+template <unsigned kRadixLag, bool kHalf, bool kProd>
 __global__ void __launch_bounds__(kLagThreads)
-lag_kernel(const float2 *__restrict__ xspec, long long xpitch, int nspec, long long nrows,
+lag_kernel(const float2 *__restrict__ xspec, long long xpitch, long long nrows,
            const int *__restrict__ row_out, float *__restrict__ cc, int half_cc, double weight,
            const float *__restrict__ task_scale, FftPlanDev plan, const float2 *__restrict__ tw,
-           const float2 *__restrict__ fold) {
+           const float2 *__restrict__ fold, float2 wodd, const int *__restrict__ row_src,
+           const int *__restrict__ row_rec) {
   extern __shared__ float2 lds[];
-  const int M = plan.n;  // nspec == M + 1
+  const int M = plan.n;
   stage_real_tables(lds, plan, tw, fold);
   const float2 *twl = lds + M + 1;
   const float2 *fl = twl + tw_lds_count(M);
   float2 pre[kLagRegs];
+  auto prefetch = [&](long long r, int part) {
+    if constexpr (kProd)
+      lag_prefetch<kHalf, true>(pre, xspec + (size_t)row_src[r] * xpitch, M + 1 - part,
+                                xspec + (size_t)row_rec[r] * xpitch, part);
+    else
+      lag_prefetch<kHalf>(pre, xspec + r * xpitch, M + 1 - part, nullptr, part);
+  };
   long long row = blockIdx.x;
-  if (row < nrows) lag_prefetch(pre, xspec + row * xpitch, nspec);
+  if (row < nrows) prefetch(row, 0);
   for (; row < nrows; row += gridDim.x) {
+#pragma unroll 1
+    for (int part = 0; part < (kHalf ? 2 : 1); ++part) {
 #pragma unroll
-    for (int i = 0; i < kLagRegs; ++i) {
-      const int k = threadIdx.x + i * kLagThreads;
-      if (k < nspec) lds[k] = pre[i];
-    }
-    __syncthreads();
-    const long long nxt = row + gridDim.x;
-    if (nxt < nrows) lag_prefetch(pre, xspec + nxt * xpitch, nspec);
-    // fold pairs (k, M-k) in place: Z[k] = (X[k] + conj X[M-k]) + i w_k (X[k] - conj X[M-k])
-    for (int k = threadIdx.x; 2 * k <= M; k += blockDim.x) {
-      if (k == 0) {
-        const float a = lds[0].x, b = lds[M].x;  // imaginary parts of DC/Nyquist ignored
-        lds[0] = make_float2(a + b, a - b);
-      } else {
-        const float2 a = lds[k];
-        const float2 b = lds[M - k];
-        const float2 s1 = cadd(a, cconj(b));
-        const float2 d1 = cmul(fold_lookup(fl, k), csub(a, cconj(b)));
-        const float2 zk = make_float2(s1.x - d1.y, s1.y + d1.x);
-        if (2 * k != M) {
-          const float2 s2 = cadd(b, cconj(a));
-          const float2 d2 = cmul(fold_lookup(fl, M - k), csub(b, cconj(a)));
-          lds[M - k] = make_float2(s2.x - d2.y, s2.y + d2.x);
-        }
-        lds[k] = zk;
+      for (int i = 0; i < kLagRegs; ++i) {
+        const int k = threadIdx.x + i * kLagThreads;
+        if (k < M + 1 - part) lds[k] = pre[i];
       }
+      __syncthreads();
+      const bool odd_next = kHalf && part == 0;
+      const long long nxt = odd_next ? row : row + gridDim.x;
+      if (nxt < nrows) prefetch(nxt, odd_next ? 1 : 0);
+      // fold pairs (k, mirror) in place: Z[k] = (X[k] + conj X[m]) + i w_k (X[k] - conj X[m]),
+      // w_m = -conj(w_k); bin 0 and the last bin pair up in Z[0]
+      const int mir = M - part;
+      for (int k = threadIdx.x; 2 * k <= mir; k += blockDim.x) {
+        if (part == 0 && k == 0) {
+          const float a = lds[0].x, b = lds[M].x;  // imaginary parts of DC/Nyquist ignored
+          lds[0] = make_float2(a + b, a - b);
+        } else {
+          float2 w = fold_lookup(fl, k);
+          if (kHalf && part) w = cmul(w, wodd);
+          const float2 a = lds[k];
+          const float2 b = lds[mir - k];
+          const float2 s1 = cadd(a, cconj(b));
+          const float2 d1 = cmul(w, csub(a, cconj(b)));
+          // the mirror's sum and difference are conj(s1) and the conjugate of d1
+          if (2 * k != mir) lds[mir - k] = make_float2(s1.x + d1.y, d1.x - s1.y);
+          lds[k] = make_float2(s1.x - d1.y, s1.y + d1.x);
+        }
+      }
+      __syncthreads();
+      // all passes but the last; the last (largest radix, stride 1) is
+      // evaluated only for the bins that hold kept lags
+      lds_fft_head<kRadixLag>(lds, 1, plan, twl, 1.f, plan.npass - 1);
+      const int out_row = row_out ? row_out[row] : (int)row;
+      float *y = cc + (size_t)out_row * (2 * half_cc + 1);
+      const double wr = task_scale ? weight * (double)task_scale[out_row] : weight;
+      // lag l = 2n + par reads Re (par 0) or Im (par 1) of z[n]
+      const int n_lo = -((half_cc + 1) / 2), n_hi = half_cc / 2;
+      for (int i = threadIdx.x; i <= n_hi - n_lo; i += blockDim.x) {
+        const int n = n_lo + i;
+        float2 z = last_pass_bin(lds, plan, twl, n < 0 ? n + M : n);
+        const int m0 = 2 * n + half_cc;
+        const bool in0 = m0 >= 0, in1 = m0 + 1 <= 2 * half_cc;
+        if (kHalf && part == 0) {
+          if (in0) y[m0] = z.x;
+          if (in1) y[m0 + 1] = z.y;
+          continue;
+        }
+        if constexpr (kHalf) {
+          float2 w = fold_lookup(fl, n < 0 ? -n : n);  // exp(2 pi i |n| / 2M)
+          if (n < 0) w.y = -w.y;
+          z = cmul(w, z);
+          if (in0) z.x += y[m0];
+          if (in1) z.y += y[m0 + 1];
+        }
+        if (in0) y[m0] = (float)((double)z.x * wr);
+        if (in1) y[m0 + 1] = (float)((double)z.y * wr);
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    // all passes but the last; the last (largest radix, stride 1) is
-    // evaluated only for the bins that hold kept lags
-    lds_fft_head<kRadixLag>(lds, 1, plan, twl, 1.f, plan.npass - 1);
-    const int out_row = row_out ? row_out[row] : (int)row;
-    float *y = cc + (size_t)out_row * (2 * half_cc + 1);
-    const double wr = task_scale ? weight * (double)task_scale[out_row] : weight;
-    // lag l = 2n + par reads Re (par 0) or Im (par 1) of Z[n mod M]
-    const int n_lo = -((half_cc + 1) / 2), n_hi = half_cc / 2;
-    for (int i = threadIdx.x; i <= n_hi - n_lo; i += blockDim.x) {
-      const int n = n_lo + i;
-      const float2 z = last_pass_bin(lds, plan, twl, n < 0 ? n + M : n);
-      const int m0 = 2 * n + half_cc;
-      if (m0 >= 0) y[m0] = (float)((double)z.x * wr);
-      if (m0 + 1 <= 2 * half_cc) y[m0 + 1] = (float)((double)z.y * wr);
-    }
-    __syncthreads();
   }
 }
 
@@ -1627,6 +1680,8 @@ struct fxc_xc_plan {
   // nfft/2 beyond one workgroup's LDS: lag synthesis by the four-step
   // inverse transform (work buffer for kLagLargeChunk rows)
   bool large_lag = false;
+  // (even nfft/2 whose half fits: two transforms in LDS, no work buffer)
+  bool half_lag = false;
   float2 *d_lwork = nullptr;
   // pairs
   int nsta = 0;
@@ -1729,7 +1784,16 @@ extern "C" int fxc_xc_plan_create(fxc_xc_plan **out, int nspec, int nstep, float
   int lag_max_radix = kLagMaxRadixDefault;
   if (const char *env = getenv("FXC_XC_LAG_MAX_RADIX")) lag_max_radix = atoi(env) >= 9 ? 9 : 8;
   const bool large_lag = real_lds_count(nfft / 2) > kLdsComplexCapacity;
-  if (large_lag) {
+  // two transforms of nfft/4 in LDS, where that length fits and factors
+  bool half_lag = large_lag && nfft % 4 == 0 && real_lds_count(nfft / 4) <= kLdsComplexCapacity;
+  if (half_lag) {
+    int radix[kMaxPasses], np = 0;
+    half_lag = factor_radices(nfft / 4, radix, &np, lag_max_radix, true) && radix[np - 1] <= 9;
+  }
+  if (half_lag) {
+    const RealFftPlan *rp = nullptr;
+    FXC_TRY(plan_cache_real(nfft / 2, 1, &rp, lag_max_radix, true));
+  } else if (large_lag) {
     int a = 0, b = 0;
     if (!large_factor(nfft / 2, &a, &b)) {
       set_error("fxc_xc_plan_create: nfft %d exceeds one workgroup and has no two-level "
@@ -1742,6 +1806,7 @@ extern "C" int fxc_xc_plan_create(fxc_xc_plan **out, int nspec, int nstep, float
   }
   fxc_xc_plan *p = new fxc_xc_plan();
   p->large_lag = large_lag;
+  p->half_lag = half_lag;
   p->nspec = nspec;
   p->nstep = nstep;
   p->nfft = nfft;
@@ -2307,7 +2372,7 @@ static int xc_lags_rows(fxc_xc_plan *p, const float2 *xs, long long xpitch, long
   FXC_CHECK_ARG(!prod_src || p->large_lag || (p->d_fix_tw && xc_lag_r0_on()),
                 "xc: the one-window product form needs the compile-time or four-step lag");
   const double weight0 = 1.0 / (double)((float)p->nfft * p->dt);
-  if (p->large_lag) {
+  if (p->large_lag && !p->half_lag) {
     // four-step inverse of the folded spectrum, kLagLargeChunk rows at a time
     const int M = p->nfft / 2;
     const LargeFft *lp = nullptr;
@@ -2336,10 +2401,16 @@ static int xc_lags_rows(fxc_xc_plan *p, const float2 *xs, long long xpitch, long
     FXC_TRY(xc_mark(p, kTimeLag, false, st));
     return FXC_OK;
   }
+  const int nreal = p->half_lag ? p->nfft / 2 : p->nfft;  // real length of one LDS transform
   const RealFftPlan *rp = nullptr;
-  FXC_TRY(plan_cache_real(p->nfft, 1, &rp, p->lag_max_radix, true));
-  const size_t lds = (size_t)real_lds_count(p->nfft / 2) * sizeof(float2);
-  auto kern = p->lag_max_radix >= 9 ? lag_kernel<kRadixLag9> : lag_kernel<kRadixLag8>;
+  FXC_TRY(plan_cache_real(nreal, 1, &rp, p->lag_max_radix, true));
+  const size_t lds = (size_t)real_lds_count(nreal / 2) * sizeof(float2);
+  const bool r9 = p->lag_max_radix >= 9;
+  auto kern = r9 ? lag_kernel<kRadixLag9, false, false> : lag_kernel<kRadixLag8, false, false>;
+  if (p->half_lag && prod_src)
+    kern = r9 ? lag_kernel<kRadixLag9, true, true> : lag_kernel<kRadixLag8, true, true>;
+  else if (p->half_lag)
+    kern = r9 ? lag_kernel<kRadixLag9, true, false> : lag_kernel<kRadixLag8, true, false>;
   FXC_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds));
   int dev = 0, ncu = 0;
@@ -2375,9 +2446,12 @@ static int xc_lags_rows(fxc_xc_plan *p, const float2 *xs, long long xpitch, long
                        row_out, d_cc, p->half_cc, weight, task_scale, p->d_fix_tw, p->d_fix_twl,
                        p->d_fix_fold, p->d_fix_roots);
   } else {
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kLagThreads), lds, st, xs, xpitch,
-                       p->nspec, nrows, row_out, d_cc, p->half_cc, weight, task_scale, rp->half.dev,
-                       rp->half.d_tw, rp->d_fold);
+    // exp(2 pi i / nfft): fold factor of bin 2 i + 1 over that of bin 2 i
+    const double a = 2.0 * M_PI / (double)p->nfft;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kLagThreads), lds, st, xs, xpitch, nrows,
+                       row_out, d_cc, p->half_cc, weight, task_scale, rp->half.dev, rp->half.d_tw,
+                       rp->d_fold, make_float2((float)std::cos(a), (float)std::sin(a)), prod_src,
+                       prod_rec);
   }
   FXC_HIP(hipGetLastError());
   FXC_TRY(xc_mark(p, kTimeLag, false, st));

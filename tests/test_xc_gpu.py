@@ -345,3 +345,32 @@ def test_fp32_matrix_tiles(gpu, nsta, nstep):
     want = (z[:, src].conj() * z[:, rec]).mean(axis=0)
     bound = (np.abs(z[:, src]) * np.abs(z[:, rec])).mean(axis=0) * (2 * nstep + 2) * 2.0 ** -24
     assert (np.abs(got - want) <= 2 * bound).all()
+
+
+@pytest.mark.parametrize("nfft,H", [(40000, 1000), (72576, 0), (74088, 2047), (75000, 2500),
+                                    (79380, 39689), (80000, 1)])
+def test_lag_halves(gpu, nfft, H):
+    """Lag transforms of two half-length transforms: the shortest and longest lengths that take
+    them, odd and even halves, no lag beside zero to every lag, odd row pitch; and the one-window
+    product form.  fp32 transforms of 2^16 points round to about log2(n) 2^-24 relative, 1e-6."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    nspec, dt, rows = nfft // 2 + 1, 0.05, 5
+    rng = np.random.default_rng(nfft)
+    X = (rng.standard_normal((rows, nspec)) + 1j * rng.standard_normal((rows, nspec))).astype(np.complex64)
+    lag = np.arange(-H, H + 1) % nfft
+
+    def want(x):
+        return np.fft.irfft(x.astype(np.complex128), n=nfft, axis=-1)[:, lag] / np.float64(np.float32(dt))
+
+    plan = XcPlan(nspec, 1, dt, H, "fp32")
+    got = plan.lags(torch.from_numpy(X).to(gpu)).cpu().numpy()
+    ref = want(X)
+    assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
+    src, rec = np.array([0, 3, 2, 4]), np.array([1, 3, 0, 2])
+    plan.set_pairs(rows, src, rec)
+    got = plan.correlate(torch.from_numpy(X[None]).to(gpu)).cpu().numpy()
+    Z = X.astype(np.complex128)
+    ref = want(Z[src].conj() * Z[rec])
+    assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
