@@ -2,6 +2,7 @@
 
 #include "fxc_fft_device.hpp"
 #include "fxc_fft_large.hpp"
+#include "fxc_workspace.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -22,12 +23,14 @@ std::map<std::tuple<int, int>, std::unique_ptr<BluesteinPlan>> g_blue;
 constexpr int kBlueThreads = 256;
 
 // B_s = DFT_m(b_s) / m, b_s[d] = conj(c_s(d)) for |d| < n (indices mod m),
-// 0 elsewhere; block 0 builds s = -1, block 1 s = +1.  Output keeps the
-// forward transform's digit-reversed layout.
+// 0 elsewhere; block 0 builds s = -1, block 1 s = +1, block 2 the spectrum of
+// the Hilbert kernel h (h[-d] = -h[d], real) in the same places.  Output keeps
+// the forward transform's digit-reversed layout.
 __global__ void __launch_bounds__(kBlueThreads)
 bluestein_bhat_kernel(const float2 *__restrict__ chirp, int n, FftPlanDev plan,
-                      const float2 *__restrict__ tw, float2 *__restrict__ out_f,
-                      float2 *__restrict__ out_i) {
+                      const float2 *__restrict__ tw, const float *__restrict__ hilb,
+                      float2 *__restrict__ out_f, float2 *__restrict__ out_i,
+                      float2 *__restrict__ out_h) {
   extern __shared__ float2 lds[];
   const int m = plan.n;
   float2 *twl = lds + m;
@@ -35,7 +38,12 @@ bluestein_bhat_kernel(const float2 *__restrict__ chirp, int n, FftPlanDev plan,
   const bool fwd = blockIdx.x == 0;
   for (int d = threadIdx.x; d < m; d += blockDim.x) {
     float2 v = make_float2(0.f, 0.f);
-    if (d < n)
+    if (blockIdx.x == 2) {
+      if (d < n)
+        v.x = hilb[d];
+      else if (d > m - n)
+        v.x = -hilb[m - d];
+    } else if (d < n)
       v = chirp[d];
     else if (d > m - n)
       v = chirp[m - d];
@@ -45,7 +53,7 @@ bluestein_bhat_kernel(const float2 *__restrict__ chirp, int n, FftPlanDev plan,
   }
   __syncthreads();
   lds_fft<kRadixAll>(lds, 1, plan, twl, -1.f);
-  float2 *o = fwd ? out_f : out_i;
+  float2 *o = fwd ? out_f : blockIdx.x == 1 ? out_i : out_h;
   const float inv_m = 1.f / (float)m;
   for (int i = threadIdx.x; i < m; i += blockDim.x) o[i] = cscale(lds[i], inv_m);
 }
@@ -54,7 +62,8 @@ void bluestein_destroy(BluesteinPlan *p) {
   dfree(p->d_chirp);
   dfree(p->d_bhat_f);
   dfree(p->d_bhat_i);
-  p->d_chirp = p->d_bhat_f = p->d_bhat_i = nullptr;
+  dfree(p->d_hhat);
+  p->d_chirp = p->d_bhat_f = p->d_bhat_i = p->d_hhat = nullptr;
 }
 
 int bluestein_create(BluesteinPlan *p, int n) {
@@ -69,6 +78,23 @@ int bluestein_create(BluesteinPlan *p, int n) {
     const double a = M_PI * (double)e / (double)n;
     chirp[j] = make_float2((float)std::cos(a), (float)-std::sin(a));
   }
+  // Hilbert kernel of length n: h[d] = (2/n) sum_k sin(2 pi k d / n), 0 < k < n/2,
+  //   = (cos(pi d/n) - cos(pi d (2K+1)/n)) / (n sin(pi d/n)), K = ceil(n/2) - 1
+  std::vector<float> hilb((size_t)n, 0.f);
+  const long long top = 2 * ((n + 1) / 2 - 1) + 1;
+  for (int d = 1; d < n; ++d) {
+    const double a = M_PI * (double)d / (double)n;
+    const double b = M_PI * (double)((long long)d * top % (2LL * n)) / (double)n;
+    hilb[d] = (float)((std::cos(a) - std::cos(b)) / ((double)n * std::sin(a)));
+  }
+  float *d_hilb = nullptr;
+  struct Temp {
+    float **p;
+    ~Temp() { dfree(*p); }
+  } hold{&d_hilb};
+  FXC_TRY(dmalloc((void **)&d_hilb, (size_t)n * sizeof(float)));
+  FXC_HIP(hipMemcpy(d_hilb, hilb.data(), (size_t)n * sizeof(float), hipMemcpyHostToDevice));
+  FXC_TRY(dmalloc((void **)&p->d_hhat, (size_t)m * sizeof(float2)));
   FXC_TRY(dmalloc((void **)&p->d_chirp, (size_t)n * sizeof(float2)));
   FXC_TRY(dmalloc((void **)&p->d_bhat_f, (size_t)m * sizeof(float2)));
   FXC_TRY(dmalloc((void **)&p->d_bhat_i, (size_t)m * sizeof(float2)));
@@ -76,8 +102,8 @@ int bluestein_create(BluesteinPlan *p, int n) {
   const size_t lds = ((size_t)m + tw_lds_count(m)) * sizeof(float2);
   FXC_HIP(hipFuncSetAttribute((const void *)bluestein_bhat_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(bluestein_bhat_kernel, dim3(2), dim3(kBlueThreads), lds, 0, p->d_chirp, n,
-                     p->fwd->dev, p->fwd->d_tw, p->d_bhat_f, p->d_bhat_i);
+  hipLaunchKernelGGL(bluestein_bhat_kernel, dim3(3), dim3(kBlueThreads), lds, 0, p->d_chirp, n,
+                     p->fwd->dev, p->fwd->d_tw, d_hilb, p->d_bhat_f, p->d_bhat_i, p->d_hhat);
   FXC_HIP(hipGetLastError());
   FXC_HIP(hipDeviceSynchronize());
   return FXC_OK;
@@ -162,6 +188,7 @@ void plan_cache_release() {
 }  // namespace fxc
 
 extern "C" void fxc_release_plans(void) {
+  fxc::workspace_release();
   fxc::large_release();
   fxc::plan_cache_release();
 }

@@ -33,6 +33,9 @@ struct BluesteinPlan {
   float2 *d_chirp = nullptr;      // [n] c_{-1}(j) = exp(-i pi j^2 / n), FP64 phases
   float2 *d_bhat_f = nullptr;     // [m] B_{-1}, digit-reversed, / m
   float2 *d_bhat_i = nullptr;     // [m] B_{+1}
+  // [m] spectrum of the length-n Hilbert transform as one convolution of real
+  // rows, digit-reversed, / m (fxc_pws.hip)
+  float2 *d_hhat = nullptr;
 };
 // Smallest m >= 2n-1 that factor_radices accepts (0 when none up to 2^16).
 int bluestein_length(int n);

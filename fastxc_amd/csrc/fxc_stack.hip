@@ -17,14 +17,15 @@
 // lengths with other prime factors (2H+1 is arbitrary) use Bluestein's
 // convolution of a factorable length m >= 2n-1, also in LDS, so every
 // length up to 8192 (PWS) / 6144 (TF-PWS) is served.
+// The PWS kernels are in fxc_pws.hip.
 // The analytic spectra of all groups are computed once; the TF-PWS voice
 // kernel keeps the modulated transforms, the weight W_f(tau) and the
 // Gaussian in LDS, so per voice only the (group-count + 1) spectra are read
 // (from L2) and one complex number is written: the S-transform is never
 // materialised in HBM.  W is accumulated in the FFT's digit-reversed order,
 // which is a consistent permutation of tau, so no reordering pass exists.
-#include "fxc_plan_cache.hpp"
-#include "fastxc_amd.h"
+#include "fxc_stack_fft.hpp"
+#include "fxc_workspace.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -37,96 +38,7 @@ namespace fxc {
 constexpr int kStkThreads = 256;
 constexpr int kStkBatch = 4;       // transforms held in LDS at once (at most)
 constexpr int kVoiceChunk = 32;    // TF-PWS voices per workgroup
-constexpr int kLdsReserve = 16;    // float2 slots left for static LDS
 constexpr int kVoiceThreads = 512; // PWS and TF-PWS voice workgroups
-
-// Length-n transform of the stacks: the direct mixed-radix plan when n
-// factors into the implemented radices (rows of n values, digit-reversed
-// output), else Bluestein's convolution of length m (rows of m values,
-// natural-order output).
-struct StackFftDev {
-  FftPlanDev fwd;              // length ld, sign -1
-  FftPlanDev inv;              // length ld, sign +1
-  int n, ld, blue;
-  const float2 *chirp;         // [n] exp(-i pi j^2 / n) (Bluestein only)
-  const float2 *bhat_f;        // [m] forward-sign convolution kernel spectrum
-  const float2 *bhat_i;        // [m] inverse-sign
-};
-
-struct StackFft {
-  StackFftDev dev{};
-  const float2 *tw_f = nullptr, *tw_i = nullptr;
-  int twc = 0;                 // LDS twiddle slots of both tables
-};
-
-__device__ __forceinline__ int stack_pos(const StackFftDev &F, int k) {
-  return F.blue ? k : fft_pos(F.fwd, k);
-}
-
-// twl: [fwd table | inv table]
-__device__ __forceinline__ void stage_stack_tw(float2 *twl, const StackFftDev &F,
-                                               const float2 *__restrict__ tw_f,
-                                               const float2 *__restrict__ tw_i) {
-  const int cf = kTwFine + F.fwd.ncoarse, ci = kTwFine + F.inv.ncoarse;
-  for (int i = threadIdx.x; i < cf + ci; i += blockDim.x) twl[i] = i < cf ? tw_f[i] : tw_i[i - cf];
-}
-
-// In-place transforms (sgn -1 forward, +1 inverse) of nt rows at stride
-// F.ld whose input is natural order in [0, n).  The caller synchronises
-// before the call; the call ends with a barrier.  Output position of bin k:
-// stack_pos(F, k).
-__device__ __forceinline__ void stack_fft(float2 *buf, int nt, const StackFftDev &F, const float2 *twl, float sgn) {
-  const float2 *twf = twl;
-  const float2 *twi = twl + kTwFine + F.fwd.ncoarse;
-  if (!F.blue) {
-    if (sgn < 0.f)
-      lds_fft<kRadixAll>(buf, nt, F.fwd, twf, -1.f);
-    else
-      lds_fft<kRadixAll>(buf, nt, F.inv, twi, 1.f);
-    return;
-  }
-  const int n = F.n, m = F.ld, total = nt * m;
-  const float cs = sgn < 0.f ? 1.f : -1.f;  // c_s = c_{-1} or its conjugate
-  const float2 *bh = sgn < 0.f ? F.bhat_f : F.bhat_i;
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int j = i % m;
-    float2 v = make_float2(0.f, 0.f);
-    if (j < n) {
-      const float2 c = F.chirp[j];
-      v = cmul(buf[i], make_float2(c.x, cs * c.y));
-    }
-    buf[i] = v;
-  }
-  __syncthreads();
-  lds_fft<kRadixAll>(buf, nt, F.fwd, twf, -1.f);
-  for (int i = threadIdx.x; i < total; i += blockDim.x) buf[i] = cmul(buf[i], bh[i % m]);
-  __syncthreads();
-  lds_fft_dit<kRadixAll>(buf, nt, F.inv, twi, 1.f);
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    const int j = i % m;
-    if (j < n) {
-      const float2 c = F.chirp[j];
-      buf[i] = cmul(buf[i], make_float2(c.x, cs * c.y));
-    }
-  }
-  __syncthreads();
-}
-
-// stack_fft with the direction and the Bluestein choice fixed at compile
-// time.  In a kernel that inlines both directions of the runtime form the
-// compiler copies the plan structure into scratch memory (976 B per lane at
-// the plan sizes here); with both choices fixed, the plan is indexed in the
-// kernel arguments.
-template <int kSgn, bool kBlue>
-__device__ __forceinline__ void stack_fft_dir(float2 *buf, int nt, const StackFftDev &F,
-                                              const float2 *twl) {
-  if constexpr (kBlue)
-    stack_fft(buf, nt, F, twl, (float)kSgn);
-  else if constexpr (kSgn < 0)
-    lds_fft<kRadixAll>(buf, nt, F.fwd, twl, -1.f);
-  else
-    lds_fft<kRadixAll>(buf, nt, F.inv, twl + kTwFine + F.fwd.ncoarse, 1.f);
-}
 
 // Analytic spectra of real rows: A[k] = 2 X[k] for 1 <= k < (n+1)/2, else 0
 // (hilbertTransformKernel after R2C).  Output natural order, [rows][n].
@@ -140,31 +52,6 @@ __device__ __forceinline__ void stack_fft_dir(float2 *buf, int nt, const StackFf
 // stays in its own row, as in a transform per row.
 constexpr int kAnalyticMaxPer = 3;
 constexpr int kLoadBatch = 8;  // loads a thread issues before it uses the first
-
-// Row t[u] and column j[u] of flat index i0 + u step in rows of n, u < kB,
-// from one division (a division per element costs a kernel that issues VALU
-// most of its time several percent).
-template <int kB>
-__device__ __forceinline__ void flat_rows(int i0, int step, int n, int (&t)[kB], int (&j)[kB]) {
-  int tt = i0 / n, jj = i0 - tt * n;
-#pragma unroll
-  for (int u = 0; u < kB; ++u) {
-    t[u] = tt;
-    j[u] = jj;
-    jj += step;
-    while (jj >= n) {
-      jj -= n;
-      ++tt;
-    }
-  }
-}
-
-// Loads of rows a kernel reads exactly once: nontemporal, so the twiddles
-// and tables every workgroup reads stay in L2.
-__device__ __forceinline__ float stream_load(const float *p) { return __builtin_nontemporal_load(p); }
-__device__ __forceinline__ float2 stream_load(const float2 *p) {
-  return __builtin_bit_cast(float2, __builtin_nontemporal_load((const unsigned long long *)p));
-}
 
 template <bool kBlue>
 __global__ void __launch_bounds__(kStkThreads)
@@ -286,92 +173,6 @@ analytic_kernel(const float *__restrict__ x, long long rows, int per_wg, StackFf
       A[(r0 + 2 * t) * n + k] = make_float2(a0.x * u0, a0.y * u0);
       if (2 * t + 1 < nr) A[(r0 + 2 * t + 1) * n + k] = make_float2(a1.x * u1, a1.y * u1);
     }
-  }
-}
-
-// |W|^power from |W|^2: power 1 (the reference) is the square root, power 2
-// the square itself, other powers powf (spec mode).
-__device__ __forceinline__ float mag_pow(float mag2, float power) {
-  if (power == 1.f) return sqrtf(mag2);
-  if (power == 2.f) return mag2;
-  return mag2 > 0.f ? powf(mag2, 0.5f * power) : 0.f;
-}
-
-// PWS: one workgroup per pair.  Thread t owns transform positions
-// p = t + k kThreads (k < kPer), so W stays in registers and the LDS holds
-// only the group rows and the twiddles.
-template <int kThreads, int kPer>
-__global__ void __launch_bounds__(kThreads)
-pws_kernel(const float2 *__restrict__ A, const float *__restrict__ weights,
-           const long long *__restrict__ offsets, const float *__restrict__ lin, StackFftDev F,
-           const float2 *__restrict__ tw_f, const float2 *__restrict__ tw_i, int nbatch,
-           float power, float *__restrict__ out) {
-  extern __shared__ float2 lds[];
-  const int n = F.n, ld = F.ld;
-  float2 *buf = lds;                     // [nbatch][ld]
-  float2 *twl = buf + (size_t)nbatch * ld;
-  stage_stack_tw(twl, F, tw_f, tw_i);
-  const int tid = threadIdx.x;
-  float2 W[kPer];
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) W[k] = make_float2(0.f, 0.f);
-  const int pair = blockIdx.x;
-  const long long g0 = offsets[pair], g1 = offsets[pair + 1];
-  const float invn = 1.f / (float)n;
-  for (long long gb = g0; gb < g1; gb += nbatch) {
-    const int nb = (int)std::min<long long>(nbatch, g1 - gb);
-    __syncthreads();
-    // half a batch: W already holds 2 kPer registers here
-    constexpr int kB = kLoadBatch / 2;
-    for (int i0 = tid; i0 < nb * n; i0 += kB * kThreads) {
-      float2 v[kB];
-      int tu[kB], ju[kB];
-      flat_rows<kB>(i0, kThreads, n, tu, ju);
-#pragma unroll
-      for (int u = 0; u < kB; ++u) {
-        const int i = i0 + u * kThreads;
-        if (i < nb * n) v[u] = stream_load(A + (gb + tu[u]) * n + ju[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < kB; ++u) {
-        const int i = i0 + u * kThreads;
-        if (i < nb * n) buf[tu[u] * ld + ju[u]] = v[u];
-      }
-    }
-    __syncthreads();
-    stack_fft(buf, nb, F, twl, 1.f);
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int p = tid + k * kThreads;
-      if (p < n) {
-        float2 acc = W[k];
-        for (int b = 0; b < nb; ++b) {
-          const float2 z = buf[b * ld + p];
-          const float re = z.x * invn, im = z.y * invn;
-          float mod = sqrtf(re * re + im * im);
-          mod = mod > 1e-7f ? mod : 1e-7f;
-          const float wg = weights[gb + b];
-          acc.x += (re / mod) * wg;
-          acc.y += (im / mod) * wg;
-        }
-        W[k] = acc;
-      }
-    }
-  }
-  __syncthreads();
-  // W is indexed by transform position: publish it in LDS, read it by lag
-  float2 *Ws = buf;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int p = tid + k * kThreads;
-    if (p < n) Ws[p] = W[k];
-  }
-  __syncthreads();
-  const float *l = lin + (size_t)pair * n;
-  float *o = out + (size_t)pair * n;
-  for (int t = tid; t < n; t += kThreads) {
-    const float2 w = Ws[stack_pos(F, t)];
-    o[t] = l[t] * mag_pow(w.x * w.x + w.y * w.y, power);
   }
 }
 
@@ -916,24 +717,7 @@ linear_stack_kernel(const float *__restrict__ x, const long long *__restrict__ o
   out[(size_t)pair * n + j] = (float)(acc / (double)(r1 - r0));
 }
 
-struct StackWork {
-  float2 *A = nullptr;      // [groups + pairs][n]
-  long long *offsets = nullptr;
-  float2 *spec = nullptr;   // [pairs][n]
-  unsigned char *active = nullptr;
-  float *gauss = nullptr;   // [nfreq][(n+1)/2 + 1] Gaussian windows of the voices
-  ~StackWork() {
-    dfree(A);
-    dfree(offsets);
-    dfree(spec);
-    dfree(active);
-    dfree(gauss);
-  }
-};
-
-// Direct plan when n factors, else the Bluestein plan.  create = false
-// only looks the plans up (no device allocation).
-static int stack_fft_plan(int n, StackFft *S, bool create = true) {
+int stack_fft_plan(int n, StackFft *S, bool create) {
   int radix[kMaxPasses], np = 0;
   const FftPlan *pf = nullptr, *pi = nullptr;
   StackFftDev &d = S->dev;
@@ -942,7 +726,7 @@ static int stack_fft_plan(int n, StackFft *S, bool create = true) {
     FXC_TRY(plan_cache_complex(n, 1, &pi, 32, create));
     d.blue = 0;
     d.ld = n;
-    d.chirp = d.bhat_f = d.bhat_i = nullptr;
+    d.chirp = d.bhat_f = d.bhat_i = d.hhat = nullptr;
   } else {
     const BluesteinPlan *bp = nullptr;
     FXC_TRY(plan_cache_bluestein(n, &bp, create));
@@ -953,6 +737,7 @@ static int stack_fft_plan(int n, StackFft *S, bool create = true) {
     d.chirp = bp->d_chirp;
     d.bhat_f = bp->d_bhat_f;
     d.bhat_i = bp->d_bhat_i;
+    d.hhat = bp->d_hhat;
   }
   d.n = n;
   d.fwd = pf->dev;
@@ -963,26 +748,12 @@ static int stack_fft_plan(int n, StackFft *S, bool create = true) {
   return FXC_OK;
 }
 
-// Rows of `ld` the LDS holds beside `fixed` other slots and `extra_rows`
-// reserved rows, capped by the largest group count of the call (0 when none
-// fit).
-static int stack_batch(const StackFft &S, size_t fixed, int extra_rows, const long long *off,
-                       int npairs) {
-  long long gmax = 1;
-  for (int i = 0; i < npairs; ++i) gmax = std::max(gmax, off[i + 1] - off[i]);
-  const long long room = (long long)kLdsComplexCapacity - kLdsReserve - (long long)fixed - S.twc -
-                         (long long)extra_rows * S.dev.ld;
-  if (room < S.dev.ld) return 0;
-  return (int)std::min<long long>(std::min<long long>(kStkBatch, gmax), room / S.dev.ld);
-}
-
-// Device offsets and the analytic spectra of every group and (with_lin,
-// TF-PWS) of every linear stack, into A [groups + pairs][n] and offsets
-// [npairs + 1] (caller's buffers).  PWS weights only the groups' phases, so
-// it leaves the linear stacks' rows out.
+// Device offsets and the analytic spectra of every group and of every linear
+// stack, into A [groups + pairs][n] and offsets [npairs + 1] (caller's
+// buffers).
 static int stack_analytic(const float *d_pre, const float *d_lin, const long long *h_off,
                           int npairs, int n, float2 *A, long long *offsets, const StackFft &S,
-                          hipStream_t st, bool with_lin) {
+                          hipStream_t st) {
   const long long ng = h_off[npairs];
   FXC_HIP(hipMemcpyAsync(offsets, h_off, (size_t)(npairs + 1) * sizeof(long long),
                          hipMemcpyHostToDevice, st));
@@ -999,20 +770,11 @@ static int stack_analytic(const float *d_pre, const float *d_lin, const long lon
                        dim3(kStkThreads), lds, st, d_pre, ng, per, S.dev, S.tw_f, S.tw_i, A);
     FXC_HIP(hipGetLastError());
   }
-  if (!with_lin) return FXC_OK;
   hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div((size_t)npairs, (size_t)(2 * per))),
                      dim3(kStkThreads), lds, st, d_lin, (long long)npairs, per, S.dev, S.tw_f,
                      S.tw_i, A + (size_t)ng * n);
   FXC_HIP(hipGetLastError());
   return FXC_OK;
-}
-
-static int stack_common(const float *d_pre, const float *d_lin, const long long *h_off, int npairs,
-                        int n, StackWork &w, const StackFft &S, hipStream_t st, bool with_lin) {
-  const long long rows = h_off[npairs] + (with_lin ? npairs : 0);
-  FXC_TRY(dmalloc((void **)&w.A, (size_t)std::max<long long>(rows, 1) * n * sizeof(float2)));
-  FXC_TRY(dmalloc((void **)&w.offsets, (size_t)(npairs + 1) * sizeof(long long)));
-  return stack_analytic(d_pre, d_lin, h_off, npairs, n, w.A, w.offsets, S, st, with_lin);
 }
 
 // The voice kernel's per-thread W registers come in steps of 4 positions.
@@ -1150,31 +912,6 @@ int stream_pws_read(const float2 *S, const float *open, const double *acc, const
 
 using namespace fxc;
 
-// PWS proper over analytic spectra A and device offsets already in place.
-static int pws_launch(const StackFft &S, int nbatch, int npairs, const float2 *A,
-                      const float *d_weights, const long long *offsets, const float *d_linear,
-                      float power, float *d_out, hipStream_t st) {
-  const int n = S.dev.n;
-  const int per = (n + kVoiceThreads - 1) / kVoiceThreads;
-  const size_t lds = ((size_t)nbatch * S.dev.ld + S.twc) * sizeof(float2);
-#define FXC_PWS(P)                                                                            \
-  if (per <= P) {                                                                            \
-    auto *k = pws_kernel<kVoiceThreads, P>;                                                  \
-    FXC_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,   \
-                                (int)lds));                                                  \
-    hipLaunchKernelGGL(k, dim3((unsigned)npairs), dim3(kVoiceThreads), lds, st, A, d_weights, \
-                       offsets, d_linear, S.dev, S.tw_f, S.tw_i, nbatch, power, d_out);      \
-    FXC_HIP(hipGetLastError());                                                              \
-    return FXC_OK;                                                                           \
-  }
-  FXC_PWS(4)
-  FXC_PWS(8)
-  FXC_PWS(16)
-#undef FXC_PWS
-  FXC_CHECK_ARG(false, "fxc_pws: length %d too long", n);
-  return FXC_ERR_ARG;
-}
-
 static int check_spec(const fxc_stack_spec *spec, float *power, int *nvoices, int n) {
   *power = 1.f;
   *nvoices = 0;
@@ -1202,29 +939,29 @@ extern "C" int fxc_pws_spec(const float *d_prestack, const float *d_weights,
   FXC_TRY(check_spec(spec, &power, &nvoices, n));
   StackFft S;
   FXC_TRY(stack_fft_plan(n, &S));
-  // the rows must also hold W (n values) after the last batch
-  const int nbatch = std::max(stack_batch(S, 0, 0, h_offsets, npairs),
-                              (int)ceil_div((size_t)n, (size_t)S.dev.ld));
-  FXC_CHECK_ARG((size_t)nbatch * S.dev.ld + S.twc + kLdsReserve <= (size_t)kLdsComplexCapacity,
-                "fxc_pws: length %d too long for the LDS transforms", n);
-  const int per = (n + kVoiceThreads - 1) / kVoiceThreads;
-  FXC_CHECK_ARG(per <= 16, "fxc_pws: length %d too long", n);
+  FXC_TRY(pws_check(S));
   hipStream_t st = (hipStream_t)stream;
-  StackWork w;
-  FXC_TRY(stack_common(d_prestack, d_linear, h_offsets, npairs, n, w, S, st, false));
-  FXC_TRY(pws_launch(S, nbatch, npairs, w.A, d_weights, w.offsets, d_linear, power, d_out, st));
-  FXC_HIP(hipStreamSynchronize(st));  // workspace is released on return
+  const size_t off_bytes = align256((size_t)(npairs + 1) * sizeof(long long));
+  Workspace w;
+  FXC_TRY(w.acquire(off_bytes + pws_scratch_bytes(h_offsets, npairs, n)));
+  long long *offsets = (long long *)w.data();
+  FXC_HIP(hipMemcpyAsync(offsets, h_offsets, (size_t)(npairs + 1) * sizeof(long long),
+                         hipMemcpyHostToDevice, st));
+  FXC_TRY(pws_run(S, d_prestack, d_weights, h_offsets, offsets, d_linear, npairs, n, power,
+                  (float2 *)(w.data() + off_bytes), d_out, st));
+  FXC_HIP(hipStreamSynchronize(st));
+  w.idle();
   return FXC_OK;
 }
 
 // ------------------------------------------------------------------------
 // PWS without allocation, for callers that cannot call hipMalloc (code
 // under HIP graph capture, tight serving loops).  The workspace of
-// fxc_pws (offsets and analytic spectra) lives in a file-scope device array
+// fxc_pws (offsets and partial sums) lives in a file-scope device array
 // of kNoallocScratchBytes per GPU, resolved to a device address once per
 // device by fxc_stack_prepare, which also builds the length's FFT plans.
 // Every call on a GPU shares that GPU's array: calls that overlap on one
-// GPU race.  Nothing in it has to start at zero (offsets and spectra are
+// GPU race.  Nothing in it has to start at zero (offsets and sums are
 // written in full before they are read), so nothing is cleared.
 // ------------------------------------------------------------------------
 namespace fxc {
@@ -1234,8 +971,9 @@ static __device__ __align__(256) unsigned char scratch[kNoallocScratchBytes];
 std::mutex g_scratch_mu;
 std::map<int, unsigned char *> g_scratch_ptr;  // device -> address of `scratch` there
 
-// Bytes of scratch fxc_pws_noalloc needs: offsets, then the spectra on a
-// 256-byte boundary.
+// Bytes of scratch fxc_pws_noalloc admits a call by: offsets, then n complex
+// values per group on a 256-byte boundary (its partial sums need no more:
+// pws_scratch_bytes).
 static size_t noalloc_bytes(long long groups, int npairs, int n, size_t *spec_off) {
   *spec_off = ((size_t)(npairs + 1) * sizeof(long long) + 255) / 256 * 256;
   return *spec_off + (size_t)std::max<long long>(groups, 1) * n * sizeof(float2);
@@ -1279,17 +1017,13 @@ extern "C" int fxc_pws_noalloc(const float *d_prestack, const float *d_weights,
                 "fxc_pws_noalloc: %d pairs with %lld groups of length %d need %zu bytes of "
                 "workspace, more than the %zu of the fixed scratch array",
                 npairs, h_offsets[npairs], n, need, kNoallocScratchBytes);
-  const int nbatch = std::max(stack_batch(S, 0, 0, h_offsets, npairs),
-                              (int)ceil_div((size_t)n, (size_t)S.dev.ld));
-  FXC_CHECK_ARG((size_t)nbatch * S.dev.ld + S.twc + kLdsReserve <= (size_t)kLdsComplexCapacity,
-                "fxc_pws_noalloc: length %d too long for the LDS transforms", n);
-  FXC_CHECK_ARG((n + kVoiceThreads - 1) / kVoiceThreads <= 16, "fxc_pws_noalloc: length %d too long",
-                n);
+  FXC_TRY(pws_check(S));
   hipStream_t st = (hipStream_t)stream;
   long long *offsets = (long long *)base;
-  float2 *A = (float2 *)(base + spec_off);
-  FXC_TRY(stack_analytic(d_prestack, d_linear, h_offsets, npairs, n, A, offsets, S, st, false));
-  FXC_TRY(pws_launch(S, nbatch, npairs, A, d_weights, offsets, d_linear, 1.f, d_out, st));
+  FXC_HIP(hipMemcpyAsync(offsets, h_offsets, (size_t)(npairs + 1) * sizeof(long long),
+                         hipMemcpyHostToDevice, st));
+  FXC_TRY(pws_run(S, d_prestack, d_weights, h_offsets, offsets, d_linear, npairs, n, 1.f,
+                  (float2 *)(base + spec_off), d_out, st));
   // complete on return, as fxc_pws (the host offsets are read by the copy)
   FXC_HIP(hipStreamSynchronize(st));
   return FXC_OK;
@@ -1326,13 +1060,24 @@ extern "C" int fxc_tfpws_spec(const float *d_prestack, const float *d_weights,
   FXC_CHECK_ARG((n + kVoiceThreads - 1) / kVoiceThreads <= 12,
                 "fxc_tfpws: length %d too long for the voice kernel", n);
   hipStream_t st = (hipStream_t)stream;
-  StackWork w;
-  FXC_TRY(stack_common(d_prestack, d_linear, h_offsets, npairs, n, w, S, st, true));
   const int nfreq = n / 2 + 1;
   const int nchunks = (nfreq + kVoiceChunk - 1) / kVoiceChunk;
   const float df = band_limited ? (float)(1.0 / ((double)n * delta)) : 0.f;
-  FXC_TRY(dmalloc((void **)&w.spec, (size_t)npairs * n * sizeof(float2)));
-  FXC_HIP(hipMemsetAsync(w.spec, 0, (size_t)npairs * n * sizeof(float2), st));
+  const int gh = (n + 1) / 2 + 1;  // Gaussian window values per voice
+  const size_t off_bytes = align256((size_t)(npairs + 1) * sizeof(long long));
+  const size_t a_bytes = align256((size_t)(h_offsets[npairs] + npairs) * n * sizeof(float2));
+  const size_t spec_bytes = align256((size_t)npairs * n * sizeof(float2));
+  const size_t act_bytes = align256((size_t)nchunks);
+  const size_t gauss_bytes = nvoices == 0 ? (size_t)nfreq * gh * sizeof(float) : 0;
+  Workspace w;
+  FXC_TRY(w.acquire(off_bytes + a_bytes + spec_bytes + act_bytes + gauss_bytes));
+  long long *offsets = (long long *)w.data();
+  float2 *A = (float2 *)(w.data() + off_bytes);
+  float2 *vspec = (float2 *)(w.data() + off_bytes + a_bytes);
+  unsigned char *active = nullptr;
+  float *gauss = (float *)(w.data() + off_bytes + a_bytes + spec_bytes + act_bytes);
+  FXC_TRY(stack_analytic(d_prestack, d_linear, h_offsets, npairs, n, A, offsets, S, st));
+  FXC_HIP(hipMemsetAsync(vspec, 0, (size_t)npairs * n * sizeof(float2), st));
   if (band_limited) {
     // chunks with no voice inside [fmin, fmax] only carry the linear spectrum
     std::vector<unsigned char> act(nchunks, 0);
@@ -1341,30 +1086,29 @@ extern "C" int fxc_tfpws_spec(const float *d_prestack, const float *d_weights,
       const double lo = a * (1.0 / ((double)n * delta)), hi = b * (1.0 / ((double)n * delta));
       act[c] = !(hi < fmin || lo > fmax);
     }
-    FXC_TRY(dmalloc((void **)&w.active, nchunks));
-    FXC_HIP(hipMemcpyAsync(w.active, act.data(), nchunks, hipMemcpyHostToDevice, st));
+    active = (unsigned char *)(w.data() + off_bytes + a_bytes + spec_bytes);
+    FXC_HIP(hipMemcpyAsync(active, act.data(), nchunks, hipMemcpyHostToDevice, st));
   }
   const long long ng = h_offsets[npairs];
   if (nvoices == 0) {
-    const int gh = (n + 1) / 2 + 1;
-    FXC_TRY(dmalloc((void **)&w.gauss, (size_t)nfreq * gh * sizeof(float)));
     hipLaunchKernelGGL(tfpws_gauss_kernel,
                        dim3((unsigned)ceil_div((size_t)gh, (size_t)kStkThreads), (unsigned)nfreq),
-                       dim3(kStkThreads), 0, st, n, nfreq, w.gauss);
+                       dim3(kStkThreads), 0, st, n, nfreq, gauss);
     FXC_HIP(hipGetLastError());
   }
   size_t lds = ((size_t)(n + 1) / 2 + (size_t)nrows * S.dev.ld + S.twc) * sizeof(float2);
-  FXC_TRY(launch_voice(n, lds, dim3((unsigned)nchunks, (unsigned)npairs), st, w.A,
-                       w.A + (size_t)ng * n, d_weights, w.offsets, S, nrows, nbatch, nfreq,
-                       power, nvoices, (const unsigned char *)w.active, w.gauss, w.spec));
+  FXC_TRY(launch_voice(n, lds, dim3((unsigned)nchunks, (unsigned)npairs), st, A,
+                       A + (size_t)ng * n, d_weights, offsets, S, nrows, nbatch, nfreq, power,
+                       nvoices, active, gauss, vspec));
   lds = ((size_t)S.dev.ld + S.twc) * sizeof(float2);
   FXC_HIP(hipFuncSetAttribute((const void *)tfpws_final_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  hipLaunchKernelGGL(tfpws_final_kernel, dim3((unsigned)npairs), dim3(kStkThreads), lds, st, w.spec,
-                     w.A + (size_t)ng * n, nfreq, band_limited, df, fmin, fmax, taper_hz, S.dev,
+  hipLaunchKernelGGL(tfpws_final_kernel, dim3((unsigned)npairs), dim3(kStkThreads), lds, st, vspec,
+                     A + (size_t)ng * n, nfreq, band_limited, df, fmin, fmax, taper_hz, S.dev,
                      S.tw_f, S.tw_i, d_out);
   FXC_HIP(hipGetLastError());
-  FXC_HIP(hipStreamSynchronize(st));  // workspace is released on return
+  FXC_HIP(hipStreamSynchronize(st));  // the workspace is given back on return
+  w.idle();
   return FXC_OK;
 }
 
@@ -1377,14 +1121,16 @@ extern "C" int fxc_linear_stack(const float *d_records, const long long *h_offse
     FXC_CHECK_ARG(h_offsets[i + 1] > h_offsets[i], "fxc_linear_stack: pair %d has no records", i);
   FXC_CHECK_ARG(npairs <= 65535, "fxc_linear_stack: at most 65535 pairs per call");
   hipStream_t st = (hipStream_t)stream;
-  StackWork w;
-  FXC_TRY(dmalloc((void **)&w.offsets, (size_t)(npairs + 1) * sizeof(long long)));
-  FXC_HIP(hipMemcpyAsync(w.offsets, h_offsets, (size_t)(npairs + 1) * sizeof(long long),
+  Workspace w;
+  FXC_TRY(w.acquire((size_t)(npairs + 1) * sizeof(long long)));
+  long long *offsets = (long long *)w.data();
+  FXC_HIP(hipMemcpyAsync(offsets, h_offsets, (size_t)(npairs + 1) * sizeof(long long),
                          hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(linear_stack_kernel,
                      dim3((unsigned)ceil_div((size_t)n, (size_t)kLinThreads), (unsigned)npairs),
-                     dim3(kLinThreads), 0, st, d_records, w.offsets, n, d_out);
+                     dim3(kLinThreads), 0, st, d_records, offsets, n, d_out);
   FXC_HIP(hipGetLastError());
-  FXC_HIP(hipStreamSynchronize(st));  // workspace is released on return
+  FXC_HIP(hipStreamSynchronize(st));  // the workspace is given back on return
+  w.idle();
   return FXC_OK;
 }

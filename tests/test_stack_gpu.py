@@ -240,3 +240,41 @@ def test_tfpws_even_length_matches_oracle(gpu, N):
         err = rel_l2(out[p], stack.tfpws(s, wg, l, delta=1.0))
         print(f"tfpws even N={N} pair={p} rel_l2={err:.3e}")
         assert err < 1e-4
+
+
+@pytest.mark.parametrize("n", [2, 3, 16, 201, 512, 513, 2003, 2048, 2049, 4096, 4099, 8190, 8192])
+def test_pws_lengths_and_splits(gpu, n):
+    """Lengths at the edges of the PWS kernel's thread and batch choices, even and odd, direct and
+    convolved, for pairs of one to nine groups (odd and even counts, one or several row batches),
+    one pair alone (rows split over workgroups) and many; a non-finite sample stays in its pair.
+    A transform rounds to about 1e-6 of the row's size, so where every envelope is above 0.02 of
+    it the phases are within 5e-5."""
+    import torch
+    from fastxc_amd import ops
+
+    rng = np.random.default_rng(n)
+    for counts in ([9], [1, 2, 3, 4, 5, 9, 1], [3] * 40):
+        off = np.concatenate([[0], np.cumsum(counts)])
+        x = (rng.standard_normal((off[-1], n)) * 10.0 ** rng.integers(-3, 3, (off[-1], 1))).astype(np.float32)
+        w = np.concatenate([np.full(c, 1.0 / c) for c in counts]).astype(np.float32)
+        lin = rng.standard_normal((len(counts), n)).astype(np.float32)
+        args = [torch.from_numpy(a).to(gpu) for a in (x, w)]
+        got = ops.pws(*args, off, torch.from_numpy(lin).to(gpu)).cpu().numpy()
+        for p in range(len(counts)):
+            g = slice(off[p], off[p + 1])
+            if n <= 4:
+                # most phases are those of rounding noise: only bounded
+                assert (np.abs(got[p]) <= np.abs(lin[p]) * 1.001).all()
+                continue
+            ref = stack.pws(x[g], w[g], lin[p])
+            # a phase turns by the transform's rounding over the envelope's size: compare where
+            # no group's envelope is small
+            a = np.abs(np.fft.ifft(stack.analytic_spectrum(x[g]), axis=-1))
+            ok = (a > 0.02 * np.abs(x[g]).max(axis=1, keepdims=True)).all(axis=0)
+            assert ok.mean() > 0.3
+            assert (np.abs(got[p] - ref)[ok] <= 1e-4 * np.abs(lin[p][ok])).all()
+        if len(counts) == 7:
+            x[off[3] + 1, n // 2] = np.inf
+            bad = ops.pws(torch.from_numpy(x).to(gpu), args[1], off, torch.from_numpy(lin).to(gpu)).cpu().numpy()
+            keep = np.arange(7) != 3
+            assert np.array_equal(bad[keep], got[keep]) and not np.isfinite(bad[3]).all()
