@@ -2,6 +2,7 @@
 
 #include "fxc_fft_device.hpp"
 #include "fxc_fft_large.hpp"
+#include "fxc_pfa.hpp"
 #include "fxc_workspace.hpp"
 
 #include <algorithm>
@@ -189,6 +190,7 @@ void plan_cache_release() {
 
 extern "C" void fxc_release_plans(void) {
   fxc::workspace_release();
+  fxc::pfa_release();
   fxc::large_release();
   fxc::plan_cache_release();
 }

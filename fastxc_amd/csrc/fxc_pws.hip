@@ -41,9 +41,12 @@ __device__ __forceinline__ float pow2_scale(float mx) {
 // samples t + k kThreads of every row, so rows stay in registers from their
 // load to their phase and W needs no exchange.  A batch with a non-finite value
 // transforms its rows one by one, so such a value stays in its own row.
+// Three waves per SIMD (168 registers): 2.38 ms for the 6000-pair call against
+// 2.61 at two waves and 3.45 at four, whose 128 registers spill; reading the
+// rows again instead of holding them took 4.06.
 // nsplit 1 writes the stack, otherwise the partial W to part [pair][split][n].
 template <int kThreads, int kPer, int kBatch, bool kBlue>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 3)
 pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
            const long long *__restrict__ offsets, const float *__restrict__ lin, StackFftDev F,
            const float2 *__restrict__ tw_f, const float2 *__restrict__ tw_i, int nsplit,

@@ -37,7 +37,6 @@ namespace fxc {
 
 constexpr int kStkThreads = 256;
 constexpr int kStkBatch = 4;       // transforms held in LDS at once (at most)
-constexpr int kVoiceChunk = 32;    // TF-PWS voices per workgroup
 constexpr int kVoiceThreads = 512; // PWS and TF-PWS voice workgroups
 
 // Analytic spectra of real rows: A[k] = 2 X[k] for 1 <= k < (n+1)/2, else 0
@@ -1097,9 +1096,13 @@ extern "C" int fxc_tfpws_spec(const float *d_prestack, const float *d_weights,
     FXC_HIP(hipGetLastError());
   }
   size_t lds = ((size_t)(n + 1) / 2 + (size_t)nrows * S.dev.ld + S.twc) * sizeof(float2);
-  FXC_TRY(launch_voice(n, lds, dim3((unsigned)nchunks, (unsigned)npairs), st, A,
-                       A + (size_t)ng * n, d_weights, offsets, S, nrows, nbatch, nfreq, power,
-                       nvoices, active, gauss, vspec));
+  if (nvoices == 0 && tfpws_pfa_length(S))
+    FXC_TRY(tfpws_pfa_run(S, A, A + (size_t)ng * n, d_weights, h_offsets, offsets, npairs, nrows,
+                          nbatch, nfreq, power, active, gauss, vspec, st));
+  else
+    FXC_TRY(launch_voice(n, lds, dim3((unsigned)nchunks, (unsigned)npairs), st, A,
+                         A + (size_t)ng * n, d_weights, offsets, S, nrows, nbatch, nfreq, power,
+                         nvoices, active, gauss, vspec));
   lds = ((size_t)S.dev.ld + S.twc) * sizeof(float2);
   FXC_HIP(hipFuncSetAttribute((const void *)tfpws_final_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

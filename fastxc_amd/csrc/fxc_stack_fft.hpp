@@ -7,6 +7,7 @@
 namespace fxc {
 
 constexpr int kLdsReserve = 16;    // float2 slots left for static LDS
+constexpr int kVoiceChunk = 32;    // TF-PWS voices per workgroup
 
 // Length-n transform of the stacks: the direct mixed-radix plan when n
 // factors into the implemented radices (rows of n values, digit-reversed
@@ -142,5 +143,13 @@ size_t pws_scratch_bytes(const long long *h_off, int npairs, int n);
 int pws_run(const StackFft &S, const float *d_pre, const float *d_weights, const long long *h_off,
             const long long *d_off, const float *d_linear, int npairs, int n, float power,
             float2 *d_scratch, float *d_out, hipStream_t st);
+
+// TF-PWS voices of lengths that are products of coprime prime powers (fxc_tfpws.hip);
+// the arguments are those of the general voice kernel's launch.
+bool tfpws_pfa_length(const StackFft &S);
+int tfpws_pfa_run(const StackFft &S, const float2 *Ag, const float2 *Alin, const float *weights,
+                  const long long *h_off, const long long *d_off, int npairs, int nrows,
+                  int nbatch, int nfreq, float power, const unsigned char *active,
+                  const float *gtab, float2 *spec, hipStream_t st);
 
 }  // namespace fxc

@@ -278,3 +278,28 @@ def test_pws_lengths_and_splits(gpu, n):
             bad = ops.pws(torch.from_numpy(x).to(gpu), args[1], off, torch.from_numpy(lin).to(gpu)).cpu().numpy()
             keep = np.arange(7) != 3
             assert np.array_equal(bad[keep], got[keep]) and not np.isfinite(bad[3]).all()
+
+
+@pytest.mark.parametrize("N,counts", [(667, [2, 4]), (667, [5, 2, 9]), (1015, [3]), (2030, [4, 1, 2]),
+                                      (3045, [3, 4]), (4669, [2]), (5336, [5])])
+def test_tfpws_coprime_lengths(gpu, N, counts):
+    """Lengths of pairwise coprime radices, odd and even, at each thread and register choice of
+    their kernel, with every group held, groups in several batches, and the linear stack in a row
+    of its own.  Voices round to about 1e-6 of the stack's size: 2e-5 over their sum."""
+    import torch
+    from fastxc_amd import ops
+
+    rng = np.random.default_rng(N + len(counts))
+    off = np.concatenate([[0], np.cumsum(counts)])
+    pre = _records(rng, off[-1], N)
+    w = np.concatenate([np.full(c, 1.0 / c) for c in counts]).astype(np.float32)
+    lin = np.stack([pre[off[p]:off[p + 1]].mean(axis=0) for p in range(len(counts))]).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    band = (0.05, 0.4, 0.05) if N == 2030 else None
+    out = ops.tfpws(d(pre), d(w), off, d(lin), band=band, delta=1.0).cpu().numpy()
+    for p in range(len(counts)):
+        g = slice(off[p], off[p + 1])
+        if counts[p] == 1 and band is None:
+            continue
+        want = stack.tfpws(pre[g], w[g], lin[p], band=band, delta=1.0)
+        assert rel_l2(out[p], want) < 2e-5
