@@ -11,6 +11,18 @@ namespace fxc {
 namespace {
 std::mutex g_mu;
 std::map<std::pair<int, int>, PfaTables> g_tables;  // (device, n)
+
+int upload(void **dst, const void *src, size_t bytes) {
+  FXC_TRY(dmalloc(dst, bytes));
+  FXC_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyHostToDevice));
+  return FXC_OK;
+}
+
+void free_tables(PfaTables &t) {
+  dfree(t.d_map);
+  dfree(t.d_tpos);
+  dfree(t.d_phase);
+}
 }  // namespace
 
 static bool pfa_plan(int n, FftPlanDev *plan) {
@@ -62,7 +74,7 @@ int pfa_tables(int n, PfaTables *out, bool create) {
     return FXC_OK;
   }
   FXC_CHECK_ARG(create, "index tables of length %d are not prepared on device %d", n, dev);
-  std::vector<unsigned> map((size_t)n, 0u);
+  std::vector<unsigned> map((size_t)n, 0u), tpos((size_t)n, 0u);
   std::vector<float2> phase((size_t)n);
   for (int k = 0; k < n; ++k) {  // k at (k mod R_p)_p
     int i = 0;
@@ -80,22 +92,15 @@ int pfa_tables(int n, PfaTables *out, bool create) {
       t += (long long)(n / p.radix[a]) * b;
     }
     map[(size_t)i] |= (unsigned)(t % n) << 16;
+    tpos[(size_t)(t % n)] = (unsigned)i;
   }
   PfaTables t;
   t.plan = p;
-  int rc = dmalloc((void **)&t.d_map, map.size() * sizeof(unsigned));
-  if (rc == FXC_OK) rc = dmalloc((void **)&t.d_phase, phase.size() * sizeof(float2));
-  if (rc == FXC_OK &&
-      (hipMemcpy(t.d_map, map.data(), map.size() * sizeof(unsigned), hipMemcpyHostToDevice) !=
-           hipSuccess ||
-       hipMemcpy(t.d_phase, phase.data(), phase.size() * sizeof(float2), hipMemcpyHostToDevice) !=
-           hipSuccess)) {
-    set_error("index table upload of length %d failed", n);
-    rc = FXC_ERR_HIP;
-  }
+  int rc = upload((void **)&t.d_map, map.data(), map.size() * sizeof(unsigned));
+  if (rc == FXC_OK) rc = upload((void **)&t.d_tpos, tpos.data(), tpos.size() * sizeof(unsigned));
+  if (rc == FXC_OK) rc = upload((void **)&t.d_phase, phase.data(), phase.size() * sizeof(float2));
   if (rc != FXC_OK) {
-    dfree(t.d_map);
-    dfree(t.d_phase);
+    free_tables(t);
     return rc;
   }
   g_tables[{dev, n}] = t;
@@ -105,10 +110,7 @@ int pfa_tables(int n, PfaTables *out, bool create) {
 
 void pfa_release() {
   std::lock_guard<std::mutex> lk(g_mu);
-  for (auto &kv : g_tables) {
-    dfree(kv.second.d_map);
-    dfree(kv.second.d_phase);
-  }
+  for (auto &kv : g_tables) free_tables(kv.second);
   g_tables.clear();
 }
 

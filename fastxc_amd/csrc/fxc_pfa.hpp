@@ -166,11 +166,12 @@ __device__ __forceinline__ void lds_pfa(float2 *buf, int ntrans, const FftPlanDe
 }
 
 // Plan and device tables of a length (cached per device, freed by
-// fxc_release_plans): map[i] = k | t << 16 of position i, phase[q] =
-// exp(-2 pi i q / n).
+// fxc_release_plans): map[i] = k | t << 16 of position i, tpos[t] = i, phase[q]
+// = exp(-2 pi i q / n).
 struct PfaTables {
   FftPlanDev plan{};
   unsigned *d_map = nullptr;
+  unsigned *d_tpos = nullptr;
   float2 *d_phase = nullptr;
 };
 // Whether n is a product of distinct radices among 2 or 4, 3, 5, 7, 23 and 29

@@ -9,7 +9,9 @@
 // z = s0 x_0 + i s1 x_1, whose spectrum is multiplied by -i sgn(k) in place, in
 // the forward transform's digit-reversed order, and transformed back by the
 // pass order that consumes it: one forward and one inverse transform per two
-// rows, in one LDS row, with no spectrum in HBM.  Rows of other lengths
+// rows, in one LDS row, with no spectrum in HBM.  Lengths of coprime axes
+// (2001 = 3 x 23 x 29) take both transforms without twiddles and their large
+// primes on the matrix instructions (fxc_pfa.hpp).  Rows of other lengths
 // (Bluestein plans) are convolved with the Hilbert kernel directly: also two
 // transforms, of the convolution length, where a Bluestein transform each way
 // takes four.
@@ -19,6 +21,7 @@
 // rows per row, through an HBM workspace of 8 n bytes per row that each call
 // allocated: 6000 pairs of up to 30 rows of 2001 (145 000 rows) 3.5 ms of
 // kernels and about 50 ms of allocation.
+#include "fxc_pfa.hpp"
 #include "fxc_stack_fft.hpp"
 
 #include <algorithm>
@@ -26,6 +29,10 @@
 namespace fxc {
 
 constexpr int kPwsMaxLen = 8192;
+
+// How a length's Hilbert transforms run: mixed-radix passes, convolution
+// (Bluestein lengths), or axes of coprime radices without twiddles.
+enum PwsForm { kPwsMixed, kPwsConv, kPwsAxes };
 
 // Scale s0, s1 are powers of two that bring each row's largest |x| into
 // [1/2, 1), so both rows of a complex row carry the transform's rounding
@@ -36,22 +43,26 @@ __device__ __forceinline__ float pow2_scale(float mx) {
   return ldexpf(1.f, -e);
 }
 
+constexpr int pws_waves(int form, int per) { return per > 8 ? 2 : form == kPwsAxes ? 4 : 3; }
+
 // One workgroup per pair and split: split s of nsplit takes the pair's row
 // pairs [s T / nsplit, (s+1) T / nsplit), kBatch at a time.  Thread t owns the
 // samples t + k kThreads of every row, so rows stay in registers from their
 // load to their phase and W needs no exchange.  A batch with a non-finite value
 // transforms its rows one by one, so such a value stays in its own row.
-// Three waves per SIMD (168 registers): 2.38 ms for the 6000-pair call against
-// 2.61 at two waves and 3.45 at four, whose 128 registers spill; reading the
-// rows again instead of holding them took 4.06.
+// Mixed radix: three waves per SIMD (168 registers), 2.38 ms for the call of
+// 6000 pairs against 2.61 at two waves and 3.45 at four, whose 128 registers
+// spill; reading the rows again instead of holding them took 4.06.  Axes: 1.64.
 // nsplit 1 writes the stack, otherwise the partial W to part [pair][split][n].
-template <int kThreads, int kPer, int kBatch, bool kBlue>
-__global__ void __launch_bounds__(kThreads, 3)
+template <int kThreads, int kPer, int kBatch, int kForm>
+__global__ void __launch_bounds__(kThreads, pws_waves(kForm, kPer))
 pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
            const long long *__restrict__ offsets, const float *__restrict__ lin, StackFftDev F,
-           const float2 *__restrict__ tw_f, const float2 *__restrict__ tw_i, int nsplit,
+           const float2 *__restrict__ tw_f, const float2 *__restrict__ tw_i,
+           const unsigned *__restrict__ map, const unsigned *__restrict__ tpos, int nsplit,
            float power, float2 *__restrict__ part, float *__restrict__ out) {
   extern __shared__ float2 lds[];
+  constexpr bool kBlue = kForm == kPwsConv, kAxes = kForm == kPwsAxes;
   constexpr int kWaves = kThreads / 64;
   __shared__ float red[2][2 * kBatch][kWaves];   // per row and wave: max |x|; sums (Bluestein)
   __shared__ float alt[2 * kBatch][kWaves];      // alternating sums (Bluestein, even n)
@@ -60,7 +71,7 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
   const int n = F.n, ld = F.ld, tid = threadIdx.x;
   float2 *buf = lds;                             // [kBatch][ld]
   float2 *twl = buf + (size_t)kBatch * ld;
-  stage_stack_tw(twl, F, tw_f, tw_i);
+  if constexpr (!kAxes) stage_stack_tw(twl, F, tw_f, tw_i);
   const int pair = blockIdx.x / nsplit, split = blockIdx.x - pair * nsplit;
   const long long g0 = offsets[pair], g1 = offsets[pair + 1];
   const long long T = (g1 - g0 + 1) / 2;         // row pairs
@@ -71,14 +82,26 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
   float2 W[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) W[k] = make_float2(0.f, 0.f);
-  // the digit-reversed positions of the bins this thread multiplies
+  // mixed radix: the digit-reversed positions of the bins this thread
+  // multiplies; axes: the positions of its samples, and the signs of the bins
+  // at its positions (bit k of neg: negative frequency, of off: bin 0 or n/2)
   int pos[kPer];
-  if constexpr (!kBlue) {
+  unsigned neg = 0, off = 0;
+  PfaLanes lanes;
+  if constexpr (kAxes) lanes = pfa_lanes(F.fwd);
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-      const int f = tid + k * kThreads;
-      pos[k] = f < n ? fft_pos(F.fwd, f) : 0;
-    }
+  for (int k = 0; k < kPer; ++k) {
+    const int f = tid + k * kThreads;
+    pos[k] = 0;
+    if constexpr (kForm == kPwsMixed)
+      if (f < n) pos[k] = fft_pos(F.fwd, f);
+    if constexpr (kAxes)
+      if (f < n) {
+        pos[k] = (int)tpos[f];
+        const int q = (int)(map[f] & 0xffffu);
+        if (q >= half) neg |= 1u << k;
+        if (q == 0 || (even && q == n / 2)) off |= 1u << k;
+      }
   }
   if (tid == 0) bad = 0;
   for (long long t0 = split * T / nsplit; t0 < t_end; t0 += kBatch) {
@@ -157,15 +180,32 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
         for (int k = 0; k < kPer; ++k) {
           const int j = tid + k * kThreads;
           if (j < n)
-            buf[t * ld + j] = make_float2(use0 ? xs[t][k].x * s0 : 0.f, use1 ? xs[t][k].y * s1 : 0.f);
+            buf[t * ld + (kAxes ? pos[k] : j)] = make_float2(use0 ? xs[t][k].x * s0 : 0.f, use1 ? xs[t][k].y * s1 : 0.f);
         }
         if constexpr (kBlue)
           for (int j = n + tid; j < ld; j += kThreads) buf[t * ld + j] = make_float2(0.f, 0.f);
       }
       __syncthreads();
       const float2 *twi = twl + kTwFine + F.fwd.ncoarse;
-      lds_fft<kRadixAll>(buf, nt, F.fwd, twl, -1.f);
-      if constexpr (kBlue) {
+      if constexpr (kAxes)
+        lds_pfa(buf, nt, F.fwd, -1.f, lanes);
+      else
+        lds_fft<kRadixAll>(buf, nt, F.fwd, twl, -1.f);
+      if constexpr (kAxes) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) {
+          const int i = tid + k * kThreads;
+          if (i >= n) continue;
+          const float s = (neg >> k) & 1 ? -1.f : 1.f;
+          const bool zero = (off >> k) & 1;
+          for (int t = 0; t < nt; ++t) {
+            const float2 z = buf[t * ld + i];
+            if (zero) (i == 0 ? dc : ny)[t] = z;  // bin 0 sits at position 0
+            // -i s z
+            buf[t * ld + i] = zero ? make_float2(0.f, 0.f) : make_float2(s * z.y, -s * z.x);
+          }
+        }
+      } else if constexpr (kBlue) {
         for (int i = tid; i < ld; i += kThreads) {
           const float2 c = F.hhat[i];
           for (int t = 0; t < nt; ++t) buf[t * ld + i] = cmul(buf[t * ld + i], c);
@@ -187,7 +227,10 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
         }
       }
       __syncthreads();
-      lds_fft_dit<kRadixAll>(buf, nt, F.inv, twi, 1.f);
+      if constexpr (kAxes)
+        lds_pfa(buf, nt, F.fwd, 1.f, lanes);
+      else
+        lds_fft_dit<kRadixAll>(buf, nt, F.inv, twi, 1.f);
 #pragma unroll
       for (int t = 0; t < kBatch; ++t) {
         if (t >= nt) break;
@@ -224,7 +267,7 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
         for (int k = 0; k < kPer; ++k) {
           const int j = tid + k * kThreads;
           if (j >= n) continue;
-          const float2 z = buf[t * ld + j];
+          const float2 z = buf[t * ld + (kAxes ? pos[k] : j)];
           const float s = even && (j & 1) ? -1.f : 1.f;
           float2 acc = W[k];
           auto add = [&](float re, float im, float w) {
@@ -282,6 +325,11 @@ size_t pws_scratch_bytes(const long long *h_off, int npairs, int n) {
   return s > 1 ? (size_t)npairs * s * n * sizeof(float2) : 0;
 }
 
+int pws_prepare(int n) {
+  PfaTables t;
+  return pfa_length(n) ? pfa_tables(n, &t) : FXC_OK;
+}
+
 int pws_check(const StackFft &S) {
   FXC_CHECK_ARG((size_t)S.dev.ld + S.twc + kLdsReserve <= (size_t)kLdsComplexCapacity,
                 "fxc_pws: length %d too long for the LDS transforms", S.dev.n);
@@ -291,6 +339,10 @@ int pws_check(const StackFft &S) {
 
 namespace {
 struct PwsArgs {
+  StackFftDev F;
+  const float2 *tw_f, *tw_i;
+  int form, twc;
+  PfaTables axes;
   const float *pre, *weights;
   const long long *off;
   const float *lin;
@@ -300,16 +352,17 @@ struct PwsArgs {
   float *out;
 };
 
-template <int kThreads, int kPer, int kBatch>
-int pws_launch(const StackFft &S, const PwsArgs &a, hipStream_t st) {
-  auto *k = S.dev.blue ? pws_kernel<kThreads, kPer, kBatch, true>
-                       : pws_kernel<kThreads, kPer, kBatch, false>;
-  const size_t lds = ((size_t)kBatch * S.dev.ld + S.twc) * sizeof(float2);
+template <int kThreads, int kPer, int kBatch, bool kAxes = false>
+int pws_launch(const PwsArgs &a, hipStream_t st) {
+  auto *k = pws_kernel<kThreads, kPer, kBatch, kAxes ? kPwsAxes : kPwsMixed>;
+  if constexpr (!kAxes)
+    if (a.form == kPwsConv) k = pws_kernel<kThreads, kPer, kBatch, kPwsConv>;
+  const size_t lds = ((size_t)kBatch * a.F.ld + a.twc) * sizeof(float2);
   FXC_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)lds));
   hipLaunchKernelGGL(k, dim3((unsigned)a.npairs * (unsigned)a.nsplit), dim3(kThreads), lds, st,
-                     a.pre, a.weights, a.off, a.lin, S.dev, S.tw_f, S.tw_i, a.nsplit, a.power,
-                     a.part, a.out);
+                     a.pre, a.weights, a.off, a.lin, a.F, a.tw_f, a.tw_i, a.axes.d_map,
+                     a.axes.d_tpos, a.nsplit, a.power, a.part, a.out);
   FXC_HIP(hipGetLastError());
   return FXC_OK;
 }
@@ -317,21 +370,40 @@ int pws_launch(const StackFft &S, const PwsArgs &a, hipStream_t st) {
 
 int pws_run(const StackFft &S, const float *d_pre, const float *d_weights, const long long *h_off,
             const long long *d_off, const float *d_linear, int npairs, int n, float power,
-            float2 *d_scratch, float *d_out, hipStream_t st) {
+            float2 *d_scratch, float *d_out, hipStream_t st, bool create) {
   FXC_TRY(pws_check(S));
-  const PwsArgs a{d_pre, d_weights, d_off, d_linear, npairs, pws_splits(h_off, npairs),
-                  power, d_scratch, d_out};
+  PwsArgs a{S.dev, S.tw_f, S.tw_i, S.dev.blue ? kPwsConv : kPwsMixed, S.twc, {}, d_pre, d_weights,
+            d_off, d_linear, npairs, pws_splits(h_off, npairs), power, d_scratch, d_out};
+  if (pfa_length(n)) {
+    FXC_TRY(pfa_tables(n, &a.axes, create));
+    a.form = kPwsAxes;
+    a.F.fwd = a.axes.plan;
+    a.twc = 0;
+  }
   // Row pairs per batch: as many as keep a thread's rows within 32 registers,
   // so that the large-radix passes (n / 29 butterflies per row) have work for
-  // the workgroup's waves.
-  if (n <= 512)
-    FXC_TRY((pws_launch<256, 2, 4>(S, a, st)));
-  else if (n <= 2048)
-    FXC_TRY((pws_launch<256, 8, 2>(S, a, st)));
-  else if (n <= 4096 && 2 * (size_t)S.dev.ld + S.twc + kLdsReserve <= (size_t)kLdsComplexCapacity)
-    FXC_TRY((pws_launch<512, 8, 2>(S, a, st)));
-  else
-    FXC_TRY((pws_launch<512, 16, 1>(S, a, st)));
+  // the workgroup's waves; one in the axes form, whose matrix passes need only
+  // 16 butterflies per wave and which four waves per SIMD serve better (2001:
+  // 1.41 ms of 6000 pairs against 1.46 at two row pairs and three waves).
+  const bool two = 2 * (size_t)S.dev.ld + S.twc + kLdsReserve <= (size_t)kLdsComplexCapacity;
+  if (a.form == kPwsAxes) {
+    if (n <= 512)
+      FXC_TRY((pws_launch<256, 2, 4, true>(a, st)));
+    else if (n <= 2048)
+      FXC_TRY((pws_launch<256, 8, 1, true>(a, st)));
+    else if (n <= 4096)
+      FXC_TRY((pws_launch<512, 8, 1, true>(a, st)));
+    else
+      FXC_TRY((pws_launch<512, 16, 1, true>(a, st)));
+  } else if (n <= 512) {
+    FXC_TRY((pws_launch<256, 2, 4>(a, st)));
+  } else if (n <= 2048) {
+    FXC_TRY((pws_launch<256, 8, 2>(a, st)));
+  } else if (n <= 4096 && two) {
+    FXC_TRY((pws_launch<512, 8, 2>(a, st)));
+  } else {
+    FXC_TRY((pws_launch<512, 16, 1>(a, st)));
+  }
   if (a.nsplit > 1) {
     hipLaunchKernelGGL(pws_join_kernel, dim3((unsigned)ceil_div((size_t)n, 256), (unsigned)npairs),
                        dim3(256), 0, st, d_scratch, d_linear, n, a.nsplit, power, d_out);

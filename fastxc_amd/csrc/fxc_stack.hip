@@ -985,6 +985,7 @@ extern "C" int fxc_stack_prepare(int n) {
   FXC_HIP(hipGetDevice(&dev));
   StackFft S;
   FXC_TRY(stack_fft_plan(n, &S, true));
+  FXC_TRY(pws_prepare(n));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   if (!g_scratch_ptr.count(dev)) {
     void *p = nullptr;
@@ -1022,7 +1023,7 @@ extern "C" int fxc_pws_noalloc(const float *d_prestack, const float *d_weights,
   FXC_HIP(hipMemcpyAsync(offsets, h_offsets, (size_t)(npairs + 1) * sizeof(long long),
                          hipMemcpyHostToDevice, st));
   FXC_TRY(pws_run(S, d_prestack, d_weights, h_offsets, offsets, d_linear, npairs, n, 1.f,
-                  (float2 *)(base + spec_off), d_out, st));
+                  (float2 *)(base + spec_off), d_out, st, false));
   // complete on return, as fxc_pws (the host offsets are read by the copy)
   FXC_HIP(hipStreamSynchronize(st));
   return FXC_OK;

@@ -138,11 +138,13 @@ int stack_fft_plan(int n, StackFft *S, bool create = true);
 // Argument error for lengths the PWS kernels do not serve.
 int pws_check(const StackFft &S);
 // PWS of every pair (offsets: device copy of h_off).  scratch_bytes from
-// pws_scratch_bytes; the caller synchronises.
+// pws_scratch_bytes; the caller synchronises.  create = false: no device
+// allocation (pws_prepare ran for the length).
+int pws_prepare(int n);
 size_t pws_scratch_bytes(const long long *h_off, int npairs, int n);
 int pws_run(const StackFft &S, const float *d_pre, const float *d_weights, const long long *h_off,
             const long long *d_off, const float *d_linear, int npairs, int n, float power,
-            float2 *d_scratch, float *d_out, hipStream_t st);
+            float2 *d_scratch, float *d_out, hipStream_t st, bool create = true);
 
 // TF-PWS voices of lengths that are products of coprime prime powers (fxc_tfpws.hip);
 // the arguments are those of the general voice kernel's launch.
