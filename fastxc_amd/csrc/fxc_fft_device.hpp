@@ -253,11 +253,12 @@ __device__ __forceinline__ float2 tw_lookup(const float2 *tw, int e) {
 }
 
 // Multiplies v[1..R-1] by w^(q*e), q = 1..R-1 (exponents modulo n).  Up to
-// radix 16 the powers come from one table read and a chain of products
-// (at most 14 roundings, ~1e-6 relative); larger radices read each power.
+// radix 16 the powers come from one table read and products: a chain up to
+// radix 9 (at most 7 roundings), above it w^(4a + b) = (w^4)^a w^b (at most 5,
+// where a chain would take 14); larger radices read each power.
 template <int R>
 __device__ __forceinline__ void apply_twiddles(float2 *v, const float2 *tw, int e, int n) {
-  if constexpr (R <= 16) {
+  if constexpr (R <= 9) {
     const float2 w = tw_lookup(tw, e);
     float2 wq = w;
     v[1] = cmul(v[1], w);
@@ -265,6 +266,21 @@ __device__ __forceinline__ void apply_twiddles(float2 *v, const float2 *tw, int 
     for (int q = 2; q < R; ++q) {
       wq = cmul(wq, w);
       v[q] = cmul(v[q], wq);
+    }
+  } else if constexpr (R <= 16) {
+    const float2 w1 = tw_lookup(tw, e);
+    const float2 w2 = cmul(w1, w1), w3 = cmul(w2, w1), w4 = cmul(w2, w2);
+    v[1] = cmul(v[1], w1);
+    v[2] = cmul(v[2], w2);
+    v[3] = cmul(v[3], w3);
+    float2 wa = w4;
+#pragma unroll
+    for (int q = 4; q < R; q += 4) {
+      v[q] = cmul(v[q], wa);
+      if (q + 1 < R) v[q + 1] = cmul(v[q + 1], cmul(wa, w1));
+      if (q + 2 < R) v[q + 2] = cmul(v[q + 2], cmul(wa, w2));
+      if (q + 3 < R) v[q + 3] = cmul(v[q + 3], cmul(wa, w3));
+      if (q + 4 < R) wa = cmul(wa, w4);
     }
   } else {
     int eq = 0;

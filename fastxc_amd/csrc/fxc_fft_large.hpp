@@ -25,6 +25,7 @@ struct LargeFft {
   int M = 0, N1 = 0, N2 = 0, sign = -1;
   const FftPlan *p1 = nullptr;  // N1 points
   const FftPlan *p2 = nullptr;  // N2 points
+  const FftPlan *pq = nullptr;  // M/2 points, where one workgroup's LDS holds them
   float2 *d_tw = nullptr;       // [M] exp(sign 2 pi i m / M)
   float2 *d_half = nullptr;     // [M + 1] exp(sign 2 pi i k / (2M)) (real fold / unfold)
 };

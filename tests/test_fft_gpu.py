@@ -37,3 +37,26 @@ def test_r2c_c2r(gpu, n, in_len):
     assert np.all(X[:, 0].imag == 0) and np.all(X[:, -1].imag == 0)
     y = ops.fft_c2r(torch.from_numpy(want.astype(np.complex64)).to(gpu), n).cpu().numpy()
     assert rel_l2(y, np.fft.irfft(want, n=n) * n) < 1e-6
+
+
+@pytest.mark.parametrize("n,in_len,rows", [(40960, 40959, 3), (40000, 1, 2), (72900, 72900, 300),
+                                           (75000, 70001, 2), (79380, 79380, 2)])
+def test_real_halves(gpu, n, in_len, rows):
+    """Real transforms of two half-length LDS transforms: about the shortest and the longest
+    length that takes them, odd and even halves, zero padding that ends inside a sample group,
+    more rows than workgroups."""
+    import torch
+    from fastxc_amd import ops
+
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((rows, in_len)).astype(np.float32)
+    X = ops.fft_r2c(torch.from_numpy(x).to(gpu), n=n).cpu().numpy()
+    want = np.fft.rfft(x.astype(np.float64), n=n)
+    assert rel_l2(X, want) < 1e-6
+    assert np.all(X[:, 0].imag == 0) and np.all(X[:, -1].imag == 0)
+    z = (rng.standard_normal((rows, n // 2 + 1)) + 1j * rng.standard_normal((rows, n // 2 + 1)))
+    z = z.astype(np.complex64)
+    ref = np.fft.irfft(z.astype(np.complex128), n=n) * n
+    for out_len in (n, in_len, n // 2 + 1):
+        y = ops.fft_c2r(torch.from_numpy(z).to(gpu), n, out_len=out_len).cpu().numpy()
+        assert rel_l2(y, ref[:, :out_len]) < 1e-6
