@@ -105,65 +105,80 @@ __global__ void station_scale_kernel(const unsigned int *__restrict__ amax_bits,
 // read 256 contiguous bytes.  One workgroup converts 64 stations x 16 bins:
 // each block of 8 windows is staged through LDS so the reads run along the
 // bins and the writes along the stations.
-constexpr int kSplitSta = 64;
 constexpr int kSplitBins = 16;
 constexpr int kSplitThreads = 256;
-constexpr int kSplitLoads = 8 * kSplitSta * kSplitBins / kSplitThreads;  // per thread and block
+constexpr int kSplitSta = 64;      // stations per workgroup
+constexpr int kSplitTile = 8 * 64; // station-windows staged at once
+constexpr int kSplitLoads = kSplitTile * kSplitBins / kSplitThreads;  // per thread and block
 
-// One workgroup's part: source stations [s0, s0 + 64) of spectra
-// [nstep][nsta][nspec], bins [k0, k0 + 16).  Source station s lands at operand
-// row sta_off + s of an operand with nsta_dst rows; station-windows whose
-// valid byte ([nstep][nsta], when given) is 0 enter as zeros.
-template <int kMode>
+// One workgroup's part: source stations [s0, s0 + kSta) of spectra
+// [nstep][nsta][nspec], bins [k0, k0 + 16), kWin = 512 / kSta windows at a time.
+// Source station s lands at operand row sta_off + s of an operand with nsta_dst
+// rows; station-windows whose valid byte ([nstep][nsta], when given) is 0 enter
+// as zeros.  The valid bytes of a block become one mask per station, applied as
+// the values leave the tile: testing each value's byte where it is loaded cost
+// as many loads again (24 segments, 12 GB of spectra: 11.8 ms for the split).
+template <int kMode, int kSta>
 __device__ __forceinline__ void split_part(const float2 *__restrict__ spec, int nstep, int nsta,
                                            int nspec, int kh, const float *__restrict__ inv_scale,
                                            const unsigned char *__restrict__ valid, int sta_off,
                                            int nsta_dst, int s0, int k0,
                                            unsigned short *__restrict__ hi,
-                                           unsigned short *__restrict__ lo) {
-  __shared__ float2 tile[8][kSplitSta][kSplitBins + 1];
+                                           unsigned short *__restrict__ lo, float2 *tile,
+                                           unsigned *mask) {
+  constexpr int kWin = kSplitTile / kSta;
+  constexpr int kPitch = kSplitBins + 1;  // tile [kWin][kSta][kPitch]
   const int tid = threadIdx.x;
-  const int ngrp = kh / 4;  // K groups of 8 values: kh/8 real + kh/8 imaginary
-  for (int wb = 0; wb < kh; wb += 8) {
-    // load windows wb..wb+7: 16 lanes read one station's 16 bins (128 bytes);
-    // every load of the block is issued before the first LDS store, so their
-    // latencies overlap
+  const int ngrp = kh / 4;  // K groups of 8 values (4 windows)
+  for (int wb = 0; wb < kh; wb += kWin) {
+    // 16 lanes read one station's 16 bins (128 bytes); every load of the block
+    // is issued before the first LDS store, so their latencies overlap
     float2 z[kSplitLoads];
 #pragma unroll
     for (int j = 0; j < kSplitLoads; ++j) {
       const int i = tid + j * kSplitThreads;
       const int kk = i % kSplitBins;
-      const int ss = (i / kSplitBins) % kSplitSta;
-      const int ww = i / (kSplitBins * kSplitSta);
+      const int ss = (i / kSplitBins) % kSta;
+      const int ww = i / (kSplitBins * kSta);
       const int w = wb + ww, sidx = s0 + ss, k = k0 + kk;
       z[j] = make_float2(0.f, 0.f);
-      if (w < nstep && sidx < nsta && k < nspec && (!valid || valid[(size_t)w * nsta + sidx]))
-        z[j] = spec[((size_t)w * nsta + sidx) * nspec + k];
+      if (w < nstep && sidx < nsta && k < nspec) z[j] = spec[((size_t)w * nsta + sidx) * nspec + k];
+    }
+    unsigned m = 0;
+    if (valid && tid < kSta && s0 + tid < nsta) {
+#pragma unroll 8
+      for (int ww = 0; ww < kWin; ++ww)
+        if (wb + ww < nstep && valid[(size_t)(wb + ww) * nsta + s0 + tid]) m |= 1u << ww;
     }
     __syncthreads();  // the previous block's conversion is done with the tile
 #pragma unroll
     for (int j = 0; j < kSplitLoads; ++j) {
       const int i = tid + j * kSplitThreads;
-      tile[i / (kSplitBins * kSplitSta)][(i / kSplitBins) % kSplitSta][i % kSplitBins] = z[j];
+      tile[(i / kSplitBins) * kPitch + i % kSplitBins] = z[j];
     }
+    if (valid && tid < kSta) mask[tid] = m;
     __syncthreads();
-    // convert: thread = (station, bin); 64 consecutive threads write 64
+    // convert: thread = (station, bin); kSta consecutive threads write
     // consecutive stations' 16-byte groups
-    for (int i = tid; i < kSplitSta * kSplitBins; i += kSplitThreads) {
-      const int ss = i % kSplitSta;
-      const int kk = i / kSplitSta;
+    for (int i = tid; i < kSta * kSplitBins; i += kSplitThreads) {
+      const int ss = i % kSta;
+      const int kk = i / kSta;
       const int sidx = s0 + ss, k = k0 + kk;
       if (sidx >= nsta || k >= nspec) continue;
       const float sc = (kMode == FXC_PREC_FP16 || kMode == FXC_PREC_FP16X3)
                            ? inv_scale[sta_off + sidx]
                            : 1.f;
+      const unsigned vm = valid ? mask[ss] : ~0u;
 #pragma unroll
-      for (int part = 0; part < 2; ++part) {  // windows wb + 4 part .. + 3
+      for (int part = 0; part < kWin / 4; ++part) {  // windows wb + 4 part .. + 3
+        const int g = wb / 4 + part;
+        if (kWin > 8 && g >= ngrp) break;  // kh is a multiple of 8
         unsigned short h[8], l[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          const float2 z = tile[4 * part + j / 2][ss][kk];
-          const float v = ((j & 1) ? z.y : z.x) * sc;
+          const int ww = 4 * part + j / 2;
+          const float2 z = tile[(ww * kSta + ss) * kPitch + kk];
+          const float v = (vm >> ww) & 1 ? ((j & 1) ? z.y : z.x) * sc : 0.f;
           if (kMode == FXC_PREC_FP16) {
             h[j] = __builtin_bit_cast(unsigned short, (_Float16)v);
             l[j] = 0;
@@ -177,7 +192,6 @@ __device__ __forceinline__ void split_part(const float2 *__restrict__ spec, int 
             l[j] = bf16_bits_rne(v - bf16_bits_to_float(hb));
           }
         }
-        const int g = 2 * (wb / 8) + part;
         const size_t o = (((size_t)k * ngrp + g) * nsta_dst + sta_off + sidx) * 8;
         uint4 hv;
         hv.x = h[0] | ((unsigned)h[1] << 16); hv.y = h[2] | ((unsigned)h[3] << 16);
@@ -194,13 +208,38 @@ __device__ __forceinline__ void split_part(const float2 *__restrict__ spec, int 
   }
 }
 
+// The workgroup's stations 64 x 8 windows at a time, or, where at most 32 or 16
+// of its stations exist, in the shape that keeps the lanes on data: 32 x 16, 16
+// x 32 (small segments, and the last workgroup of an array).
+template <int kMode>
+__device__ __forceinline__ void split_stations(const float2 *__restrict__ spec, int nstep, int nsta,
+                                               int nspec, int kh,
+                                               const float *__restrict__ inv_scale,
+                                               const unsigned char *__restrict__ valid,
+                                               int sta_off, int nsta_dst, int s0, int k0,
+                                               unsigned short *__restrict__ hi,
+                                               unsigned short *__restrict__ lo) {
+  __shared__ float2 tile[kSplitTile * (kSplitBins + 1)];
+  __shared__ unsigned mask[kSplitSta];
+  const int left = nsta - s0;
+  if (left > 32)
+    split_part<kMode, 64>(spec, nstep, nsta, nspec, kh, inv_scale, valid, sta_off, nsta_dst, s0, k0,
+                          hi, lo, tile, mask);
+  else if (left > 16)
+    split_part<kMode, 32>(spec, nstep, nsta, nspec, kh, inv_scale, valid, sta_off, nsta_dst, s0, k0,
+                          hi, lo, tile, mask);
+  else
+    split_part<kMode, 16>(spec, nstep, nsta, nspec, kh, inv_scale, valid, sta_off, nsta_dst, s0, k0,
+                          hi, lo, tile, mask);
+}
+
 template <int kMode>
 __global__ void __launch_bounds__(kSplitThreads)
 split_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int nspec, int kh,
              const float *__restrict__ inv_scale, unsigned short *__restrict__ hi,
              unsigned short *__restrict__ lo, int bin0) {
-  split_part<kMode>(spec, nstep, nsta, nspec, kh, inv_scale, nullptr, 0, nsta,
-                    blockIdx.y * kSplitSta, bin0 + blockIdx.x * kSplitBins, hi, lo);
+  split_stations<kMode>(spec, nstep, nsta, nspec, kh, inv_scale, nullptr, 0, nsta,
+                        blockIdx.y * kSplitSta, bin0 + blockIdx.x * kSplitBins, hi, lo);
 }
 
 // Uneven segments in one launch: segment z = blockIdx.z holds spectra
@@ -223,9 +262,9 @@ split_segments_kernel(const float2 *__restrict__ spec, const unsigned char *__re
   const SplitSeg sg = segs[blockIdx.z];
   const int s0 = blockIdx.y * kSplitSta;
   if (s0 >= sg.nsta) return;  // the whole workgroup leaves before any barrier
-  split_part<kMode>(spec + sg.spec_off, sg.nstep, sg.nsta, nspec, kh, nullptr,
-                    valid ? valid + sg.valid_off : nullptr, sg.sta_off, nsta_dst, s0,
-                    blockIdx.x * kSplitBins, hi, lo);
+  split_stations<kMode>(spec + sg.spec_off, sg.nstep, sg.nsta, nspec, kh, nullptr,
+                        valid ? valid + sg.valid_off : nullptr, sg.sta_off, nsta_dst, s0,
+                        blockIdx.x * kSplitBins, hi, lo);
 }
 
 // ---------------------------------------------------------------------------

@@ -251,3 +251,29 @@ def test_batch_autotune_searches_and_caches(gpu, tmp_path):
     assert res2["cached"] and (res2["grouping"], res2["max_rows"]) == (res["grouping"], res["max_rows"])
     b.close()
     b2.close()
+
+
+def test_split_shapes_and_gap_values(gpu):
+    """Station counts at the edges of the split's workgroup shapes (16, 32 and 64 stations and
+    their remainders) and window counts on both sides of a block; the values under a gap are
+    non-finite, as a StepPack may hold anything there, and must not be used."""
+    import torch
+    from fastxc_amd.ops import XcBatch
+
+    rng = np.random.default_rng(71)
+    seg, nfft, H, dt = 300, 720, 40, 0.1
+    nsta = [2, 16, 17, 32, 33, 64, 65, 80, 97, 129]
+    nstep = [33, 8, 9, 16, 17, 31, 32, 41, 8, 24]
+    specs = [_spectra(rng, w, n, seg, nfft, dt) for n, w in zip(nsta, nstep)]
+    valid = [(rng.random((w, n)) >= 0.1).astype(np.uint8) for n, w in zip(nsta, nstep)]
+    dirty = [s.copy() for s in specs]
+    for z, v in zip(dirty, valid):
+        z[v == 0] = np.nan
+    vmask = XcBatch.pack([torch.from_numpy(v) for v in valid], gpu)
+    for grouping in (0, 1):
+        b = XcBatch(nfft // 2 + 1, dt, H, nsta, nstep, gaps="exclude")
+        b.set_grouping(grouping)
+        cc = b.correlate(XcBatch.pack([torch.from_numpy(z) for z in dirty], gpu), vmask).cpu().numpy()
+        clean = [np.where(v[:, :, None] == 0, 0, z).astype(np.complex64) for z, v in zip(specs, valid)]
+        _check_segments(b, cc, clean, valid, "exclude", nfft, H, dt)
+        b.close()
