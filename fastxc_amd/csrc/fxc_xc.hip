@@ -722,7 +722,8 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
   extern __shared__ __align__(16) float2 stage[];  // [kTilePairs][kBinChunk], swizzled
   __shared__ int rows[kTilePairs];
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  // (a uniform wave index keeps the operand bases in scalar registers)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int lane_r = lane & 15, lane_g = lane >> 4;
   constexpr bool kSplit = kMode == FXC_PREC_BF16X3 || kMode == FXC_PREC_FP16X3;
