@@ -158,6 +158,30 @@ __device__ __forceinline__ void stream_store(float2 *p, float2 v) {
   __builtin_nontemporal_store(__builtin_bit_cast(unsigned long long, v), (unsigned long long *)p);
 }
 
+// The pending time-domain normalisation of one sample (d: its weight).
+__device__ __forceinline__ float normalised(float v, int mode, float d) {
+  if (mode == kLoadRunabs) {
+    v = (!isfinite(d) || d < kMinValD) ? 0.f : v / d;
+    if (!isfinite(v)) v = 0.f;
+    v = v > kMaxVal ? kMaxVal : (v < -kMaxVal ? -kMaxVal : v);
+  } else if (mode == kLoadOnebit) {
+    v = v > 0.f ? 1.f : (v < 0.f ? -1.f : 0.f);
+  }
+  return v;
+}
+
+// One bin of the output spectrum: x dt, sanitised, optionally phase-only.
+__device__ __forceinline__ float2 output_bin(float2 v, float dt, int phase_only) {
+  v = cscale(v, dt);
+  if (!cfinite(v)) v = make_float2(0.f, 0.f);
+  if (phase_only) {
+    const float a = hypotf(v.x, v.y);
+    v = (!isfinite(a) || a <= kMinVal) ? make_float2(0.f, 0.f) : cscale(v, 1.f / a);
+    if (!cfinite(v)) v = make_float2(0.f, 0.f);
+  }
+  return v;
+}
+
 // Loads one row of the time series into the float view of LDS applying the
 // pending time-domain normalisation (reference order: x/w with 0 for an
 // invalid weight, non-finite -> 0, clip to +-MAXVAL; or sign(x)), then zero
@@ -181,19 +205,7 @@ __device__ inline void load_row(float *ldsf, int twoM, const float *__restrict__
     for (int u = 0; u < kB; ++u) {
       const int i = i0 + u * blockDim.x;
       if (i >= twoM) continue;
-      float v = 0.f;
-      if (i < seg) {
-        v = xv[u];
-        if (mode == kLoadRunabs) {
-          const float d = wv[u];
-          v = (!isfinite(d) || d < kMinValD) ? 0.f : v / d;
-          if (!isfinite(v)) v = 0.f;
-          v = v > kMaxVal ? kMaxVal : (v < -kMaxVal ? -kMaxVal : v);
-        } else if (mode == kLoadOnebit) {
-          v = v > 0.f ? 1.f : (v < 0.f ? -1.f : 0.f);
-        }
-      }
-      ldsf[i] = v;
+      ldsf[i] = i < seg ? normalised(xv[u], mode, wv[u]) : 0.f;
     }
   }
   __syncthreads();
@@ -419,12 +431,12 @@ s2s_weight_tile_kernel(const void *__restrict__ data, long long row_pitch, int w
 
 // ---------------------------------------------------------------------------
 // Whitening forward: load (normalised) row, R2C(seg) x dt, sanitise; write
-// X[k] and |X[k]|, k < seg/2+1 (core/spectrum.cu:178-230 up to the weight).
+// X[k], k < seg/2+1 (core/spectrum.cu:178-230 up to the weight).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kS2sThreads)
 s2s_whiten_fwd_kernel(const float *__restrict__ x, int seg, int nch, int mode,
                       const float *__restrict__ w, RealTables ts, float dt,
-                      float2 *__restrict__ X, float *__restrict__ amp, long long fpitch) {
+                      float2 *__restrict__ X, long long fpitch) {
   extern __shared__ float2 lds[];
   const FftPlanDev &plan = ts.plan;
   const int M = plan.n;
@@ -436,12 +448,10 @@ s2s_whiten_fwd_kernel(const float *__restrict__ x, int seg, int nch, int mode,
            w ? w + (size_t)frame * seg : nullptr);
   lds_fft(lds, 1, plan, tw_fwd, -1.f);
   float2 *Xr = X + (size_t)row * fpitch;
-  float *ar = amp + (size_t)row * fpitch;
   spectral_emit(lds, plan, fold, [&](int k, float2 v) {
     v = cscale(v, dt);
     if (!cfinite(v)) v = make_float2(0.f, 0.f);
     stream_store(Xr + k, v);
-    stream_store(ar + k, sqrtf(v.x * v.x + v.y * v.y));
   });
 }
 
@@ -534,15 +544,7 @@ s2s_whiten_inv_kernel(const float2 *__restrict__ X, long long fpitch, const floa
   lds_fft(lds, 1, to.plan, two_fwd, -1.f);
   float2 *o = out + (size_t)row * nspec;
   spectral_emit(lds, to.plan, fold_o, [&](int k, float2 v) {
-    if (k >= nspec) return;
-    v = cscale(v, dt);
-    if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    if (phase_only) {
-      const float a = hypotf(v.x, v.y);
-      v = (!isfinite(a) || a <= kMinVal) ? make_float2(0.f, 0.f) : cscale(v, 1.f / a);
-      if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    }
-    stream_store(o + k, v);
+    if (k < nspec) stream_store(o + k, output_bin(v, dt, phase_only));
   });
 }
 
@@ -564,15 +566,7 @@ s2s_output_kernel(const float *__restrict__ x, int seg, int nch, int mode,
   lds_fft(lds, 1, plan, tw_fwd, -1.f);
   float2 *o = out + (size_t)row * nspec;
   spectral_emit(lds, plan, fold, [&](int k, float2 v) {
-    if (k >= nspec) return;
-    v = cscale(v, dt);
-    if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    if (phase_only) {
-      const float a = hypotf(v.x, v.y);
-      v = (!isfinite(a) || a <= kMinVal) ? make_float2(0.f, 0.f) : cscale(v, 1.f / a);
-      if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    }
-    stream_store(o + k, v);
+    if (k < nspec) stream_store(o + k, output_bin(v, dt, phase_only));
   });
 }
 
@@ -700,11 +694,9 @@ s2sL_pre_kernel(const float *__restrict__ traces, int npts, int nfiles,
   }
 }
 
-// X[k] = sanitise(X[k] dt) (times resp[k] when given; |X| into amp when
-// given), k < nbin, every row.
+// X[k] = sanitise(X[k] dt) (times resp[k] when given), k < nbin, every row.
 __global__ void s2sL_spec_kernel(float2 *__restrict__ X, long long pitch, int nbin, float dt,
-                                 const float *__restrict__ resp, float *__restrict__ amp,
-                                 long long apitch) {
+                                 const float *__restrict__ resp) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= nbin) return;
   const long long row = blockIdx.y;
@@ -712,7 +704,6 @@ __global__ void s2sL_spec_kernel(float2 *__restrict__ X, long long pitch, int nb
   if (!cfinite(v)) v = make_float2(0.f, 0.f);
   if (resp) v = cscale(v, resp[k]);
   X[row * pitch + k] = v;
-  if (amp) amp[row * apitch + k] = sqrtf(v.x * v.x + v.y * v.y);
 }
 
 // Pending time-domain normalisation applied in place (load_row's rules).
@@ -1171,38 +1162,21 @@ __device__ __forceinline__ void fused_emit(float2 *lds, int seg, const float2 *_
   fixed_fft_fwd<FPN, kS2sThreads>(lds, tw0n, twln);
   fixed_r2c_emit<FPN>(lds, foldn, [&](int k, float2 v) {
     if (kOut && k >= nspec) return;
-    v = cscale(v, dt);
-    if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    if (kOut && phase_only) {
-      const float a = hypotf(v.x, v.y);
-      v = (!isfinite(a) || a <= kMinVal) ? make_float2(0.f, 0.f) : cscale(v, 1.f / a);
-      if (!cfinite(v)) v = make_float2(0.f, 0.f);
-    }
-    stream_store(dst + k, v);
+    stream_store(dst + k, output_bin(v, dt, kOut && phase_only));
   }, (int)((reinterpret_cast<uintptr_t>(dst) >> 3) & 15));
 }
 
-template <class FPF, class FPN, bool kOut>
-__global__ void __launch_bounds__(kS2sThreads)
-s2s_front_kernel(const float *__restrict__ traces, int npts, int nfiles,
-                 const int *__restrict__ steps, int shift, int seg, int taper_size,
-                 FixedTables tf, FixedTables tn, const float *__restrict__ resp0, float dt,
-                 double inv_weight, int norm_mode, int runabs_win, int phase_only, int comp_sums,
-                 float2 *__restrict__ dst, long long dpitch, int nspec) {
-  extern __shared__ float2 lds[];
-  constexpr int kData = (FPF::kM > FPN::kM ? FPF::kM : FPN::kM) + 1;
-  float2 *twlf = lds + kData;
-  float2 *twln = twlf + fixed_lds_tw_count<FPF>();
-  float2 *foldf = twln + fixed_lds_tw_count<FPN>();
-  float2 *foldn = foldf + fold_lds_count(FPF::kM);
-  float *bs = (float *)(foldn + fold_lds_count(FPN::kM));
-  stage_fixed<FPF>(twlf, foldf, tf);
-  stage_fixed<FPN>(twln, foldn, tn);
+// Window cut, preprocess and broad-band prefilter of one row in LDS: x[0..seg)
+// in the float view (compute.cu:34-86).
+template <class FPF>
+__device__ __forceinline__ void prefilter_row(float2 *lds, const float *__restrict__ src,
+                                              long long off, int npts, int seg, int taper_size,
+                                              const FixedTables &tf, const float2 *twlf,
+                                              const float2 *foldf,
+                                              const float *__restrict__ resp0, float dt,
+                                              double inv_weight) {
   float *ldsf = (float *)lds;
-  const int row = blockIdx.x;
-  const int step = row / nfiles, file = row - step * nfiles;
-  preprocess_row<2 * FPF::kM>(ldsf, traces + (size_t)file * npts,
-                              (long long)steps[step] * shift, npts, seg, taper_size);
+  preprocess_row<2 * FPF::kM>(ldsf, src, off, npts, seg, taper_size);
   constexpr int Mf = FPF::kM;
   // this thread's response values, loaded while the forward transform runs
   float2 rsp[fixed_pair_trips<FPF>()];
@@ -1225,12 +1199,87 @@ s2s_front_kernel(const float *__restrict__ traces, int npts, int nfiles,
   fixed_fft_inv<FPF, kS2sThreads>(lds, tf.tw0, twlf);
   for (int i = threadIdx.x; i < seg; i += blockDim.x) ldsf[i] = (float)((double)ldsf[i] * inv_weight);
   __syncthreads();
+}
+
+template <class FPF, class FPN, bool kOut>
+__global__ void __launch_bounds__(kS2sThreads)
+s2s_front_kernel(const float *__restrict__ traces, int npts, int nfiles,
+                 const int *__restrict__ steps, int shift, int seg, int taper_size,
+                 FixedTables tf, FixedTables tn, const float *__restrict__ resp0, float dt,
+                 double inv_weight, int norm_mode, int runabs_win, int phase_only, int comp_sums,
+                 float2 *__restrict__ dst, long long dpitch, int nspec) {
+  extern __shared__ float2 lds[];
+  constexpr int kData = (FPF::kM > FPN::kM ? FPF::kM : FPN::kM) + 1;
+  float2 *twlf = lds + kData;
+  float2 *twln = twlf + fixed_lds_tw_count<FPF>();
+  float2 *foldf = twln + fixed_lds_tw_count<FPN>();
+  float2 *foldn = foldf + fold_lds_count(FPF::kM);
+  float *bs = (float *)(foldn + fold_lds_count(FPN::kM));
+  stage_fixed<FPF>(twlf, foldf, tf);
+  stage_fixed<FPN>(twln, foldn, tn);
+  float *ldsf = (float *)lds;
+  const int row = blockIdx.x;
+  const int step = row / nfiles, file = row - step * nfiles;
+  prefilter_row<FPF>(lds, traces + (size_t)file * npts, (long long)steps[step] * shift, npts, seg,
+                     taper_size, tf, twlf, foldf, resp0, dt, inv_weight);
   if (comp_sums)
     normalise_row<AccComp>(ldsf, seg, norm_mode, runabs_win, bs);
   else
     normalise_row<Acc64>(ldsf, seg, norm_mode, runabs_win, bs);
   fused_emit<FPN, kOut>(lds, seg, tn.tw0, twln, foldn, dt, phase_only,
                         dst + (size_t)row * dpitch, nspec);
+}
+
+// Whitened bins -> x[0..seg) = C2R x inv_weight in the float view of LDS.
+// get(i, k, a, b): the thread's i-th pair a = X[k], b = X[Ms - k].
+template <class FPS, class G>
+__device__ __forceinline__ void whitened_inverse(float2 *lds, int seg, const FixedTables &ts,
+                                                 const float2 *twls, const float2 *folds,
+                                                 double inv_weight, const G &get) {
+  constexpr int Ms = FPS::kM;
+  // fold into the digit-reversed positions of the inverse (every value read
+  // before any is written): Z[k] = S + i D with S = X[k] + conj X[Ms-k],
+  // D = conj(w_k) (X[k] - conj X[Ms-k]), w_k = exp(-i pi k / Ms).  Bin Ms-k
+  // folds from the same two values, Z[Ms-k] = conj S + i conj D (w_{Ms-k} =
+  // -conj w_k), so a thread takes the pair (k, Ms-k) for k = 0 .. Ms/2; k = 0
+  // (with X[Ms]) and k = Ms/2 fold alone.  Two loads per pair and 2 x
+  // kPairPer values held across the barrier.
+  static_assert(Ms % 2 == 0, "pairwise fold needs an even half length");
+  constexpr int kHalf = Ms / 2;
+  constexpr int kPairPer = (kHalf + 1 + kS2sThreads - 1) / kS2sThreads;
+  float2 zk[kPairPer], zm[kPairPer];
+#pragma unroll
+  for (int i = 0; i < kPairPer; ++i) {
+    const int k = threadIdx.x + i * kS2sThreads;
+    if (k <= kHalf) {
+      float2 a, b;
+      get(i, k, a, b);
+      b = cconj(b);
+      if (k == 0) {
+        a.y = 0.f;
+        b.y = 0.f;
+      }
+      const float2 sv = cadd(a, b);
+      const float2 dv = cmul(cconj(fold_lookup(folds, k)), csub(a, b));
+      zk[i] = make_float2(sv.x - dv.y, sv.y + dv.x);
+      zm[i] = make_float2(sv.x + dv.y, dv.x - sv.y);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPairPer; ++i) {
+    const int k = threadIdx.x + i * kS2sThreads;
+    if (k <= kHalf) {
+      lds[fixed_pos<FPS>(k)] = zk[i];
+      if (k != 0 && k != kHalf) lds[fixed_pos<FPS>(Ms - k)] = zm[i];
+    }
+  }
+  __syncthreads();
+  fixed_fft_inv<FPS, kS2sThreads>(lds, ts.tw0, twls);
+  float *ldsf = (float *)lds;
+  for (int i = threadIdx.x; i < seg; i += blockDim.x)
+    ldsf[i] = (float)((double)ldsf[i] * inv_weight);
+  __syncthreads();
 }
 
 template <class FPS, class FPN, bool kOut>
@@ -1306,54 +1355,199 @@ s2s_back_kernel(float2 *X, long long fpitch, int seg, int i1, int i2, int i3, in
     }
   }
   __syncthreads();
-  // fold into the digit-reversed positions of the inverse (every value read
-  // before any is written): Z[k] = S + i D with S = X[k] + conj X[Ms-k],
-  // D = conj(w_k) (X[k] - conj X[Ms-k]), w_k = exp(-i pi k / Ms).  Bin Ms-k
-  // folds from the same two values, Z[Ms-k] = conj S + i conj D (w_{Ms-k} =
-  // -conj w_k), so a thread takes the pair (k, Ms-k) for k = 0 .. Ms/2; k = 0
-  // (with X[Ms]) and k = Ms/2 fold alone.  Two loads per pair and 2 x
-  // kPairPer values held across the barrier.
-  static_assert(Ms % 2 == 0, "pairwise fold needs an even half length");
-  constexpr int kHalf = Ms / 2;
-  constexpr int kPairPer = (kHalf + 1 + kS2sThreads - 1) / kS2sThreads;
-  float2 zk[kPairPer], zm[kPairPer];
-#pragma unroll
-  for (int i = 0; i < kPairPer; ++i) {
-    const int k = threadIdx.x + i * kS2sThreads;
-    if (k <= kHalf) {
-      float2 a = lds[k];
-      float2 b = cconj(lds[Ms - k]);
-      if (k == 0) {
-        a.y = 0.f;
-        b.y = 0.f;
-      }
-      const float2 sv = cadd(a, b);
-      const float2 dv = cmul(cconj(fold_lookup(folds, k)), csub(a, b));
-      zk[i] = make_float2(sv.x - dv.y, sv.y + dv.x);
-      zm[i] = make_float2(sv.x + dv.y, dv.x - sv.y);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < kPairPer; ++i) {
-    const int k = threadIdx.x + i * kS2sThreads;
-    if (k <= kHalf) {
-      lds[fixed_pos<FPS>(k)] = zk[i];
-      if (k != 0 && k != kHalf) lds[fixed_pos<FPS>(Ms - k)] = zm[i];
-    }
-  }
-  __syncthreads();
-  fixed_fft_inv<FPS, kS2sThreads>(lds, ts.tw0, twls);
+  whitened_inverse<FPS>(lds, seg, ts, twls, folds, inv_weight_seg,
+                        [&](int, int k, float2 &a, float2 &b) {
+                          a = lds[k];
+                          b = lds[Ms - k];
+                        });
   float *ldsf = (float *)lds;
-  for (int i = threadIdx.x; i < seg; i += blockDim.x)
-    ldsf[i] = (float)((double)ldsf[i] * inv_weight_seg);
-  __syncthreads();
   if (comp_sums)
     normalise_row<AccComp>(ldsf, seg, norm_mode, runabs_win, bs);
   else
     normalise_row<Acc64>(ldsf, seg, norm_mode, runabs_win, bs);
   fused_emit<FPN, kOut>(lds, seg, tn.tw0, twln, foldn, dt, phase_only, dst + (size_t)row * dpitch,
                         nspec);
+}
+
+// ---------------------------------------------------------------------------
+// The same production lengths where a row does not own its weights (several
+// channels share a frame's running means) or the normalisation works in bands
+// (RUN-ABS-MF): the steps of the five-kernel path, cut at the running means
+// over a frame's channels, with the transforms on the compile-time plans.
+//   prefilter: window cut, preprocess, prefilter -> x
+//   row:       x, pending normalisation, R2C(seg) -> X or R2C(nfft_out) -> out
+//   shared:    X / w (w the frame's weights), taper, C2R(seg) -> x, or on to
+//              R2C(nfft_out) -> out
+// One workgroup holds a row in the LDS of its compute unit, so the vector and
+// LDS work of the transforms is what each kernel costs, and a runtime plan's
+// index arithmetic is most of that (29 against 12 us per transform of 18000
+// points).  14100 rows of three-channel frames: prefilter 3.54 -> 2.62 ms, row
+// 2.29 -> 1.70 ms, shared with the output transform 4.19 -> 2.53 ms.
+// ---------------------------------------------------------------------------
+template <class FPF>
+__global__ void __launch_bounds__(kS2sThreads)
+s2s_fixed_prefilter_kernel(const float *__restrict__ traces, int npts, int nfiles,
+                           const int *__restrict__ steps, int shift, int seg, int taper_size,
+                           FixedTables tf, const float *__restrict__ resp0, float dt,
+                           double inv_weight, float *__restrict__ xout) {
+  extern __shared__ float2 lds[];
+  float2 *twlf = lds + FPF::kM + 1;
+  float2 *foldf = twlf + fixed_lds_tw_count<FPF>();
+  stage_fixed<FPF>(twlf, foldf, tf);
+  const int row = blockIdx.x;
+  const int step = row / nfiles, file = row - step * nfiles;
+  prefilter_row<FPF>(lds, traces + (size_t)file * npts, (long long)steps[step] * shift, npts, seg,
+                     taper_size, tf, twlf, foldf, resp0, dt, inv_weight);
+  float2 *y = (float2 *)(xout + (size_t)row * seg);  // seg is even
+  for (int i = threadIdx.x; 2 * i < seg; i += blockDim.x) stream_store(y + i, lds[i]);
+}
+
+// FPS is the window's plan (seg = 2 FPS::kM): x is read as FPS::kM pairs.
+template <class FPS, class FPN, bool kOut>
+__global__ void __launch_bounds__(kS2sThreads)
+s2s_fixed_row_kernel(const float *__restrict__ x, int nch, int mode, const float *__restrict__ w,
+                     FixedTables tn, float dt, int phase_only, float2 *__restrict__ dst,
+                     long long dpitch, int nspec) {
+  extern __shared__ float2 lds[];
+  constexpr int kData = (FPS::kM > FPN::kM ? FPS::kM : FPN::kM) + 1;
+  float2 *twln = lds + kData;
+  float2 *foldn = twln + fixed_lds_tw_count<FPN>();
+  stage_fixed<FPN>(twln, foldn, tn);
+  const int row = blockIdx.x;
+  constexpr int kPer = (FPS::kM + kS2sThreads - 1) / kS2sThreads;
+  const float2 *xr = (const float2 *)x + (size_t)row * FPS::kM;
+  const float2 *wr = (const float2 *)w + (size_t)(row / nch) * FPS::kM;
+  // every load of the row and of its weights before the first is used
+  float2 v[kPer], d[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = threadIdx.x + j * kS2sThreads;
+    v[j] = d[j] = make_float2(0.f, 0.f);
+    if (i < FPS::kM) {
+      v[j] = stream_load(xr + i);
+      if (mode == kLoadRunabs) d[j] = wr[i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = threadIdx.x + j * kS2sThreads;
+    if (i < FPS::kM)
+      lds[i] = make_float2(normalised(v[j].x, mode, d[j].x), normalised(v[j].y, mode, d[j].y));
+  }
+  __syncthreads();
+  fused_emit<FPN, kOut>(lds, 2 * FPS::kM, tn.tw0, twln, foldn, dt, phase_only,
+                        dst + (size_t)row * dpitch, nspec);
+}
+
+// Where s2s_fixed_shared_kernel takes the row after the inverse.  ToRow: to
+// x.  ToFixed: the output transform on a compile-time plan.  ToRuntime: on a
+// runtime plan (the output length follows the lag, the other two do not).
+struct ToRow {
+  float *x;
+  __host__ __device__ constexpr int len() const { return 0; }
+  __host__ __device__ constexpr int slots() const { return 0; }
+  __device__ void stage(float2 *) const {}
+  template <class FPS>
+  __device__ void run(float2 *lds, const float2 *, int row) const {
+    float2 *y = (float2 *)x + (size_t)row * FPS::kM;
+    for (int i = threadIdx.x; i < FPS::kM; i += blockDim.x) stream_store(y + i, lds[i]);
+  }
+};
+template <class FP>
+struct ToFixed {
+  FixedTables t;
+  float dt;
+  int phase_only, nspec;
+  float2 *out;
+  __host__ __device__ constexpr int len() const { return FP::kM; }
+  __host__ __device__ constexpr int slots() const {
+    return fixed_lds_tw_count<FP>() + fused_fold_count(FP::kM);
+  }
+  __device__ void stage(float2 *tab) const {
+    stage_fixed<FP>(tab, tab + fixed_lds_tw_count<FP>(), t);
+  }
+  template <class FPS>
+  __device__ void run(float2 *lds, const float2 *tab, int row) const {
+    fused_emit<FP, true>(lds, 2 * FPS::kM, t.tw0, tab, tab + fixed_lds_tw_count<FP>(), dt,
+                         phase_only, out + (size_t)row * nspec, nspec);
+  }
+};
+struct ToRuntime {
+  RealTables t;
+  float dt;
+  int phase_only, nspec;
+  float2 *out;
+  __host__ __device__ int len() const { return t.plan.n; }
+  __host__ __device__ int slots() const { return tw_lds_count(t.plan.n) + fold_lds_count(t.plan.n); }
+  __device__ void stage(float2 *tab) const {
+    const int ntw = tw_lds_count(t.plan.n);
+    for (int i = threadIdx.x; i < ntw; i += blockDim.x) tab[i] = t.tw_fwd[i];
+    for (int i = threadIdx.x; i < fold_lds_count(t.plan.n); i += blockDim.x) tab[ntw + i] = t.fold[i];
+  }
+  template <class FPS>
+  __device__ void run(float2 *lds, const float2 *tab, int row) const {
+    for (int i = FPS::kM + (int)threadIdx.x; i < t.plan.n; i += blockDim.x)
+      lds[i] = make_float2(0.f, 0.f);
+    __syncthreads();
+    lds_fft(lds, 1, t.plan, tab, -1.f);
+    float2 *o = out + (size_t)row * nspec;
+    spectral_emit(lds, t.plan, tab + tw_lds_count(t.plan.n), [&](int k, float2 v) {
+      if (k < nspec) stream_store(o + k, output_bin(v, dt, phase_only));
+    });
+  }
+};
+
+// float2 slots of s2s_fixed_shared_kernel: [data][tables of FPS][tables of To]
+template <class FPS, class To>
+__host__ __device__ constexpr int fixed_shared_slots(const To &to) {
+  return (FPS::kM > to.len() ? FPS::kM : to.len()) + 1 + fixed_lds_tw_count<FPS>() +
+         fused_fold_count(FPS::kM) + to.slots();
+}
+
+template <class FPS, class To>
+__global__ void __launch_bounds__(kS2sThreads)
+s2s_fixed_shared_kernel(const float2 *__restrict__ X, long long fpitch,
+                        const float *__restrict__ ww, int nch, const float *__restrict__ staper,
+                        FixedTables ts, double inv_weight, To to) {
+  extern __shared__ float2 lds[];
+  constexpr int Ms = FPS::kM;
+  float2 *twls = lds + (Ms > to.len() ? Ms : to.len()) + 1;
+  float2 *folds = twls + fixed_lds_tw_count<FPS>();
+  float2 *tab = folds + fused_fold_count(Ms);
+  stage_fixed<FPS>(twls, folds, ts);
+  to.stage(tab);
+  const int row = blockIdx.x;
+  const float2 *Xr = X + (size_t)row * fpitch;
+  const float *wr = ww + (size_t)(row / nch) * fpitch;
+  auto whitened_from = [&](float2 v, float d, float tp) -> float2 {
+    v = (!isfinite(d) || d < kMinValD) ? make_float2(0.f, 0.f) : make_float2(v.x / d, v.y / d);
+    v = cscale(v, tp);
+    if (!cfinite(v)) v = make_float2(0.f, 0.f);
+    return v;
+  };
+  // every load of the pairs (k, Ms - k) before the first is used
+  constexpr int kPairPer = (Ms / 2 + 1 + kS2sThreads - 1) / kS2sThreads;
+  float2 xa[kPairPer], xb[kPairPer];
+  float da[kPairPer], db[kPairPer], ta[kPairPer], tb[kPairPer];
+#pragma unroll
+  for (int i = 0; i < kPairPer; ++i) {
+    const int k = threadIdx.x + i * kS2sThreads;
+    if (k <= Ms / 2) {
+      xa[i] = stream_load(Xr + k);
+      xb[i] = stream_load(Xr + Ms - k);
+      da[i] = wr[k];
+      db[i] = wr[Ms - k];
+      ta[i] = staper[k];
+      tb[i] = staper[Ms - k];
+    }
+  }
+  __syncthreads();  // the staged tables
+  whitened_inverse<FPS>(lds, 2 * Ms, ts, twls, folds, inv_weight,
+                        [&](int i, int, float2 &a, float2 &b) {
+                          a = whitened_from(xa[i], da[i], ta[i]);
+                          b = whitened_from(xb[i], db[i], tb[i]);
+                        });
+  to.template run<FPS>(lds, tab, row);
 }
 
 }  // namespace fxc
@@ -1379,7 +1573,7 @@ struct fxc_s2s_plan {
   long long cap_rows = 0, cap_frames = 0;
   float *d_x = nullptr, *d_w = nullptr, *d_xb = nullptr, *d_total = nullptr;
   float2 *d_X = nullptr, *d_base = nullptr;
-  float *d_amp = nullptr, *d_ww = nullptr;
+  float *d_ww = nullptr;
   int *d_steps = nullptr;
   int cap_steps = 0;
   // long-window path (transforms beyond one workgroup's LDS)
@@ -1388,8 +1582,9 @@ struct fxc_s2s_plan {
   float2 *d_L = nullptr;             // [rows][lpitch]
   float2 *d_Lw = nullptr;            // four-step work, kLargeChunk rows
   long long cap_L = 0;
-  // fused one-channel path at the production lengths (s2s_front/back_kernel)
-  bool fused = false;
+  // compile-time plans at the production lengths: the fused one-channel path
+  // (s2s_front/back_kernel), or the s2s_fixed_* kernels
+  bool fixed = false, fixed_out = false, fused = false;
   float2 *d_fx = nullptr;  // pass-0 and LDS base twiddles of the three plans
   float *d_staper = nullptr;  // spectral taper factor of each whitening bin
   int comp_sums = 0;          // spec mode: compensated-FP32 running means (fxc_s2s_set_sums)
@@ -1421,15 +1616,17 @@ static int set_lds(K kern, size_t bytes) {
   return FXC_OK;
 }
 
-// The fused path applies to one channel, every normalisation but RUN-ABS-MF,
-// and the production lengths; FXC_S2S_FUSED=0 keeps the five-kernel path.
-static int s2s_fused_setup(fxc_s2s_plan *p) {
+// At the production lengths the transforms run on compile-time plans: fused
+// for one channel and every normalisation but RUN-ABS-MF, as the fixed kernels
+// of the five-kernel path otherwise.  The output length follows the lag kept:
+// where it is another than S2sFixO's only that transform stays on its runtime
+// plan.  FXC_S2S_FUSED=0 keeps every transform on the runtime plans.
+static int s2s_fixed_setup(fxc_s2s_plan *p) {
   const fxc_s2s_config &c = p->cfg;
   const char *env = getenv("FXC_S2S_FUSED");
   if (env && atoi(env) == 0) return FXC_OK;
-  if (c.num_ch != 1 || c.normalize == 1 || c.nfft_filter / 2 != S2sFixF::kM ||
-      c.seg / 2 != S2sFixS::kM || c.nfft_out / 2 != S2sFixO::kM)
-    return FXC_OK;
+  if (c.nfft_filter / 2 != S2sFixF::kM || c.seg / 2 != S2sFixS::kM) return FXC_OK;
+  if (fixed_shared_slots<S2sFixS>(ToRuntime{p->to}) > kLdsComplexCapacity) return FXC_OK;
   std::vector<float2> all;
   size_t off[6];
   auto add = [&](const std::vector<float2> &v, size_t *o) {
@@ -1464,7 +1661,9 @@ static int s2s_fused_setup(fxc_s2s_plan *p) {
     FXC_TRY(dmalloc((void **)&p->d_staper, tp.size() * sizeof(float)));
     FXC_HIP(hipMemcpy(p->d_staper, tp.data(), tp.size() * sizeof(float), hipMemcpyHostToDevice));
   }
-  p->fused = true;
+  p->fixed = true;
+  p->fixed_out = c.nfft_out / 2 == S2sFixO::kM;
+  p->fused = p->fixed_out && c.num_ch == 1 && c.normalize != 1;
   return FXC_OK;
 }
 
@@ -1545,7 +1744,7 @@ extern "C" int fxc_s2s_plan_create(fxc_s2s_plan **out, const fxc_s2s_config *cfg
     delete p;
     return rc;
   }
-  if (!large && (rc = s2s_fused_setup(p)) != FXC_OK) {
+  if (!large && (rc = s2s_fixed_setup(p)) != FXC_OK) {
     fxc_s2s_plan_destroy(p);
     return rc;
   }
@@ -1556,7 +1755,7 @@ extern "C" int fxc_s2s_plan_create(fxc_s2s_plan **out, const fxc_s2s_config *cfg
 extern "C" int fxc_s2s_plan_destroy(fxc_s2s_plan *p) {
   if (!p) return FXC_OK;
   for (void *q : {(void *)p->d_resp, (void *)p->d_x, (void *)p->d_w, (void *)p->d_xb,
-                  (void *)p->d_total, (void *)p->d_X, (void *)p->d_base, (void *)p->d_amp,
+                  (void *)p->d_total, (void *)p->d_X, (void *)p->d_base,
                   (void *)p->d_ww, (void *)p->d_steps, (void *)p->d_L, (void *)p->d_Lw,
                   (void *)p->d_fx, (void *)p->d_staper})
     dfree(q);
@@ -1600,16 +1799,13 @@ static int s2s_ensure(fxc_s2s_plan *p, long long rows, long long frames, int nst
   }
   if (rows > p->cap_rows) {
     for (void *q : {(void *)p->d_x, (void *)p->d_xb, (void *)p->d_total, (void *)p->d_X,
-                    (void *)p->d_base, (void *)p->d_amp})
+                    (void *)p->d_base})
       dfree(q);
-    p->d_x = p->d_xb = p->d_total = p->d_amp = nullptr;
+    p->d_x = p->d_xb = p->d_total = nullptr;
     p->d_X = p->d_base = nullptr;
     p->cap_rows = 0;
     FXC_TRY(dmalloc((void **)&p->d_x, (size_t)rows * c.seg * sizeof(float)));
-    if (c.whiten) {
-      FXC_TRY(dmalloc((void **)&p->d_X, (size_t)rows * p->fpitch * sizeof(float2)));
-      FXC_TRY(dmalloc((void **)&p->d_amp, (size_t)rows * p->fpitch * sizeof(float)));
-    }
+    if (c.whiten) FXC_TRY(dmalloc((void **)&p->d_X, (size_t)rows * p->fpitch * sizeof(float2)));
     if (c.normalize == 1) {
       FXC_TRY(dmalloc((void **)&p->d_xb, (size_t)rows * c.seg * sizeof(float)));
       FXC_TRY(dmalloc((void **)&p->d_total, (size_t)rows * c.seg * sizeof(float)));
@@ -1668,16 +1864,69 @@ static int launch_weight(bool cplx, const void *data, long long pitch, int width
   return FXC_OK;
 }
 
+// Launches of the compile-time kernels that stand in for the steps of the
+// five-kernel path (p->fixed).
+static int launch_fixed_prefilter(fxc_s2s_plan *p, const float *d_traces, int nfiles,
+                                  long long rows, hipStream_t st) {
+  const fxc_s2s_config &c = p->cfg;
+  constexpr size_t lds = (size_t)(S2sFixF::kM + 1 + fixed_lds_tw_count<S2sFixF>() +
+                                  fused_fold_count(S2sFixF::kM)) * sizeof(float2);
+  auto kern = s2s_fixed_prefilter_kernel<S2sFixF>;
+  FXC_TRY(set_lds(kern, lds));
+  const double inv_f = 1.0 / (double)((float)c.nfft_filter * c.delta);
+  hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kS2sThreads), lds, st, d_traces, c.npts,
+                     nfiles, p->d_steps, c.shift, c.seg, p->taper_size, p->fxf, p->d_resp, c.delta,
+                     inv_f, p->d_x);
+  FXC_HIP(hipGetLastError());
+  return FXC_OK;
+}
+
+template <class FPN, bool kOut>
+static int launch_fixed_row(fxc_s2s_plan *p, long long rows, const FixedTables &tn, int mode,
+                            const float *w, float2 *dst, long long dpitch, hipStream_t st) {
+  const fxc_s2s_config &c = p->cfg;
+  constexpr size_t lds = (size_t)fused_lds_count<S2sFixS, FPN>() * sizeof(float2);
+  auto kern = s2s_fixed_row_kernel<S2sFixS, FPN, kOut>;
+  FXC_TRY(set_lds(kern, lds));
+  hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kS2sThreads), lds, st, p->d_x, c.num_ch,
+                     mode, w, tn, c.delta, c.phase_only, dst, dpitch, p->nspec);
+  FXC_HIP(hipGetLastError());
+  return FXC_OK;
+}
+
+template <class To>
+static int launch_fixed_shared(fxc_s2s_plan *p, long long rows, const To &to, hipStream_t st) {
+  const fxc_s2s_config &c = p->cfg;
+  const size_t lds = (size_t)fixed_shared_slots<S2sFixS>(to) * sizeof(float2);
+  auto kern = s2s_fixed_shared_kernel<S2sFixS, To>;
+  FXC_TRY(set_lds(kern, lds));
+  const double inv_s = 1.0 / (double)((float)c.seg * c.delta);
+  hipLaunchKernelGGL(kern, dim3((unsigned)rows), dim3(kS2sThreads), lds, st, p->d_X, p->fpitch,
+                     p->d_ww, c.num_ch, p->d_staper, p->fxs, inv_s, to);
+  FXC_HIP(hipGetLastError());
+  return FXC_OK;
+}
+
 // Whitening of the rows in d_x (mode/w: pending normalisation).  With
 // `out` set the inverse also produces the output spectrum.
 static int s2s_whiten(fxc_s2s_plan *p, long long rows, long long frames, int mode, const float *w,
                       float2 *out, hipStream_t st) {
   const fxc_s2s_config &c = p->cfg;
+  if (p->fixed) {
+    FXC_TRY((launch_fixed_row<S2sFixS, false>(p, rows, p->fxs, mode, w, p->d_X, p->fpitch, st)));
+    FXC_TRY(launch_weight(true, p->d_X, p->fpitch, p->fwidth, c.num_ch, p->whiten_win, frames,
+                          p->d_ww, p->fpitch, st));
+    if (!out) return launch_fixed_shared(p, rows, ToRow{p->d_x}, st);
+    if (p->fixed_out)
+      return launch_fixed_shared(
+          p, rows, ToFixed<S2sFixO>{p->fxo, c.delta, c.phase_only, p->nspec, out}, st);
+    return launch_fixed_shared(p, rows, ToRuntime{p->to, c.delta, c.phase_only, p->nspec, out}, st);
+  }
   const int Ms = c.seg / 2;
   size_t lds = lds_bytes(Ms + 1, Ms);
   FXC_TRY(set_lds(s2s_whiten_fwd_kernel, lds));
   hipLaunchKernelGGL(s2s_whiten_fwd_kernel, dim3((unsigned)rows), dim3(kS2sThreads), lds, st,
-                     p->d_x, c.seg, c.num_ch, mode, w, p->ts, c.delta, p->d_X, p->d_amp, p->fpitch);
+                     p->d_x, c.seg, c.num_ch, mode, w, p->ts, c.delta, p->d_X, p->fpitch);
   FXC_HIP(hipGetLastError());
   FXC_TRY(launch_weight(true, p->d_X, p->fpitch, p->fwidth, c.num_ch, p->whiten_win, frames,
                         p->d_ww, p->fpitch, st));
@@ -1728,7 +1977,7 @@ static int s2sL_whiten(fxc_s2s_plan *p, long long rows, long long frames, int mo
   }
   FXC_TRY(s2sL_r2c(p, c.seg, p->d_x, c.seg, c.seg, p->d_X, p->fpitch, rows, st));
   hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(p->fwidth, rows), dim3(256), 0, st, p->d_X,
-                     p->fpitch, p->fwidth, c.delta, (const float *)nullptr, p->d_amp, p->fpitch);
+                     p->fpitch, p->fwidth, c.delta, (const float *)nullptr);
   FXC_HIP(hipGetLastError());
   FXC_TRY(launch_weight(true, p->d_X, p->fpitch, p->fwidth, c.num_ch, p->whiten_win, frames,
                         p->d_ww, p->fpitch, st));
@@ -1764,7 +2013,7 @@ static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles,
   const double inv_f = 1.0 / (double)((float)c.nfft_filter * c.delta);
   FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, c.seg, c.seg, p->d_L, p->lpitch, rows, st));
   hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(nbf, rows), dim3(256), 0, st, p->d_L, p->lpitch,
-                     nbf, c.delta, p->d_resp, (float *)nullptr, 0LL);
+                     nbf, c.delta, p->d_resp);
   FXC_HIP(hipGetLastError());
   FXC_TRY(s2sL_c2r(p, c.nfft_filter, p->d_L, p->lpitch, p->d_x, c.seg, c.seg, inv_f, rows, st));
   int mode = kLoadPlain;
@@ -1781,7 +2030,7 @@ static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles,
     // base spectrum R2C(nfft_filter) x dt, then per band C2R(base |H_i|^2)
     FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, c.seg, c.seg, p->d_base, p->bpitch, rows, st));
     hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(nbf, rows), dim3(256), 0, st, p->d_base,
-                       p->bpitch, nbf, c.delta, (const float *)nullptr, (float *)nullptr, 0LL);
+                       p->bpitch, nbf, c.delta, (const float *)nullptr);
     FXC_HIP(hipGetLastError());
     FXC_HIP(hipMemsetAsync(p->d_total, 0, (size_t)rows * c.seg * sizeof(float), st));
     for (int i = 1; i < c.filter_count; ++i) {
@@ -1900,10 +2149,14 @@ extern "C" int fxc_s2s_process(fxc_s2s_plan *p, const float *d_traces, int nfile
   size_t lds = lds_bytes(Mf + 1, Mf);
   FXC_TRY(set_lds(s2s_prefilter_kernel, lds));
   const double inv_f = 1.0 / (double)((float)c.nfft_filter * c.delta);
-  hipLaunchKernelGGL(s2s_prefilter_kernel, dim3((unsigned)rows), dim3(kS2sThreads), lds, st,
-                     d_traces, c.npts, nfiles, p->d_steps, c.shift, c.seg, p->taper_size, p->tf,
-                     p->d_resp, c.delta, inv_f, p->d_x);
-  FXC_HIP(hipGetLastError());
+  if (p->fixed) {
+    FXC_TRY(launch_fixed_prefilter(p, d_traces, nfiles, rows, st));
+  } else {
+    hipLaunchKernelGGL(s2s_prefilter_kernel, dim3((unsigned)rows), dim3(kS2sThreads), lds, st,
+                       d_traces, c.npts, nfiles, p->d_steps, c.shift, c.seg, p->taper_size, p->tf,
+                       p->d_resp, c.delta, inv_f, p->d_x);
+    FXC_HIP(hipGetLastError());
+  }
   int mode = kLoadPlain;
   const float *w = nullptr;
   if (c.whiten == 1 || c.whiten == 3) FXC_TRY(s2s_whiten(p, rows, frames, kLoadPlain, nullptr, nullptr, st));
@@ -1940,6 +2193,9 @@ extern "C" int fxc_s2s_process(fxc_s2s_plan *p, const float *d_traces, int nfile
   }
   if (c.whiten == 2 || c.whiten == 3) {
     FXC_TRY(s2s_whiten(p, rows, frames, mode, w, (float2 *)d_out, st));
+  } else if (p->fixed_out) {
+    FXC_TRY((launch_fixed_row<S2sFixO, true>(p, rows, p->fxo, mode, w, (float2 *)d_out, p->nspec,
+                                             st)));
   } else {
     const int Mo = c.nfft_out / 2;
     lds = lds_bytes(Mo + 1, Mo);

@@ -169,6 +169,35 @@ def test_fused_production_path(gpu, tmp_path, monkeypatch, whiten, normalize, ph
     assert rel_l2(out5, want) < 1e-5
 
 
+@pytest.mark.parametrize("nch,whiten,normalize,lag", [
+    (3, 2, 3, 100), (3, 3, 3, 110), (2, 1, 2, 40), (1, 2, 3, 40), (1, 1, 3, 60), (3, 0, 3, 100), (3, 0, 0, 80)])
+def test_compile_time_plans(gpu, tmp_path, monkeypatch, nch, whiten, normalize, lag):
+    """Shared running means (several channels) or an output length that has no
+    compile-time plan, at seg 36000 / 36288: the compile-time transforms between
+    the running means against the FP64 oracle, no further from it than the
+    runtime plans of the same steps (FXC_S2S_FUSED=0) within the 1e-6 that the
+    transforms of either may be off."""
+    import torch
+
+    path = str(tmp_path / "filter.txt")
+    s2s.write_filter_file(path, 0.1, "0.1/2")
+    plan = s2s.plan_lengths(2 * 3600, 0.1, 3600, 3600, lag, s2s.read_filters(path))
+    assert (plan.seg, plan.nfft_filter) == (36000, 36288)
+    assert (plan.nfft_out == 37044) == (lag == 100)
+    rng = np.random.default_rng(60 + 4 * whiten + normalize + lag)
+    tr = _traces(rng, 2 * nch, plan.npts)
+    steps = [0, 1]
+    out = _gpu_plan(plan, nch, whiten, normalize, 0).process(torch.from_numpy(tr).to(gpu), steps).cpu().numpy()
+    monkeypatch.setenv("FXC_S2S_FUSED", "0")
+    out5 = _gpu_plan(plan, nch, whiten, normalize, 0).process(torch.from_numpy(tr).to(gpu), steps).cpu().numpy()
+    win = s2s.cut_windows(tr.astype(np.float64), plan, steps)
+    want = s2s.process_batch(win.reshape(-1, nch, plan.seg), plan, whiten, normalize,
+                             False).reshape(len(steps), 2 * nch, -1)
+    err, err5 = rel_l2(out, want), rel_l2(out5, want)
+    print(f"nch={nch} whiten={whiten} normalize={normalize} lag={lag} rel_l2={err:.3e} runtime {err5:.3e}")
+    assert err < 1e-5 and err < err5 + 1e-6
+
+
 @pytest.mark.parametrize("whiten,normalize", [(2, 3), (3, 3), (1, 3)])
 def test_compensated_fp32_running_means(gpu, tmp_path, whiten, normalize):
     """Spec mode fxc_s2s_set_sums(1): the running means (RUN-ABS weights,
