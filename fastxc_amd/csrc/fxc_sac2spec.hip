@@ -17,6 +17,7 @@
 // the normalisation divide and clip, whitening divide and taper, and the
 // phase-only option are all folded into those passes.  Sums the reference
 // takes in FP64 (mean, trend, running means) stay FP64.
+#include <type_traits>
 #include "fxc_fft_fixed.hpp"
 #include "fxc_fft_large.hpp"
 #include "fxc_plan_cache.hpp"
@@ -425,6 +426,109 @@ s2s_weight_tile_kernel(const void *__restrict__ data, long long row_pitch, int w
       float v = acc[m];
       if (!isfinite(v) || v < kMinVal) v = kMinVal;
       w[k] = v;
+    }
+  }
+}
+
+// The tiled weights for windows up to kHold x kWThreads - kWTile + 1 samples
+// (kHold odd).  The old tile above stages doubles in LDS and passes over them
+// three times, with every channel's loads waiting for the one before; here the
+// values go through LDS once as floats (they are floats) to reach the thread
+// that owns kHold consecutive ones, which forms the FP64 prefix from registers
+// and writes it once, and the next channel's loads are in flight meanwhile.
+// An odd kHold spreads those runs over all LDS banks.  What is left is the
+// latency of a channel's three barriers at four workgroups per compute unit.
+// 4700 frames of three channels of 36000: RUN-ABS (301 samples) 1.60 -> 0.60 ms
+// = 4.5 TB/s of rows read and weights written, whitening (72 bins) 0.90 ->
+// 0.52 ms.
+template <bool kCplx, int kHold>
+__global__ void __launch_bounds__(kWThreads, kHold < 23 ? 4 : 3)
+s2s_weight_held_kernel(const void *__restrict__ data, long long row_pitch, int width, int nch,
+                       int win, float *__restrict__ wout, long long w_pitch) {
+  static_assert(kHold % 2 == 1, "odd runs");
+  __shared__ double S[kHold * kWThreads];
+  __shared__ double wave_tot[kWThreads / 64];
+  float *F = (float *)S;
+  const long long frame = blockIdx.x;
+  const int t0 = blockIdx.y * kWTile;
+  const int T = min(kWTile, width - t0);
+  const int base = t0 - win / 2;
+  const double inv = 1.0 / (double)win;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  using V = typename std::conditional<kCplx, float2, float>::type;
+  V v[kHold];
+  const bool inside = base >= 0 && base + kHold * kWThreads <= width;
+  auto load = [&](int ch) {
+    const V *x = (const V *)data + (frame * nch + ch) * row_pitch;
+    if (inside) {  // uniform row addresses, one lane offset
+#pragma unroll
+      for (int m = 0; m < kHold; ++m) v[m] = (x + base + m * kWThreads)[(unsigned)tid];
+    } else {
+      int t = tid;
+      asm volatile("" : "+v"(t));  // keeps the indexes out of registers across the channels
+#pragma unroll
+      for (int m = 0; m < kHold; ++m) {
+        const int i = base + t + m * kWThreads;
+        v[m] = V{};
+        if (i >= 0 && i < width) v[m] = x[i];
+      }
+    }
+  };
+  float acc[kWPerThread];
+#pragma unroll
+  for (int m = 0; m < kWPerThread; ++m) acc[m] = 0.f;
+  load(0);
+  for (int ch = 0; ch < nch; ++ch) {
+    __syncthreads();  // the previous channel's reads of S are done
+#pragma unroll
+    for (int m = 0; m < kHold; ++m) {
+      if constexpr (kCplx)
+        F[tid + m * kWThreads] = sqrtf(v[m].x * v[m].x + v[m].y * v[m].y);
+      else
+        F[tid + m * kWThreads] = fabsf(v[m]);
+    }
+    __syncthreads();
+    float own[kHold];
+    double run = 0.0;
+#pragma unroll
+    for (int m = 0; m < kHold; ++m) {
+      own[m] = F[tid * kHold + m];
+      run += own[m];
+    }
+    double incl = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const double y = __shfl_up(incl, off);
+      if (lane >= off) incl += y;
+    }
+    if (lane == 63) wave_tot[wid] = incl;
+    __syncthreads();  // wave_tot, and every read of F
+    double pre = incl - run;
+    for (int w = 0; w < wid; ++w) pre += wave_tot[w];
+#pragma unroll
+    for (int m = 0; m < kHold; ++m) {
+      pre += own[m];
+      S[tid * kHold + m] = pre;
+    }
+    if (ch + 1 < nch) load(ch + 1);  // in flight during the window sums
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kWPerThread; ++m) {
+      const int k = tid + m * kWThreads;
+      if (k < T) {
+        const double sum = S[k + win - 1] - (k > 0 ? S[k - 1] : 0.0);
+        acc[m] += (float)(inv * sum);
+      }
+    }
+  }
+  float *w = wout + frame * w_pitch + t0;
+#pragma unroll
+  for (int m = 0; m < kWPerThread; ++m) {
+    const int k = tid + m * kWThreads;
+    if (k < T) {
+      float o = acc[m];
+      if (!isfinite(o) || o < kMinVal) o = kMinVal;
+      w[k] = o;
     }
   }
 }
@@ -1833,8 +1937,25 @@ static int s2s_ensure(fxc_s2s_plan *p, long long rows, long long frames, int nst
 
 static int launch_weight(bool cplx, const void *data, long long pitch, int width, int nch, int win,
                          long long frames, float *w, long long wpitch, hipStream_t st) {
+  const unsigned tiles = (unsigned)ceil_div((size_t)width, (size_t)kWTile);
+  // the shortest run that covers tile and window: 17 takes windows to 257
+  // samples, 19 to 769 (both four workgroups per compute unit), 23 to 1793
+  // (three); beyond, the runs cost more registers than the passes they save
+  auto held = [&](auto kern, int hold) {
+    if (win < 1 || win > hold * kWThreads - kWTile + 1) return false;
+    hipLaunchKernelGGL(kern, dim3((unsigned)frames, tiles), dim3(kWThreads), 0, st, data, pitch,
+                       width, nch, win, w, wpitch);
+    return true;
+  };
+  if (cplx ? held(s2s_weight_held_kernel<true, 17>, 17) || held(s2s_weight_held_kernel<true, 19>, 19) ||
+                 held(s2s_weight_held_kernel<true, 23>, 23)
+           : held(s2s_weight_held_kernel<false, 17>, 17) ||
+                 held(s2s_weight_held_kernel<false, 19>, 19) ||
+                 held(s2s_weight_held_kernel<false, 23>, 23)) {
+    FXC_HIP(hipGetLastError());
+    return FXC_OK;
+  }
   if (win >= 1 && win <= kWTileMaxWin) {
-    const unsigned tiles = (unsigned)ceil_div((size_t)width, (size_t)kWTile);
     const size_t lds = (size_t)(kWTile + win - 1) * sizeof(double);
     const dim3 grid((unsigned)frames, tiles);
     const void *fn = cplx ? (const void *)s2s_weight_tile_kernel<true>

@@ -198,6 +198,31 @@ def test_compile_time_plans(gpu, tmp_path, monkeypatch, nch, whiten, normalize, 
     assert err < 1e-5 and err < err5 + 1e-6
 
 
+@pytest.mark.parametrize("dt,seg_s,low,nch", [
+    (1.0, 3600, 0.05, 3),     # 61 samples: runs of 17; rows shorter than a tile
+    (0.05, 409.6, 0.1, 2),    # 599: runs of 19; two whole tiles
+    (0.05, 600, 0.04, 3),     # 1499: runs of 23
+    (0.05, 600, 0.02, 2),     # 2997: the general tile
+    (1.0, 14400, 0.05, 2)])   # 288 whitening bins: runs of 19 of complex rows
+def test_running_mean_runs(gpu, tmp_path, dt, seg_s, low, nch):
+    """The run lengths of the tiled running means and the windows between them,
+    against the FP64 oracle (sums are FP64 in both: the bound is the one of the
+    transforms around them)."""
+    import torch
+
+    path = str(tmp_path / "filter.txt")
+    s2s.write_filter_file(path, dt, f"{low}/{0.4 / dt if dt == 1.0 else 2}")
+    plan = s2s.plan_lengths(2 * seg_s, dt, seg_s, seg_s, 20, s2s.read_filters(path))
+    rng = np.random.default_rng(int(seg_s + 100 * low))
+    tr = _traces(rng, 2 * nch, plan.npts)
+    out = _gpu_plan(plan, nch, 2, 3, 0).process(torch.from_numpy(tr).to(gpu), [0, 1]).cpu().numpy()
+    win = s2s.cut_windows(tr.astype(np.float64), plan, [0, 1])
+    want = s2s.process_batch(win.reshape(-1, nch, plan.seg), plan, 2, 3, False).reshape(2, 2 * nch, -1)
+    err = rel_l2(out, want)
+    print(f"dt={dt} seg={plan.seg} low={low} rel_l2={err:.3e}")
+    assert err < 1e-5
+
+
 @pytest.mark.parametrize("whiten,normalize", [(2, 3), (3, 3), (1, 3)])
 def test_compensated_fp32_running_means(gpu, tmp_path, whiten, normalize):
     """Spec mode fxc_s2s_set_sums(1): the running means (RUN-ABS weights,
