@@ -1,5 +1,6 @@
 // Four-step FFT over HBM for lengths beyond one workgroup's LDS (see
 // fxc_fft_large.hpp for the decomposition).
+#include "fxc_fft_half.hpp"
 #include "fxc_fft_large.hpp"
 #include "fxc_plan_cache.hpp"
 
@@ -142,140 +143,6 @@ __global__ void large_unpack_kernel(const float2 *__restrict__ z, int M, float *
   if (2 * j + 1 < out_len) yr[2 * j + 1] = (float)((double)v.y * scale);
 }
 
-// ---------------------------------------------------------------------------
-// Real transforms of n = 2M = 4Q samples whose M complex values exceed the LDS
-// but whose Q do not (one-hour windows at 20 Hz: Q = 18000 .. 18522): a
-// workgroup runs the two Q-point transforms of a row one after the other in its
-// LDS and combines them, instead of four passes over HBM (pack, columns, rows,
-// unfold).  The first half's result waits in natural order in a scratch row of
-// the workgroup (Q complex, L2).  Bound: the LDS transforms, as for the lengths
-// that fit.  1440 rows of 72000: 0.50 ms forward and 0.46 ms inverse against
-// 1.55 ms each in four passes.
-// ---------------------------------------------------------------------------
-constexpr int kHalfThreads = 1024;
-
-// [data: Q][twiddles]
-static size_t half_lds_bytes(int Q) { return ((size_t)Q + tw_lds_count(Q)) * sizeof(float2); }
-
-// Forward: z[j] = x[2j] + i x[2j+1] (zero past in_len) splits into its even and
-// odd elements, Z[k] = E[k] + w^k O[k] and Z[k + Q] = E[k] - w^k O[k], w =
-// exp(-2 pi i / M).  Bins k and Q - k of both halves give Z at k, Q - k, Q + k
-// and M - k, two mirror pairs of the unfold.
-template <unsigned kMask>
-__global__ void __launch_bounds__(kHalfThreads)
-half_r2c_kernel(const float *__restrict__ in, long long in_dist, int in_len, long long rows,
-                float2 *__restrict__ out, long long out_dist, float scale, FftPlanDev plan,
-                const float2 *__restrict__ tw, const float2 *__restrict__ twM,
-                const float2 *__restrict__ half, float2 *__restrict__ scratch) {
-  extern __shared__ float2 lds[];
-  const int Q = plan.n, M = 2 * Q, tid = threadIdx.x;
-  float2 *twl = lds + Q;
-  for (int i = tid; i < kTwFine + plan.ncoarse; i += kHalfThreads) twl[i] = tw[i];
-  float2 *E = scratch + (size_t)blockIdx.x * Q;
-  for (long long row = blockIdx.x; row < rows; row += gridDim.x) {
-    const float *x = in + row * in_dist;
-    float2 *X = out + row * out_dist;
-#pragma unroll 1
-    for (int part = 0; part < 2; ++part) {
-      __syncthreads();  // the previous half is read
-#pragma unroll 8
-      for (int j = tid; j < Q; j += kHalfThreads) {
-        const int a = 4 * j + 2 * part;
-        lds[j] = make_float2(a < in_len ? x[a] : 0.f, a + 1 < in_len ? x[a + 1] : 0.f);
-      }
-      __syncthreads();
-      lds_fft<kMask>(lds, 1, plan, twl, -1.f);
-      if (part == 0)
-        for (int k = tid; k < Q; k += kHalfThreads) E[k] = lds[fft_pos(plan, k)];
-    }
-    // X[k] = (a + conj b)/2 - (i/2) h_k (a - conj b) of a = Z[k], b = Z[M-k], and
-    // its mirror X[M-k] = conj((a + conj b)/2) - (i/2) conj(h_k (a - conj b))
-    auto unfold = [&](int k, float2 a, float2 b) {
-      const float2 e = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));
-      const float2 d = cmul(half[k], make_float2(0.5f * (a.x - b.x), 0.5f * (a.y + b.y)));
-      X[k] = make_float2((e.x + d.y) * scale, (e.y - d.x) * scale);
-      X[M - k] = make_float2((e.x - d.y) * scale, (-e.y - d.x) * scale);
-    };
-    for (int k = tid; 2 * k <= Q; k += kHalfThreads) {
-      const float2 e0 = E[k], o0 = lds[fft_pos(plan, k)];
-      const float2 p0 = cmul(twM[k], o0);  // w^k O[k]
-      const float2 zk = cadd(e0, p0), zkq = csub(e0, p0);
-      if (k == 0) {
-        // Z[0] is its own mirror: X[0] and X[M] are real; so is Z[Q]
-        X[0] = make_float2((zk.x + zk.y) * scale, 0.f);
-        X[M] = make_float2((zk.x - zk.y) * scale, 0.f);
-        const float2 d = cmul(half[Q], make_float2(0.f, zkq.y));
-        X[Q] = make_float2((zkq.x + d.y) * scale, -d.x * scale);
-        continue;
-      }
-      const float2 e1 = E[Q - k], o1 = lds[fft_pos(plan, Q - k)];
-      const float2 p1 = cmul(twM[Q - k], o1);
-      const float2 zq = cadd(e1, p1), zm = csub(e1, p1);  // Z[Q-k], Z[M-k]
-      unfold(k, zk, zm);
-      if (2 * k != Q) unfold(Q - k, zq, zkq);
-    }
-  }
-}
-
-// Inverse: the folded spectrum Z splits into its even and odd bins, each closed
-// under the fold's mirror (2i with 2(Q-i), 2i+1 with 2(Q-1-i)+1), and
-// z[n] = F_0[n] + w^n F_1[n], z[n + Q] = F_0[n] - w^n F_1[n], w = exp(2 pi i / M).
-template <unsigned kMask>
-__global__ void __launch_bounds__(kHalfThreads)
-half_c2r_kernel(const float2 *__restrict__ in, long long in_dist, long long rows,
-                float *__restrict__ out, long long out_dist, int out_len, double scale,
-                FftPlanDev plan, const float2 *__restrict__ tw, const float2 *__restrict__ twM,
-                const float2 *__restrict__ half, float2 *__restrict__ scratch) {
-  extern __shared__ float2 lds[];
-  const int Q = plan.n, M = 2 * Q, tid = threadIdx.x;
-  float2 *twl = lds + Q;
-  for (int i = tid; i < kTwFine + plan.ncoarse; i += kHalfThreads) twl[i] = tw[i];
-  float2 *F = scratch + (size_t)blockIdx.x * Q;
-  for (long long row = blockIdx.x; row < rows; row += gridDim.x) {
-    const float2 *X = in + row * in_dist;
-    float *y = out + row * out_dist;
-#pragma unroll 1
-    for (int part = 0; part < 2; ++part) {
-      __syncthreads();  // the previous half is read
-      const int mir = Q - part;
-#pragma unroll 4
-      for (int i = tid; 2 * i <= mir; i += kHalfThreads) {
-        const int k = 2 * i + part;
-        const float2 a = X[k], b = X[M - k];
-        if (k == 0) {
-          lds[0] = make_float2(a.x + b.x, a.x - b.x);  // imaginary parts ignored
-        } else {
-          const float2 s = make_float2(a.x + b.x, a.y - b.y);
-          const float2 d = cmul(half[k], make_float2(a.x - b.x, a.y + b.y));
-          if (2 * i != mir) lds[mir - i] = make_float2(s.x + d.y, d.x - s.y);
-          lds[i] = make_float2(s.x - d.y, s.y + d.x);
-        }
-      }
-      __syncthreads();
-      lds_fft<kMask>(lds, 1, plan, twl, 1.f);
-      if (part == 0)
-        for (int n = tid; n < Q; n += kHalfThreads) F[n] = lds[fft_pos(plan, n)];
-    }
-    auto put = [&](int n, float2 v) {
-      if (2 * n < out_len) y[2 * n] = (float)((double)v.x * scale);
-      if (2 * n + 1 < out_len) y[2 * n + 1] = (float)((double)v.y * scale);
-    };
-    for (int n = tid; n < Q; n += kHalfThreads) {
-      const float2 f0 = F[n], p = cmul(twM[n], lds[fft_pos(plan, n)]);
-      put(n, cadd(f0, p));
-      put(n + Q, csub(f0, p));
-    }
-  }
-}
-
-static int half_grid(long long rows, unsigned *grid) {
-  int dev = 0, ncu = 0;
-  FXC_HIP(hipGetDevice(&dev));
-  FXC_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-  *grid = (unsigned)std::min<long long>(rows, std::max(ncu, 1));
-  return FXC_OK;
-}
-
 namespace {
 std::mutex g_large_mu;
 std::map<std::tuple<int, int, int>, std::unique_ptr<LargeFft>> g_large;
@@ -394,18 +261,9 @@ int large_r2c(int n, const float *in, long long in_dist, int in_len, float2 *out
   const int M = n / 2;
   const LargeFft *p = nullptr;
   FXC_TRY(large_plan(M, -1, &p));
-  if (p->pq && rows > 0) {
-    unsigned grid = 0;
-    FXC_TRY(half_grid(rows, &grid));
-    const size_t lds = half_lds_bytes(M / 2);
-    auto k = half_r2c_kernel<kRadixSmooth>;
-    FXC_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kHalfThreads), lds, st, in, in_dist, in_len, rows, out,
-                       out_dist, scale, p->pq->dev, p->pq->d_tw, p->d_tw, p->d_half, work);
-    FXC_HIP(hipGetLastError());
-    return FXC_OK;
-  }
+  if (p->pq && rows > 0)
+    return half_r2c(p, in, in_dist, in_len, out, out_dist, rows, work, PlainSample{},
+                    ScaledBin{scale}, st);
   float2 *w0 = work, *w1 = work + (size_t)rows * M;
   hipLaunchKernelGGL(large_pack_kernel, grid_rows(M, rows, 256), dim3(256), 0, st, in, in_dist,
                      in_len, w0, M);
@@ -423,18 +281,8 @@ int large_c2r(int n, const float2 *in, long long in_dist, float *out, long long 
   const int M = n / 2;
   const LargeFft *p = nullptr;
   FXC_TRY(large_plan(M, 1, &p));
-  if (p->pq && rows > 0) {
-    unsigned grid = 0;
-    FXC_TRY(half_grid(rows, &grid));
-    const size_t lds = half_lds_bytes(M / 2);
-    auto k = half_c2r_kernel<kRadixSmooth>;
-    FXC_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)lds));
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kHalfThreads), lds, st, in, in_dist, rows, out,
-                       out_dist, out_len, scale, p->pq->dev, p->pq->d_tw, p->d_tw, p->d_half, work);
-    FXC_HIP(hipGetLastError());
-    return FXC_OK;
-  }
+  if (p->pq && rows > 0)
+    return half_c2r(p, in, in_dist, out, out_dist, out_len, rows, work, scale, PlainBin{}, st);
   float2 *w0 = work, *w1 = work + (size_t)rows * M;
   hipLaunchKernelGGL(large_fold_kernel, grid_rows(M, rows, 256), dim3(256), 0, st, in, in_dist, M,
                      p->d_half, w0);

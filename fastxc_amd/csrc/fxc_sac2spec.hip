@@ -19,6 +19,7 @@
 // takes in FP64 (mean, trend, running means) stay FP64.
 #include <type_traits>
 #include "fxc_fft_fixed.hpp"
+#include "fxc_fft_half.hpp"
 #include "fxc_fft_large.hpp"
 #include "fxc_plan_cache.hpp"
 #include "fastxc_amd.h"
@@ -748,8 +749,10 @@ __global__ void s2s_mf_accum_kernel(const float *__restrict__ xb, const float *_
 // ---------------------------------------------------------------------------
 // Long windows (transforms beyond one workgroup's LDS, e.g. dt 0.05 s: seg
 // 72000, filter FFT 72576, output FFT 74088).  The same steps in the same
-// order as the fused kernels above, as element-wise passes over HBM rows
-// around the four-step transforms of fxc_fft_large.
+// order as the fused kernels above.  A transform whose halves fit the LDS
+// (fxc_fft_half.hpp) takes the steps beside it into its loads and stores:
+// 1440 windows of 72000 4.18 -> 3.59 ms against passes of their own, which
+// longer transforms (four steps over HBM, fxc_fft_large) keep.
 // ---------------------------------------------------------------------------
 // Window cut, non-finite -> 0, demean, detrend (FP64 sums) and edge taper of
 // one row into x[row][seg] (the front of s2s_prefilter_kernel).
@@ -798,49 +801,53 @@ s2sL_pre_kernel(const float *__restrict__ traces, int npts, int nfiles,
   }
 }
 
-// X[k] = sanitise(X[k] dt) (times resp[k] when given), k < nbin, every row.
-__global__ void s2sL_spec_kernel(float2 *__restrict__ X, long long pitch, int nbin, float dt,
-                                 const float *__restrict__ resp) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nbin) return;
-  const long long row = blockIdx.y;
-  float2 v = cscale(X[row * pitch + k], dt);
-  if (!cfinite(v)) v = make_float2(0.f, 0.f);
-  if (resp) v = cscale(v, resp[k]);
-  X[row * pitch + k] = v;
-}
-
-// Pending time-domain normalisation applied in place (load_row's rules).
-__global__ void s2sL_norm_kernel(float *__restrict__ x, int seg, int nch, int mode,
-                                 const float *__restrict__ w) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= seg) return;
-  const long long row = blockIdx.y;
-  float v = x[row * seg + i];
-  if (mode == kLoadRunabs) {
-    const float d = w[(row / nch) * seg + i];
-    v = (!isfinite(d) || d < kMinValD) ? 0.f : v / d;
-    if (!isfinite(v)) v = 0.f;
-    v = v > kMaxVal ? kMaxVal : (v < -kMaxVal ? -kMaxVal : v);
-  } else if (mode == kLoadOnebit) {
-    v = v > 0.f ? 1.f : (v < 0.f ? -1.f : 0.f);
+// The steps between the transforms, each the value of one sample or bin.
+// NormSample: the pending time-domain normalisation.  SpecBin: X dt, sanitised
+// (times resp[k] when given).  WhitenBin: X / ww (0 for an invalid weight),
+// spectral taper, sanitised.  OutBin: the output spectrum.
+struct NormSample {
+  int seg, nch, mode;
+  const float *w;
+  __device__ __forceinline__ float operator()(long long row, int i, float v) const {
+    return normalised(v, mode, mode == kLoadRunabs ? w[(row / nch) * seg + i] : 0.f);
   }
-  x[row * seg + i] = v;
-}
+};
+struct SpecBin {
+  float dt;
+  const float *resp;
+  __device__ __forceinline__ float2 operator()(long long, int k, float2 v) const {
+    v = cscale(v, dt);
+    if (!cfinite(v)) v = make_float2(0.f, 0.f);
+    return resp ? cscale(v, resp[k]) : v;
+  }
+};
+struct WhitenBin {
+  const float *ww;
+  long long fpitch;
+  int nch, i1, i2, i3, i4;
+  __device__ __forceinline__ float2 operator()(long long row, int k, float2 v) const {
+    const float d = ww[(row / nch) * fpitch + k];
+    v = (!isfinite(d) || d < kMinValD) ? make_float2(0.f, 0.f) : make_float2(v.x / d, v.y / d);
+    v = cscale(v, spec_taper(k, i1, i2, i3, i4));
+    if (!cfinite(v)) v = make_float2(0.f, 0.f);
+    return v;
+  }
+};
+struct OutBin {
+  float dt;
+  int phase_only;
+  __device__ __forceinline__ float2 operator()(long long, int, float2 v) const {
+    return output_bin(v, dt, phase_only);
+  }
+};
 
-// Whitening: X / ww (0 for an invalid weight), spectral taper, sanitise.
-__global__ void s2sL_whiten_kernel(float2 *__restrict__ X, long long fpitch, int nbin,
-                                   const float *__restrict__ ww, int nch, int i1, int i2, int i3,
-                                   int i4) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nbin) return;
+// The same in place, where the transform runs in four steps over HBM.
+template <class Op, class V>
+__global__ void s2sL_apply_kernel(V *__restrict__ x, long long pitch, int n, Op op) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
   const long long row = blockIdx.y;
-  float2 v = X[row * fpitch + k];
-  const float d = ww[(row / nch) * fpitch + k];
-  v = (!isfinite(d) || d < kMinValD) ? make_float2(0.f, 0.f) : make_float2(v.x / d, v.y / d);
-  v = cscale(v, spec_taper(k, i1, i2, i3, i4 < nbin ? i4 : nbin));
-  if (!cfinite(v)) v = make_float2(0.f, 0.f);
-  X[row * fpitch + k] = v;
+  x[row * pitch + i] = op(row, i, x[row * pitch + i]);
 }
 
 // One band of RUN-ABS-MF: dst[k] = base[k] resp[k].
@@ -850,21 +857,6 @@ __global__ void s2sL_band_kernel(const float2 *__restrict__ base, long long bpit
   if (k >= nbin) return;
   const long long row = blockIdx.y;
   dst[row * bpitch + k] = cscale(base[row * bpitch + k], resp[k]);
-}
-
-// Output spectrum: x dt, sanitise, optional phase-only, in place.
-__global__ void s2sL_out_kernel(float2 *__restrict__ out, int nspec, float dt, int phase_only) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nspec) return;
-  const long long row = blockIdx.y;
-  float2 v = cscale(out[row * nspec + k], dt);
-  if (!cfinite(v)) v = make_float2(0.f, 0.f);
-  if (phase_only) {
-    const float a = hypotf(v.x, v.y);
-    v = (!isfinite(a) || a <= kMinVal) ? make_float2(0.f, 0.f) : cscale(v, 1.f / a);
-    if (!cfinite(v)) v = make_float2(0.f, 0.f);
-  }
-  out[row * nspec + k] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -2066,48 +2058,70 @@ static int s2s_whiten(fxc_s2s_plan *p, long long rows, long long frames, int mod
   return FXC_OK;
 }
 
-// Long-window path: four-step real transforms in chunks of kLargeChunk rows.
-static int s2sL_r2c(fxc_s2s_plan *p, int n, const float *x, long long xd, int in_len, float2 *X,
-                    long long Xd, long long rows, hipStream_t st) {
-  for (long long r = 0; r < rows; r += kLargeChunk)
-    FXC_TRY(large_r2c(n, x + r * xd, xd, in_len, X + r * Xd, Xd, std::min(kLargeChunk, rows - r),
-                      p->d_Lw, 1.f, st));
+static dim3 s2sL_grid(long long n, long long rows) {
+  return dim3((unsigned)ceil_div((size_t)n, (size_t)256), (unsigned)rows);
+}
+
+template <class Op, class V>
+static int s2sL_apply(V *x, long long pitch, int n, long long rows, const Op &op, hipStream_t st) {
+  hipLaunchKernelGGL((s2sL_apply_kernel<Op, V>), s2sL_grid(n, rows), dim3(256), 0, st, x, pitch, n,
+                     op);
+  FXC_HIP(hipGetLastError());
   return FXC_OK;
 }
 
-static int s2sL_c2r(fxc_s2s_plan *p, int n, const float2 *X, long long Xd, float *x, long long xd,
-                    int out_len, double scale, long long rows, hipStream_t st) {
+// Long-window path: X = bin(R2C(sample(x))) and x = C2R(bin(X)).  Where half a
+// transform fits the LDS the two are part of it; otherwise they are passes of
+// their own (in place) around four-step transforms of kLargeChunk rows.
+template <class SampleOp, class BinOp>
+static int s2sL_r2c(fxc_s2s_plan *p, int n, float *x, const SampleOp &sample, float2 *X,
+                    long long Xd, const BinOp &bin, long long rows, hipStream_t st) {
+  const int seg = p->cfg.seg;
+  const LargeFft *f = nullptr;
+  FXC_TRY(large_plan(n / 2, -1, &f));
+  if (f->pq) return half_r2c(f, x, seg, seg, X, Xd, rows, p->d_Lw, sample, bin, st);
+  if (!std::is_same<SampleOp, PlainSample>::value) FXC_TRY(s2sL_apply(x, seg, seg, rows, sample, st));
   for (long long r = 0; r < rows; r += kLargeChunk)
-    FXC_TRY(large_c2r(n, X + r * Xd, Xd, x + r * xd, xd, out_len, std::min(kLargeChunk, rows - r),
+    FXC_TRY(large_r2c(n, x + r * seg, seg, seg, X + r * Xd, Xd, std::min(kLargeChunk, rows - r),
+                      p->d_Lw, 1.f, st));
+  return s2sL_apply(X, Xd, n / 2 + 1, rows, bin, st);
+}
+
+template <class BinOp>
+static int s2sL_c2r(fxc_s2s_plan *p, int n, float2 *X, long long Xd, const BinOp &bin, float *x,
+                    double scale, long long rows, hipStream_t st) {
+  const int seg = p->cfg.seg;
+  const LargeFft *f = nullptr;
+  FXC_TRY(large_plan(n / 2, 1, &f));
+  if (f->pq) return half_c2r(f, X, Xd, x, seg, seg, rows, p->d_Lw, scale, bin, st);
+  if (!std::is_same<BinOp, PlainBin>::value) FXC_TRY(s2sL_apply(X, Xd, n / 2 + 1, rows, bin, st));
+  for (long long r = 0; r < rows; r += kLargeChunk)
+    FXC_TRY(large_c2r(n, X + r * Xd, Xd, x + r * seg, seg, seg, std::min(kLargeChunk, rows - r),
                       p->d_Lw, scale, st));
   return FXC_OK;
 }
 
-static dim3 s2sL_grid(long long n, long long rows) {
-  return dim3((unsigned)ceil_div((size_t)n, (size_t)256), (unsigned)rows);
+// R2C of the d_x rows with their pending normalisation (mode, weights w).
+template <class BinOp>
+static int s2sL_r2c_x(fxc_s2s_plan *p, int n, int mode, const float *w, float2 *X, long long Xd,
+                      const BinOp &bin, long long rows, hipStream_t st) {
+  const fxc_s2s_config &c = p->cfg;
+  if (mode == kLoadPlain) return s2sL_r2c(p, n, p->d_x, PlainSample{}, X, Xd, bin, rows, st);
+  return s2sL_r2c(p, n, p->d_x, NormSample{c.seg, c.num_ch, mode, w}, X, Xd, bin, rows, st);
 }
 
 // Whitening of d_x rows (pending normalisation `mode`, weights w first).
 static int s2sL_whiten(fxc_s2s_plan *p, long long rows, long long frames, int mode,
                        const float *w, hipStream_t st) {
   const fxc_s2s_config &c = p->cfg;
-  if (mode != kLoadPlain) {
-    hipLaunchKernelGGL(s2sL_norm_kernel, s2sL_grid(c.seg, rows), dim3(256), 0, st, p->d_x, c.seg,
-                       c.num_ch, mode, w);
-    FXC_HIP(hipGetLastError());
-  }
-  FXC_TRY(s2sL_r2c(p, c.seg, p->d_x, c.seg, c.seg, p->d_X, p->fpitch, rows, st));
-  hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(p->fwidth, rows), dim3(256), 0, st, p->d_X,
-                     p->fpitch, p->fwidth, c.delta, (const float *)nullptr);
-  FXC_HIP(hipGetLastError());
+  FXC_TRY(s2sL_r2c_x(p, c.seg, mode, w, p->d_X, p->fpitch, SpecBin{c.delta, nullptr}, rows, st));
   FXC_TRY(launch_weight(true, p->d_X, p->fpitch, p->fwidth, c.num_ch, p->whiten_win, frames,
                         p->d_ww, p->fpitch, st));
-  hipLaunchKernelGGL(s2sL_whiten_kernel, s2sL_grid(p->fwidth, rows), dim3(256), 0, st, p->d_X,
-                     p->fpitch, p->fwidth, p->d_ww, c.num_ch, c.idx[0], c.idx[1], c.idx[2],
-                     c.idx[3]);
-  FXC_HIP(hipGetLastError());
   const double inv_seg = 1.0 / (double)((float)c.seg * c.delta);
-  return s2sL_c2r(p, c.seg, p->d_X, p->fpitch, p->d_x, c.seg, c.seg, inv_seg, rows, st);
+  return s2sL_c2r(p, c.seg, p->d_X, p->fpitch,
+                  WhitenBin{p->d_ww, p->fpitch, c.num_ch, c.idx[0], c.idx[1], c.idx[2],
+                            std::min(c.idx[3], p->fwidth)},
+                  p->d_x, inv_seg, rows, st);
 }
 
 static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles, long long rows,
@@ -2132,11 +2146,9 @@ static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles,
   FXC_HIP(hipGetLastError());
   const int nbf = c.nfft_filter / 2 + 1;
   const double inv_f = 1.0 / (double)((float)c.nfft_filter * c.delta);
-  FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, c.seg, c.seg, p->d_L, p->lpitch, rows, st));
-  hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(nbf, rows), dim3(256), 0, st, p->d_L, p->lpitch,
-                     nbf, c.delta, p->d_resp);
-  FXC_HIP(hipGetLastError());
-  FXC_TRY(s2sL_c2r(p, c.nfft_filter, p->d_L, p->lpitch, p->d_x, c.seg, c.seg, inv_f, rows, st));
+  FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, PlainSample{}, p->d_L, p->lpitch,
+                   SpecBin{c.delta, p->d_resp}, rows, st));
+  FXC_TRY(s2sL_c2r(p, c.nfft_filter, p->d_L, p->lpitch, PlainBin{}, p->d_x, inv_f, rows, st));
   int mode = kLoadPlain;
   const float *w = nullptr;
   if (c.whiten == 1 || c.whiten == 3) FXC_TRY(s2sL_whiten(p, rows, frames, kLoadPlain, nullptr, st));
@@ -2149,17 +2161,14 @@ static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles,
     mode = kLoadOnebit;
   } else if (c.normalize == 1) {
     // base spectrum R2C(nfft_filter) x dt, then per band C2R(base |H_i|^2)
-    FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, c.seg, c.seg, p->d_base, p->bpitch, rows, st));
-    hipLaunchKernelGGL(s2sL_spec_kernel, s2sL_grid(nbf, rows), dim3(256), 0, st, p->d_base,
-                       p->bpitch, nbf, c.delta, (const float *)nullptr);
-    FXC_HIP(hipGetLastError());
+    FXC_TRY(s2sL_r2c(p, c.nfft_filter, p->d_x, PlainSample{}, p->d_base, p->bpitch,
+                     SpecBin{c.delta, nullptr}, rows, st));
     FXC_HIP(hipMemsetAsync(p->d_total, 0, (size_t)rows * c.seg * sizeof(float), st));
     for (int i = 1; i < c.filter_count; ++i) {
       hipLaunchKernelGGL(s2sL_band_kernel, s2sL_grid(nbf, rows), dim3(256), 0, st, p->d_base,
                          p->bpitch, nbf, p->d_resp + (size_t)i * nbf, p->d_L);
       FXC_HIP(hipGetLastError());
-      FXC_TRY(s2sL_c2r(p, c.nfft_filter, p->d_L, p->bpitch, p->d_xb, c.seg, c.seg, inv_f, rows,
-                       st));
+      FXC_TRY(s2sL_c2r(p, c.nfft_filter, p->d_L, p->bpitch, PlainBin{}, p->d_xb, inv_f, rows, st));
       FXC_TRY(launch_weight(false, p->d_xb, c.seg, c.seg, c.num_ch, p->mf_win[i], frames, p->d_w,
                             c.seg, st));
       const int nbr = (int)ceil_div(c.seg, 256);
@@ -2172,17 +2181,11 @@ static int s2s_process_large(fxc_s2s_plan *p, const float *d_traces, int nfiles,
   }
   if (c.whiten == 2 || c.whiten == 3) {
     FXC_TRY(s2sL_whiten(p, rows, frames, mode, w, st));
-  } else if (mode != kLoadPlain) {
-    hipLaunchKernelGGL(s2sL_norm_kernel, s2sL_grid(c.seg, rows), dim3(256), 0, st, p->d_x, c.seg,
-                       c.num_ch, mode, w);
-    FXC_HIP(hipGetLastError());
+    mode = kLoadPlain;
   }
   // output spectrum: zero pad to nfft_out, R2C, x dt, sanitise, phase-only
-  FXC_TRY(s2sL_r2c(p, c.nfft_out, p->d_x, c.seg, c.seg, d_out, p->nspec, rows, st));
-  hipLaunchKernelGGL(s2sL_out_kernel, s2sL_grid(p->nspec, rows), dim3(256), 0, st, d_out,
-                     p->nspec, c.delta, c.phase_only);
-  FXC_HIP(hipGetLastError());
-  return FXC_OK;
+  return s2sL_r2c_x(p, c.nfft_out, mode, w, d_out, p->nspec, OutBin{c.delta, c.phase_only}, rows,
+                    st);
 }
 
 template <class FPN, bool kOut>
