@@ -1212,35 +1212,40 @@ __device__ __forceinline__ void normalise_row(float *x, int n, int mode, int win
 // Window cut + non-finite -> 0 + demean/detrend (FP64 sums) + cosine taper
 // into the float view of LDS, zero padded to kTwoM samples
 // (compute.cu:34-58, core/preprocess.cu:23-105).  Every load of the window
-// is issued before the first LDS store, so their latencies overlap.
+// is issued before the first use, and the samples stay in registers until they
+// are detrended (bound: FP64 issue; through LDS in each pass 1000 x 24 windows
+// took 11.97 ms, so 11.71).
 template <int kTwoM>
 __device__ __forceinline__ void preprocess_row(float *ldsf, const float *__restrict__ src, long long off,
                                       int npts, int seg, int taper_size) {
   constexpr int kPer = (kTwoM + kS2sThreads - 1) / kS2sThreads;
   double s = 0.0, unused1 = 0.0, unused2 = 0.0;
+  // this thread's samples stay in registers through the passes; the opaque copies
+  // of the index keep one pass's index arithmetic out of the next one's registers
   float v[kPer];
+  const int avail = (int)max(0LL, min((long long)seg, npts - off));
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
     const int i = threadIdx.x + j * kS2sThreads;
-    v[j] = (i < seg && off + i < npts) ? stream_load(src + off + i) : 0.f;
+    v[j] = i < avail ? stream_load(src + off + j * kS2sThreads + (unsigned)threadIdx.x) : 0.f;
   }
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const int i = threadIdx.x + j * kS2sThreads;
-    if (i < kTwoM) {
-      const float x = isfinite(v[j]) ? v[j] : 0.f;
-      ldsf[i] = x;
-      s += x;  // zero past seg
-    }
+    v[j] = isfinite(v[j]) ? v[j] : 0.f;
+    s += v[j];  // zero past seg
   }
   block_sum3(s, unused1, unused2);
   const double mean = s / seg;
   double s1 = 0.0, si = 0.0;
-  for (int i = threadIdx.x; i < seg; i += blockDim.x) {
-    const float v = (float)((double)ldsf[i] - mean);
-    ldsf[i] = v;
-    s1 += v;
-    si += (double)v * i;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = t + j * kS2sThreads;
+    v[j] = i < seg ? (float)((double)v[j] - mean) : 0.f;
+    s1 += v[j];
+    si += (double)v[j] * i;
+    if (j % 12 == 11) __builtin_amdgcn_sched_barrier(0);
   }
   unused1 = 0.0;
   block_sum3(s1, si, unused1);
@@ -1251,15 +1256,22 @@ __device__ __forceinline__ void preprocess_row(float *ldsf, const float *__restr
   const double det = a11 * a22 - a12 * a12;
   const double ca = (a22 * si - a12 * s1) / det;
   const double cb = (a11 * s1 - a12 * si) / det;
-  for (int i = threadIdx.x; i < seg; i += blockDim.x) {
-    float v = (float)((double)ldsf[i] - (ca * i + cb));
-    float factor = 1.f;
-    if (i < taper_size)
-      factor = (float)(0.5 * (1.0 - cos(M_PI * i / taper_size)));
-    else if (i >= seg - taper_size)
-      factor = (float)(0.5 * (1.0 - cos(M_PI * (seg - i) / taper_size)));
-    ldsf[i] = v * factor;
+  asm volatile("" : "+v"(t));
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int i = t + j * kS2sThreads;
+    if (i < kTwoM) ldsf[i] = i < seg ? (float)((double)v[j] - (ca * i + cb)) : 0.f;
+    if (j % 12 == 11) __builtin_amdgcn_sched_barrier(0);
   }
+  // the edges, by the thread that wrote them (the start's taper wins where they meet)
+  auto taper = [&](int i, int m) {
+    ldsf[i] *= (float)(0.5 * (1.0 - cos(M_PI * m / taper_size)));
+  };
+  for (int i = threadIdx.x; i < min(taper_size, seg); i += kS2sThreads) taper(i, i);
+  const int e0 = max(taper_size, seg - taper_size);
+  for (int i = e0 + (int)((threadIdx.x + kS2sThreads - e0 % kS2sThreads) % kS2sThreads); i < seg;
+       i += kS2sThreads)
+    taper(i, seg - i);
   __syncthreads();
 }
 
