@@ -1509,7 +1509,7 @@ s2s_back_kernel(float2 *X, long long fpitch, int seg, int i1, int i2, int i3, in
 // One workgroup holds a row in the LDS of its compute unit, so the vector and
 // LDS work of the transforms is what each kernel costs, and a runtime plan's
 // index arithmetic is most of that (29 against 12 us per transform of 18000
-// points).  14100 rows of three-channel frames: prefilter 3.54 -> 2.62 ms, row
+// points).  14100 rows of three-channel frames: prefilter 3.54 -> 2.46 ms, row
 // 2.29 -> 1.70 ms, shared with the output transform 4.19 -> 2.53 ms.
 // ---------------------------------------------------------------------------
 template <class FPF>

@@ -28,12 +28,15 @@ extern "C" {
 
 /* Message of the last failed call on this thread. */
 const char *fxc_last_error(void);
-/* Frees cached FFT plans (twiddle tables) of every device. */
+/* Frees cached FFT plans (twiddle and index tables) and idle stack workspaces of
+ * every device. */
 void fxc_release_plans(void);
 
 /* ---------------------------------------------------------------- FFT --
  * Batched transforms on the workgroup LDS FFT (lengths whose n (complex) or
- * n/2 (real) factor into 2,3,5,7,23,29 and fit 20480 complex values).
+ * n/2 (real) factor into 2,3,5,7,23,29 and fit 20480 complex values; longer
+ * real lengths run as two such transforms per row where n/4 fits, and longer
+ * ones still in four steps over memory).
  * Replace the cuFFT plans of native/sac2spec/device_memory.cu:23-32,
  * native/xc/memory/memory.cu:478-483, native/pws/worker/gpu.cu:197-227 and
  * native/tfpws/core/tfpws_workspace.cu:190-235.  Unnormalised; `scale`
@@ -54,7 +57,7 @@ int fxc_fft_c2r(const float *d_in, long long in_dist, float *d_out, long long ou
  * Spectra layout: [nstep][nsta][nspec] complex64, the StepPack v3 payload
  * order (native/xc/io/input.cu:46-67).  Output: [npairs][2*half_cc+1] float,
  * row t for task t = (src[t], rec[t]) in the caller's order. */
-#define FXC_PREC_FP32 0   /* fp32 vector FMA (reference arithmetic) */
+#define FXC_PREC_FP32 0   /* fp32 matrix instructions (reference precision) */
 #define FXC_PREC_BF16X3 1 /* split-bf16 hi+lo MFMA, fp32 accumulation */
 #define FXC_PREC_FP16 2   /* fp16 MFMA with per-station power-of-2 scale */
 #define FXC_PREC_PLAIN 3  /* the reference's step order: per-window fp32 stack RMW */
@@ -87,8 +90,9 @@ int fxc_xc_lags(fxc_xc_plan *plan, const float *d_xspec, long long nrows, float 
                 void *stream);
 /* Per-kernel timing with HIP events recorded on the launch stream (no
  * reference counterpart; used by the benchmark).  get_timing waits for the
- * events and returns milliseconds and launch counts for the split,
- * contraction and lag-synthesis kernels since the last set_timing. */
+ * events and returns milliseconds and launch counts for the split (FP32: the
+ * operand transpose), contraction and lag-synthesis kernels since the last
+ * set_timing. */
 int fxc_xc_set_timing(fxc_xc_plan *plan, int enable);
 int fxc_xc_get_timing(fxc_xc_plan *plan, double *ms3, long long *launches3);
 /* Spec mode (no reference counterpart: the reference contracts all nspec
@@ -234,9 +238,9 @@ int fxc_tfpws_spec(const float *d_prestack, const float *d_weights, const long l
 /* PWS without device allocation.  No counterpart in the reference: it is
  * for callers that cannot allocate (code under HIP graph capture, tight
  * serving loops).  Same arguments and result as fxc_pws (power 1); its
- * workspace (offsets and the groups' analytic spectra, 8 (npairs+1) +
- * 8 n groups bytes) lives in a fixed 64 MiB device array per GPU, held until
- * the process ends; larger calls are FXC_ERR_ARG.  fxc_stack_prepare(n)
+ * workspace lives in a fixed 64 MiB device array per GPU, held until the
+ * process ends; calls of more than that many bytes, counted as 8 (npairs+1) +
+ * 8 n groups, are FXC_ERR_ARG.  fxc_stack_prepare(n)
  * must run first on the device (once per device and length): it builds
  * the length-n FFT plans and resolves the array's device address (it
  * allocates; fxc_pws_noalloc then calls no hipMalloc/hipFree).  Calls on
