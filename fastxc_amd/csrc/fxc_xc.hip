@@ -302,22 +302,23 @@ constexpr int kChunkGroup = 8;
 // takes chunks 8 g + x only: each XCD's L2 then serves one chunk of every
 // station's spectra at a time.  Within an XCD's stream j = 0, 1, ... (tile
 // j mod ntiles of chunk group j / ntiles) the U = gridDim.x / 8 workgroups of
-// the XCD take runs of kRun consecutive j, so a workgroup's consecutive items
-// are mostly neighbouring tiles of one tile row at one chunk, which share
-// their source stations.  (gridDim.x is a multiple of 8.)
+// the XCD take runs of 2^lg_run consecutive j, so a workgroup's consecutive
+// items are mostly neighbouring tiles of one tile row at one chunk, which
+// share their source stations.  (gridDim.x is a multiple of 8.)
+constexpr int kRunLog = 3;
 struct ItemWalk {
-  static constexpr int kRun = 8;
-  int ntiles, nchunks, xcd, wu, nu;
+  int ntiles, nchunks, lg_run, xcd, wu, nu;
   long long nj;
-  __device__ __forceinline__ ItemWalk(int ntiles_, int nchunks_)
-      : ntiles(ntiles_), nchunks(nchunks_), xcd(blockIdx.x & 7), wu(blockIdx.x >> 3),
-        nu(gridDim.x >> 3),
+  __device__ __forceinline__ ItemWalk(int ntiles_, int nchunks_, int lg_run_ = kRunLog)
+      : ntiles(ntiles_), nchunks(nchunks_), lg_run(lg_run_), xcd(blockIdx.x & 7),
+        wu(blockIdx.x >> 3), nu(gridDim.x >> 3),
         nj((long long)ntiles_ * ((nchunks_ + kChunkGroup - 1) / kChunkGroup)) {}
   // next valid item at or after this workgroup's k-th (items whose chunk is
   // past the end are skipped); -1 when none is left
   __device__ __forceinline__ long long next(long long k, int &tile, int &chunk) const {
     for (;; ++k) {
-      const long long j = (k / kRun) * nu * kRun + (long long)wu * kRun + k % kRun;
+      const long long run = k >> lg_run;
+      const long long j = ((run * nu + wu) << lg_run) + (k - (run << lg_run));
       if (j >= nj) return -1;
       const long long g = j / ntiles;
       tile = (int)(j - g * ntiles);
@@ -326,6 +327,18 @@ struct ItemWalk {
     }
   }
 };
+// Run length of an FP32 launch of nj items per XCD over nu workgroups: the
+// longest whose fullest workgroup takes at most an eighth more items than runs
+// of one would give it; one tile shares nothing between its chunks.  With
+// runs of 8 alone few items kept most workgroups idle (one tile x 118 chunks: 16
+// of 256 busy).
+static int f32_run_log(long long nj, long long nu, int ntiles) {
+  if (ntiles == 1) return 0;
+  const long long even = ceil_div(nj, nu);
+  int lg = kRunLog;
+  while (lg > 0 && ((long long)ceil_div(nj, nu << lg) << lg) * 8 > even * 9) --lg;
+  return lg;
+}
 
 // MFMA contraction.  Per bin: Cr = A.B1, Ci = A.B2 with a_s = [Re | Im] and
 // b2_s = [Im | -Re], so conj(a)*b = Cr + i Ci.  Results are staged in LDS as
@@ -862,7 +875,7 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
 // ms + contraction 14.7 ms (matrix pipe busy 65 %) against 33.7 ms for the
 // vector-ALU form it replaced, which issued the same flops at half the rate
 // and re-read station rows with 8 x 8 pairs per thread; 8 stations x 24
-// windows 17 + 37 us against 85 us.
+// windows 17 + 27 us against 85 us.
 // ---------------------------------------------------------------------------
 constexpr int kF32Group = 4;     // windows per matrix step
 constexpr int kF32TrThreads = 256;
@@ -1026,10 +1039,10 @@ __global__ void __launch_bounds__(kF32Compute + kF32Store) __attribute__((amdgpu
 contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int steps,
                     const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
                     float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
-                    int slab0, int nchunks) {
+                    int slab0, int nchunks, int lg_run) {
   extern __shared__ __align__(16) float2 stage[];  // [2][kF32PhasePairs][kBinChunk], swizzled
   const int tid = threadIdx.x;
-  const ItemWalk walk(ntiles, nchunks);
+  const ItemWalk walk(ntiles, nchunks, lg_run);
   int tile = 0, chunk = 0;
   long long item = walk.next(0, tile, chunk);
   if (item < 0) return;  // the whole workgroup
@@ -2344,8 +2357,10 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
       if (p->f32_slab > 0) FXC_TRY(xc_f32_transpose(p, d_spec, c0 + b, n, st));
       FXC_TRY(xc_mark(p, kTimeContract, true, st));
       const unsigned items = ntl * (unsigned)(ceil_div(n, kChunkGroup) * kChunkGroup);
-      hipLaunchKernelGGL(kern, dim3(std::min(grid, items)), dim3(kF32Compute + kF32Store), lds, st,
-                         p->d_f32, p->nsta, p->nspec, steps, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n);
+      const unsigned wgs = std::min(grid, items);
+      hipLaunchKernelGGL(kern, dim3(wgs), dim3(kF32Compute + kF32Store), lds, st, p->d_f32, p->nsta,
+                         p->nspec, steps, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n,
+                         f32_run_log(items / kChunkGroup, wgs / kChunkGroup, (int)ntl));
       FXC_HIP(hipGetLastError());
       FXC_TRY(xc_mark(p, kTimeContract, false, st));
     }

@@ -374,3 +374,31 @@ def test_lag_halves(gpu, nfft, H):
     Z = X.astype(np.complex128)
     ref = want(Z[src].conj() * Z[rec])
     assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+def test_fp32_few_items_share_the_chip(gpu):
+    """One 32 x 32 station tile has one work item per 16 bins.  Its items go to as many compute
+    units as there are items, so it takes well under the time of eight tiles (in runs of eight
+    items per workgroup both took the same time)."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    nspec, nstep, nsta = 1876, 64, 320
+    g = torch.Generator(device=gpu)
+    g.manual_seed(3)
+    spec = torch.randn((nstep, nsta, nspec), generator=g, device=gpu, dtype=torch.complex64)
+    ms = []
+    for ntile in (1, 8):
+        rec = np.arange(32, 32 + 32 * ntile)
+        plan = XcPlan(nspec, nstep, 1.0, 100, "fp32")
+        plan.set_pairs(nsta, np.repeat(np.arange(32), len(rec)), np.tile(rec, 32))
+        plan.correlate(spec)
+        best = np.inf
+        for _ in range(5):
+            plan.set_timing(True)
+            plan.correlate(spec)
+            best = min(best, plan.get_timing()["contract_ms"])
+        ms.append(best)
+        plan.close()
+    print(f"contraction of 1 and 8 tiles: {ms[0]:.4f} {ms[1]:.4f} ms")
+    assert ms[0] < 0.7 * ms[1]
