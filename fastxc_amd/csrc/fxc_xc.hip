@@ -340,6 +340,94 @@ static int f32_run_log(long long nj, long long nu, int ntiles) {
   return lg;
 }
 
+// ---------------------------------------------------------------------------
+// FP32 contraction on the vector ALU, straight from the spectra: thread = (bin,
+// 8 x 8 micro-tile of pairs), for pair lists and window counts that would not
+// pay for the transposed operand of contract_f32_kernel (xc_f32_vector).
+// Bound: the window loop's load latency; 8 consecutive workgroups take 8
+// consecutive bin chunks of one tile, one per XCD.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(256)
+contract_f32v_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int nspec,
+                     const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
+                     float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
+                     int chunk0, int nchunks) {
+  __shared__ int rows[kTilePairs];
+  __shared__ int active[16];
+  const int group = blockIdx.x / (ntiles * kChunkGroup);
+  const int item = blockIdx.x - group * (ntiles * kChunkGroup);
+  const int tile = item / kChunkGroup;
+  int chunk = group * kChunkGroup + (item - tile * kChunkGroup);
+  if (chunk >= nchunks) return;  // the whole workgroup
+  chunk += chunk0;
+  const int tid = threadIdx.x;
+  const int *trow = tile_rows + (size_t)tile * kTilePairs;
+  for (int i = tid; i < kTilePairs; i += blockDim.x) rows[i] = trow[i];
+  if (tid < 16) active[tid] = 0;
+  __syncthreads();
+  for (int i = tid; i < kTilePairs; i += blockDim.x) {
+    if (rows[i] >= 0) {
+      const int mi = (i >> 5) >> 3, mj = (i & 31) >> 3;
+      active[mi * 4 + mj] = 1;
+    }
+  }
+  __syncthreads();
+  const int b = tid & 15;
+  const int g = tid >> 4;
+  const int mi = g >> 2, mj = g & 3;
+  const int k = chunk * kBinChunk + b;
+  if (k >= nspec || !active[g]) return;
+  const TileDesc td = tiles[tile];
+  const int s0 = td.src_base + mi * 8;
+  const int r0 = td.rec_base + mj * 8;
+  float2 acc[8][8];
+#pragma unroll
+  for (int a = 0; a < 8; ++a)
+#pragma unroll
+    for (int c = 0; c < 8; ++c) acc[a][c] = make_float2(0.f, 0.f);
+  // software pipeline: loads of window w+1 are in flight while window w is
+  // accumulated
+  const size_t wstride = (size_t)nsta * nspec;
+  float2 sv[8], rv[8], sn[8], rn[8];
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+    sv[a] = (s0 + a < nsta) ? spec[(size_t)(s0 + a) * nspec + k] : make_float2(0.f, 0.f);
+    rv[a] = (r0 + a < nsta) ? spec[(size_t)(r0 + a) * nspec + k] : make_float2(0.f, 0.f);
+  }
+  for (int w = 0; w < nstep; ++w) {
+    if (w + 1 < nstep) {
+      const float2 *base = spec + (size_t)(w + 1) * wstride + k;
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        sn[a] = (s0 + a < nsta) ? base[(size_t)(s0 + a) * nspec] : make_float2(0.f, 0.f);
+        rn[a] = (r0 + a < nsta) ? base[(size_t)(r0 + a) * nspec] : make_float2(0.f, 0.f);
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        // conj(s) * r
+        acc[a][c].x += sv[a].x * rv[c].x + sv[a].y * rv[c].y;
+        acc[a][c].y += sv[a].x * rv[c].y - sv[a].y * rv[c].x;
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+      sv[a] = sn[a];
+      rv[a] = rn[a];
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < 8; ++a) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int row = rows[(mi * 8 + a) * kTile + mj * 8 + c];
+      if (row >= 0) store_stream(xspec + (size_t)row * xpitch + k, cscale(acc[a][c], scale));
+    }
+  }
+}
+
 // MFMA contraction.  Per bin: Cr = A.B1, Ci = A.B2 with a_s = [Re | Im] and
 // b2_s = [Im | -Re], so conj(a)*b = Cr + i Ci.  Results are staged in LDS as
 // [pair][bin] and written as 128-byte rows.
@@ -1025,8 +1113,8 @@ __device__ __forceinline__ void f32_bin(const float2 (&src)[kSteps > 0 ? kSteps 
 // with the same waves writing; 16.7 so and without held sources; 19.3 in half
 // tiles with two workgroups per CU, which read half as much again per pair).  One barrier per
 // phase; both kinds of waves pass the same number of them.
-// op holds bins [16 slab0, ...): the chunks of this launch are slab0 ..
-// slab0 + nchunks - 1.  Blocks of 16 x 16 stations without listed pairs are
+// op holds bins [16 chunk0, ...): the chunks of this launch are chunk0 ..
+// chunk0 + nchunks - 1.  Blocks of 16 x 16 stations without listed pairs are
 // skipped.
 // kSteps > 0 (up to kF32HeldSteps): the depth in steps; the sources of the
 // wave's two bins stay in registers while consecutive items share them.
@@ -1039,7 +1127,7 @@ __global__ void __launch_bounds__(kF32Compute + kF32Store) __attribute__((amdgpu
 contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int steps,
                     const TileDesc *__restrict__ tiles, const int *__restrict__ tile_rows,
                     float2 *__restrict__ xspec, long long xpitch, int ntiles, float scale,
-                    int slab0, int nchunks, int lg_run) {
+                    int chunk0, int nchunks, int lg_run) {
   extern __shared__ __align__(16) float2 stage[];  // [2][kF32PhasePairs][kBinChunk], swizzled
   const int tid = threadIdx.x;
   const ItemWalk walk(ntiles, nchunks, lg_run);
@@ -1065,7 +1153,7 @@ contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int step
     while (item >= 0) {
       int ntile = tile, nchunk = chunk;
       const long long nitem = walk.next(item + 1, ntile, nchunk);
-      const int k = (slab0 + chunk) * kBinChunk + b;
+      const int k = (chunk0 + chunk) * kBinChunk + b;
 #pragma unroll 1
       for (int h = 0; h < 2; ++h) {
         int cur[kPer];
@@ -1114,7 +1202,7 @@ contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int step
     return (unsigned)(lane_g * nsta + (s < nsta ? s : nsta - 1));
   };
   auto bin_ptr = [&](int c, int b) {
-    const int k = c * kBinChunk + b, last = nspec - 1 - slab0 * kBinChunk;
+    const int k = c * kBinChunk + b, last = nspec - 1 - chunk0 * kBinChunk;
     return op + (size_t)(k < last ? k : last) * bin_elems;
   };
   // source halves listed with receiver half h (0: the phase has no pairs)
@@ -1759,11 +1847,12 @@ struct fxc_xc_plan {
   unsigned short *d_hi = nullptr, *d_lo = nullptr;
   size_t split_elems = 0;
   bool ws_shared = false;
-  // FP32 form: transposed spectra of slab_chunks 16-bin chunks at a time
-  // (every chunk when the memory allows)
+  // FP32 form: transposed spectra, or (f32_vector, set by each call) none
   float2 *d_f32 = nullptr;
   size_t f32_elems = 0;
-  int f32_slab = 0;
+  bool f32_vector = false;
+  // what the tiles list: strips of 8 sources x 32 receivers, blocks of 16 x 16
+  long long strips = 0, blocks = 0;
   unsigned int *d_amax = nullptr;
   float *d_inv_scale = nullptr, *d_scale = nullptr;
   int scale_cap = 0;
@@ -1983,6 +2072,7 @@ int xc_set_pairs_on(fxc_xc_plan *p, int nsta, const int *h_src, const int *h_rec
   p->chunk_tile_begin.clear();
   p->chunk_row_begin.clear();
   p->npairs = 0;
+  p->strips = p->blocks = 0;
   p->nsta = nsta;
   if (npairs == 0) return FXC_OK;
   const int nblk = (nsta + kTile - 1) / kTile;
@@ -2026,8 +2116,13 @@ int xc_set_pairs_on(fxc_xc_plan *p, int nsta, const int *h_src, const int *h_rec
       td.src_base = (int)(kv.first / nblk) * kTile;
       td.rec_base = (int)(kv.first % nblk) * kTile;
       td.blocks = 0;
-      for (auto &e : cp)
+      unsigned strip = 0;
+      for (auto &e : cp) {
         td.blocks |= 1 << (2 * (e.first / kTile / 16) + e.first % kTile / 16);
+        strip |= 1u << (e.first / kTile / 8);
+      }
+      p->strips += __builtin_popcount(strip);
+      p->blocks += __builtin_popcount(td.blocks);
       p->h_tiles.push_back(td);
       const size_t off = rows.size();
       rows.resize(off + kTilePairs, -1);
@@ -2159,44 +2254,74 @@ static void xc_chunks(const fxc_xc_plan *p, int *first, int *count) {
   *count = band ? p->band_c1 - p->band_c0 : ceil_div(p->nspec, kBinChunk);
 }
 
+// Launch of f32_transpose_kernel for n chunks: 16 stations x 16 windows per
+// workgroup for at most 16 stations, otherwise 64 x 4.
+static dim3 f32_transpose_grid(const fxc_xc_plan *p, int n) {
+  const int wpad = (int)ceil_div(p->nstep, kF32Group) * kF32Group;
+  const int sta = p->nsta <= 16 ? 16 : 64;
+  return dim3((unsigned)n, (unsigned)ceil_div(p->nsta, sta), (unsigned)ceil_div(wpad, 256 / sta));
+}
+
 // Transposed operand of the FP32 form for chunks [c0, c0 + n).
 static int xc_f32_transpose(fxc_xc_plan *p, const float2 *d_spec, int c0, int n, hipStream_t st) {
   FXC_TRY(xc_mark(p, kTimeSplit, true, st));
   const int wpad = (int)ceil_div(p->nstep, kF32Group) * kF32Group;
-  const int sta = p->nsta <= 16 ? 16 : 64;
-  auto kern = sta == 16 ? f32_transpose_kernel<16> : f32_transpose_kernel<64>;
-  hipLaunchKernelGGL(kern,
-                     dim3((unsigned)n, (unsigned)ceil_div(p->nsta, sta),
-                          (unsigned)ceil_div(wpad, 256 / sta)),
-                     dim3(kF32TrThreads), 0, st, d_spec, p->nstep, p->nsta, p->nspec,
-                     c0 * kBinChunk, wpad, p->d_f32);
+  auto kern = p->nsta <= 16 ? f32_transpose_kernel<16> : f32_transpose_kernel<64>;
+  hipLaunchKernelGGL(kern, f32_transpose_grid(p, n), dim3(kF32TrThreads), 0, st, d_spec, p->nstep,
+                     p->nsta, p->nspec, c0 * kBinChunk, wpad, p->d_f32);
   FXC_HIP(hipGetLastError());
   return xc_mark(p, kTimeSplit, false, st);
 }
 
-// Workspace of the transposed operand: every chunk of the band, or, where the
-// device has no room for that, as many as fit (then each slab of chunks is
-// transposed and contracted in turn).
+// Whether the FP32 form contracts on the vector ALU straight from the spectra:
+// where that takes less time than transposing every station's spectra and
+// contracting them on the matrix instructions, which few listed pairs or one
+// or two windows do not pay for.  Estimates in microseconds, from 445 calls (2 to
+// 1000 stations, 1 to 200 windows, 1876 to 37045 bins; all pairs, lists of 1 to
+// 1000 random ones, single sources, neighbours, station components):
+//   vector: the latency of the window loop, two workgroups per compute unit,
+//     or the issue of the listed strips;
+//   matrix: both copies of the spectra, and the latency of the items, one
+//     workgroup per unit, or the listed blocks.
+// The form chosen is within 0.4 % of the faster one on average and 28 % at
+// worst (two pairs of 40 stations x 200 windows); matrix always: 31 % on
+// average, 600 stations x 47 windows with one pair 2160 us against 133, one
+// source 3190 against 1720.  All pairs take the matrix form from 2 or 3 windows
+// on.  One window is always the vector form's, whose operand would be three
+// quarters zeros: 33 stations at 1 Hz 29.7 us against 31.6, 400 stations 2005
+// against 2040, 100 stations at 5 Hz 331 against 325.
+// FXC_XC_F32=vector or matrix overrides (tests).
+static bool xc_f32_vector(const fxc_xc_plan *p) {
+  if (f32_transpose_grid(p, 1).z > 65535) return true;  // the transpose's launch limit
+  if (const char *env = getenv("FXC_XC_F32")) {
+    if (strcmp(env, "vector") == 0) return true;
+    if (strcmp(env, "matrix") == 0) return false;
+  }
+  if (p->nstep == 1) return true;
+  int c0 = 0, n = 0;
+  xc_chunks(p, &c0, &n);
+  const double C = n, W = p->nstep, pad = (double)ceil_div(p->nstep, kF32Group) * kF32Group;
+  const double tc = C * (double)p->h_tiles.size();
+  const double vec =
+      std::max(std::ceil(tc / 512) * (1.1 + 0.76 * W), (double)p->strips * C * (3.8e-3 + 1.44e-3 * W));
+  const double mat = (double)p->nsta * C * (W + pad) * 21e-6 +
+                     std::max(std::ceil(tc / 256) * (1.3 + 0.1 * pad),
+                              (double)p->blocks * C * (3e-3 + 0.5e-3 * pad));
+  return vec < mat;
+}
+
+// Workspace of the transposed operand.
 static int xc_f32_workspace(fxc_xc_plan *p) {
   int c0 = 0, n = 0;
   xc_chunks(p, &c0, &n);
-  const size_t chunk = (size_t)kBinChunk * p->nsta * ceil_div(p->nstep, kF32Group) * kF32Group;
-  if (chunk * n > p->f32_elems && !(p->f32_slab > 0 && p->f32_elems >= chunk * kChunkGroup)) {
-    dfree(p->d_f32);
-    p->d_f32 = nullptr;
-    p->f32_elems = 0;
-    for (int m = n;; m = std::max(kChunkGroup, m / 2)) {
-      const int rc = dmalloc((void **)&p->d_f32, chunk * m * sizeof(float2));
-      if (rc == FXC_OK) {
-        p->f32_elems = chunk * m;
-        break;
-      }
-      (void)hipGetLastError();  // out of memory: a smaller slab
-      if (m <= kChunkGroup) return rc;
-    }
-  }
-  const size_t fit = p->f32_elems / chunk;
-  p->f32_slab = fit >= (size_t)n ? 0 : (int)(fit / kChunkGroup) * kChunkGroup;
+  const size_t elems =
+      (size_t)kBinChunk * n * p->nsta * ceil_div(p->nstep, kF32Group) * kF32Group;
+  if (elems <= p->f32_elems) return FXC_OK;
+  dfree(p->d_f32);
+  p->d_f32 = nullptr;
+  p->f32_elems = 0;
+  FXC_TRY(dmalloc((void **)&p->d_f32, elems * sizeof(float2)));
+  p->f32_elems = elems;
   return FXC_OK;
 }
 
@@ -2204,8 +2329,12 @@ static int xc_f32_workspace(fxc_xc_plan *p) {
 static int xc_prepare_spectra(fxc_xc_plan *p, const float2 *d_spec, hipStream_t st) {
   if (p->precision == FXC_PREC_PLAIN) return FXC_OK;
   if (p->precision == FXC_PREC_FP32) {
-    FXC_TRY(xc_f32_workspace(p));
-    if (p->f32_slab > 0) return FXC_OK;  // transposed slab by slab
+    p->f32_vector = xc_f32_vector(p);
+    if (!p->f32_vector && xc_f32_workspace(p) != FXC_OK) {
+      (void)hipGetLastError();  // no room for the operand: the form without one
+      p->f32_vector = true;
+    }
+    if (p->f32_vector) return FXC_OK;
     int c0 = 0, n = 0;
     xc_chunks(p, &c0, &n);
     return xc_f32_transpose(p, d_spec, c0, n, st);
@@ -2332,7 +2461,7 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
   const float scale = 1.0f / (float)p->nstep;
   const TileDesc *tiles = p->d_tiles + t0;
   const int *trows = p->d_tile_rows + t0 * kTilePairs;
-  if (p->precision != FXC_PREC_FP32) FXC_TRY(xc_mark(p, kTimeContract, true, st));
+  FXC_TRY(xc_mark(p, kTimeContract, true, st));
   if (p->precision == FXC_PREC_PLAIN) {
     const long long r0 = p->chunk_row_begin[c], nrows = p->chunk_row_begin[c + 1] - r0;
     const int nbk = ceil_div(p->nspec, 256);
@@ -2343,6 +2472,9 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
       hipLaunchKernelGGL(plain_accum_kernel, dim3((unsigned)grid), dim3(256), 0, st,
                          d_spec + w * win, p->nspec, p->d_row_src + r0, p->d_row_rec + r0, nrows,
                          dst, p->xpitch, nbk, scale);
+  } else if (p->precision == FXC_PREC_FP32 && p->f32_vector) {
+    hipLaunchKernelGGL(contract_f32v_kernel, dim3(nwg), dim3(256), 0, st, d_spec, p->nstep, p->nsta,
+                       p->nspec, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0, nbc);
   } else if (p->precision == FXC_PREC_FP32) {
     const size_t lds = (size_t)kTilePairs * kBinChunk * sizeof(float2);
     const int steps = (int)ceil_div(p->nstep, kF32Group);
@@ -2351,20 +2483,10 @@ static int xc_contract_chunk(fxc_xc_plan *p, const float2 *d_spec, long long c, 
                                 (int)lds));
     unsigned grid = 0;
     FXC_TRY(xc_persistent_grid(&grid));
-    const int slab = p->f32_slab > 0 ? p->f32_slab : nbc;
-    for (int b = 0; b < nbc; b += slab) {
-      const int n = std::min(slab, nbc - b);
-      if (p->f32_slab > 0) FXC_TRY(xc_f32_transpose(p, d_spec, c0 + b, n, st));
-      FXC_TRY(xc_mark(p, kTimeContract, true, st));
-      const unsigned items = ntl * (unsigned)(ceil_div(n, kChunkGroup) * kChunkGroup);
-      const unsigned wgs = std::min(grid, items);
-      hipLaunchKernelGGL(kern, dim3(wgs), dim3(kF32Compute + kF32Store), lds, st, p->d_f32, p->nsta,
-                         p->nspec, steps, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0 + b, n,
-                         f32_run_log(items / kChunkGroup, wgs / kChunkGroup, (int)ntl));
-      FXC_HIP(hipGetLastError());
-      FXC_TRY(xc_mark(p, kTimeContract, false, st));
-    }
-    return FXC_OK;
+    const unsigned wgs = std::min(grid, nwg);
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(kF32Compute + kF32Store), lds, st, p->d_f32, p->nsta,
+                       p->nspec, steps, tiles, trows, dst, p->xpitch, (int)ntl, scale, c0, nbc,
+                       f32_run_log(nwg / kChunkGroup, wgs / kChunkGroup, (int)ntl));
   } else {
     const size_t lds = (size_t)kTilePairs * kBinChunk * sizeof(float2);
     // grid.y carries the tile count to the launcher (the launch itself is 1-D)

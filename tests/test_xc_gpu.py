@@ -376,13 +376,14 @@ def test_lag_halves(gpu, nfft, H):
     assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
 
 
-def test_fp32_few_items_share_the_chip(gpu):
-    """One 32 x 32 station tile has one work item per 16 bins.  Its items go to as many compute
+def test_fp32_few_items_share_the_chip(gpu, monkeypatch):
+    """One 32 x 32 station tile of the matrix form has one work item per 16 bins.  Its items go to as many compute
     units as there are items, so it takes well under the time of eight tiles (in runs of eight
     items per workgroup both took the same time)."""
     import torch
     from fastxc_amd.ops import XcPlan
 
+    monkeypatch.setenv("FXC_XC_F32", "matrix")  # whose items these are
     nspec, nstep, nsta = 1876, 64, 320
     g = torch.Generator(device=gpu)
     g.manual_seed(3)
@@ -402,3 +403,59 @@ def test_fp32_few_items_share_the_chip(gpu):
         plan.close()
     print(f"contraction of 1 and 8 tiles: {ms[0]:.4f} {ms[1]:.4f} ms")
     assert ms[0] < 0.7 * ms[1]
+
+
+@pytest.mark.parametrize("form", ["vector", "matrix"])
+@pytest.mark.parametrize("nsta,nstep,pairs", [(70, 1, "all"), (70, 2, "all"), (33, 5, "all"), (130, 7, "one"),
+                                              (130, 3, "source"), (97, 13, "random"), (40, 100, "random")])
+def test_fp32_both_forms(gpu, monkeypatch, form, nsta, nstep, pairs):
+    """The FP32 contraction on the vector ALU and on the matrix instructions, for dense and sparse
+    pair lists (duplicates, either order, one station with itself), a band, and row chunks, against
+    the FP64 stack.  fp32 sums of 2 nstep products: relative error below 2 nstep 2^-24 of sum
+    |a||b|."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    monkeypatch.setenv("FXC_XC_F32", form)
+    nspec = 201
+    rng = np.random.default_rng(nsta * 1000 + nstep)
+    spec = (rng.standard_normal((nstep, nsta, nspec)) +
+            1j * rng.standard_normal((nstep, nsta, nspec))).astype(np.complex64)
+    src, rec = {"all": np.triu_indices(nsta), "one": (np.array([nsta - 1]), np.array([3])),
+                "source": (np.full(nsta, 37), np.arange(nsta)),
+                "random": tuple(rng.integers(0, nsta, (2, 60)))}[pairs]
+    src, rec = np.concatenate([src, src[:2]]), np.concatenate([rec, rec[:2]])
+    z = spec.astype(np.complex128)
+    want = (z[:, src].conj() * z[:, rec]).mean(axis=0)
+    bound = (np.abs(z[:, src]) * np.abs(z[:, rec])).mean(axis=0) * (2 * nstep + 2) * 2.0 ** -24
+    sd = torch.from_numpy(spec).to(gpu)
+    for chunk, band in ((0, None), (17, None), (0, (70, 130))):
+        plan = XcPlan(nspec, nstep, 0.1, 20, "fp32", chunk_rows=chunk)
+        if band:
+            plan.set_band(*band)
+        plan.set_pairs(nsta, src, rec)
+        got = plan.cross_spectra(sd).cpu().numpy()
+        lo, hi = (band[0] // 16 * 16, (band[1] // 16 + 1) * 16) if band else (0, nspec)
+        assert (np.abs(got - want) <= 2 * bound)[:, lo:hi].all()
+        assert not got[:, :lo].any() and not got[:, hi:].any()
+        plan.close()
+
+
+def test_fp32_sparse_pairs_need_no_operand(gpu):
+    """A few pairs of many stations are contracted from the spectra themselves: the call holds no
+    transposed copy of them (whose cost is that of every station)."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    nspec, nstep, nsta = 9262, 8, 200
+    spec = torch.zeros((nstep, nsta, nspec), device=gpu, dtype=torch.complex64)
+    plan = XcPlan(nspec, nstep, 0.2, 100, "fp32")
+    plan.set_pairs(nsta, [3, 150], [190, 20])
+    out = torch.empty((2, 201), device=gpu)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan.correlate(spec, out)
+    torch.cuda.synchronize()
+    held = free - torch.cuda.mem_get_info()[0]
+    print(f"held {held} of {spec.numel() * 8} bytes of spectra")
+    assert held < spec.numel() * 8 // 4
