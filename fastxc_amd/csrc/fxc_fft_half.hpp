@@ -5,6 +5,7 @@
 #include "fxc_plan_cache.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace fxc {
 
@@ -151,6 +152,31 @@ half_c2r_kernel(const float2 *__restrict__ in, long long in_dist, long long rows
       put(n + Q, csub(f0, p));
     }
   }
+}
+
+// Whether a call of `rows` rows takes the halves.  A row is one workgroup's, so
+// few rows leave the chip to the serial chain of two transforms, where the four
+// passes spread over it.  Measured over 21 lengths from 40960 to 80640 (times of
+// the halves over those of the passes, r2c / c2r):
+//   Q <= 12000            1 row 0.94 / 0.91, 16 rows 0.93 / 0.92;
+//   Q > 12000             1 row 1.03-1.10 / 0.98-1.04, 8 rows 1.00-1.05 / 0.96-1.02,
+//                         24 rows 0.92-0.97 / 0.88-0.93;
+//   Q > 17000, radix 21   (few butterflies of many registers) 1 row 1.10-1.23 /
+//                         1.04-1.15, 16 rows 1.01-1.06 / 0.96-1.01, 32 rows
+//                         0.92-0.99 / 0.90-0.95.
+// fused: with a call's steps inside the halves and passes of their own beside the
+// four (sac2spec of one channel at 20 Hz, 72000 samples): 1 row 382 against 317
+// us, 12 rows 412 against 379, 16 rows 411 against 396, 24 rows 415 against 415,
+// and with the multi-band running mean 16 rows 745 against 757.
+// FXC_FFT_HALVES=0 or 1 overrides (tests).
+inline bool half_pays(const LargeFft *p, long long rows, bool fused) {
+  if (!p->pq || rows < 1) return false;
+  if (const char *env = getenv("FXC_FFT_HALVES")) return atoi(env) != 0;
+  if (p->pq->dev.n <= 12000) return true;
+  if (fused) return rows >= 16;
+  const bool r21 = p->pq->dev.n > 17000 && p->pq->dev.radix[0] == 21;
+  if (p->sign > 0) return rows >= (r21 ? 16 : 1);
+  return rows >= (r21 ? 24 : 12);
 }
 
 inline int half_grid(long long rows, unsigned *grid) {

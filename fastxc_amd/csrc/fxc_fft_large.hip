@@ -255,15 +255,9 @@ int large_c2c(const LargeFft *p, const float2 *in, long long in_dist, float2 *ou
   return FXC_OK;
 }
 
-int large_r2c(int n, const float *in, long long in_dist, int in_len, float2 *out,
-              long long out_dist, long long rows, float2 *work, float scale, hipStream_t st) {
-  FXC_CHECK_ARG(n >= 8 && n % 2 == 0, "fft: real length %d must be even", n);
-  const int M = n / 2;
-  const LargeFft *p = nullptr;
-  FXC_TRY(large_plan(M, -1, &p));
-  if (p->pq && rows > 0)
-    return half_r2c(p, in, in_dist, in_len, out, out_dist, rows, work, PlainSample{},
-                    ScaledBin{scale}, st);
+int four_step_r2c(const LargeFft *p, const float *in, long long in_dist, int in_len, float2 *out,
+                  long long out_dist, long long rows, float2 *work, float scale, hipStream_t st) {
+  const int M = p->M;
   float2 *w0 = work, *w1 = work + (size_t)rows * M;
   hipLaunchKernelGGL(large_pack_kernel, grid_rows(M, rows, 256), dim3(256), 0, st, in, in_dist,
                      in_len, w0, M);
@@ -275,14 +269,10 @@ int large_r2c(int n, const float *in, long long in_dist, int in_len, float2 *out
   return FXC_OK;
 }
 
-int large_c2r(int n, const float2 *in, long long in_dist, float *out, long long out_dist,
-              int out_len, long long rows, float2 *work, double scale, hipStream_t st) {
-  FXC_CHECK_ARG(n >= 8 && n % 2 == 0, "fft: real length %d must be even", n);
-  const int M = n / 2;
-  const LargeFft *p = nullptr;
-  FXC_TRY(large_plan(M, 1, &p));
-  if (p->pq && rows > 0)
-    return half_c2r(p, in, in_dist, out, out_dist, out_len, rows, work, scale, PlainBin{}, st);
+int four_step_c2r(const LargeFft *p, const float2 *in, long long in_dist, float *out,
+                  long long out_dist, int out_len, long long rows, float2 *work, double scale,
+                  hipStream_t st) {
+  const int M = p->M;
   float2 *w0 = work, *w1 = work + (size_t)rows * M;
   hipLaunchKernelGGL(large_fold_kernel, grid_rows(M, rows, 256), dim3(256), 0, st, in, in_dist, M,
                      p->d_half, w0);
@@ -292,6 +282,27 @@ int large_c2r(int n, const float2 *in, long long in_dist, float *out, long long 
                      out_dist, out_len, scale);
   FXC_HIP(hipGetLastError());
   return FXC_OK;
+}
+
+int large_r2c(int n, const float *in, long long in_dist, int in_len, float2 *out,
+              long long out_dist, long long rows, float2 *work, float scale, hipStream_t st) {
+  FXC_CHECK_ARG(n >= 8 && n % 2 == 0, "fft: real length %d must be even", n);
+  const LargeFft *p = nullptr;
+  FXC_TRY(large_plan(n / 2, -1, &p));
+  if (half_pays(p, rows, false))
+    return half_r2c(p, in, in_dist, in_len, out, out_dist, rows, work, PlainSample{},
+                    ScaledBin{scale}, st);
+  return four_step_r2c(p, in, in_dist, in_len, out, out_dist, rows, work, scale, st);
+}
+
+int large_c2r(int n, const float2 *in, long long in_dist, float *out, long long out_dist,
+              int out_len, long long rows, float2 *work, double scale, hipStream_t st) {
+  FXC_CHECK_ARG(n >= 8 && n % 2 == 0, "fft: real length %d must be even", n);
+  const LargeFft *p = nullptr;
+  FXC_TRY(large_plan(n / 2, 1, &p));
+  if (half_pays(p, rows, false))
+    return half_c2r(p, in, in_dist, out, out_dist, out_len, rows, work, scale, PlainBin{}, st);
+  return four_step_c2r(p, in, in_dist, out, out_dist, out_len, rows, work, scale, st);
 }
 
 void large_release() {

@@ -49,6 +49,13 @@ int large_r2c(int n, const float *in, long long in_dist, int in_len, float2 *out
 // the product in double.  work: 2 x rows x M complex.
 int large_c2r(int n, const float2 *in, long long in_dist, float *out, long long out_dist,
               int out_len, long long rows, float2 *work, double scale, hipStream_t st);
+// The four-step form alone (plan of n/2 points with the sign of the direction);
+// large_r2c and large_c2r take two halves in LDS where half_pays says so.
+int four_step_r2c(const LargeFft *p, const float *in, long long in_dist, int in_len, float2 *out,
+                  long long out_dist, long long rows, float2 *work, float scale, hipStream_t st);
+int four_step_c2r(const LargeFft *p, const float2 *in, long long in_dist, float *out,
+                  long long out_dist, int out_len, long long rows, float2 *work, double scale,
+                  hipStream_t st);
 // Complex elements of work the real transforms of length n need per row.
 inline long long large_real_work(int n) { return 2LL * (n / 2); }
 // Frees every cached four-step plan's tables (fxc_release_plans).

@@ -2103,19 +2103,21 @@ static int s2sL_apply(V *x, long long pitch, int n, long long rows, const Op &op
 }
 
 // Long-window path: X = bin(R2C(sample(x))) and x = C2R(bin(X)).  Where half a
-// transform fits the LDS the two are part of it; otherwise they are passes of
-// their own (in place) around four-step transforms of kLargeChunk rows.
+// transform fits the LDS and the rows are enough (half_pays) the two are part of
+// it; otherwise they are passes of their own (in place) around four-step
+// transforms of kLargeChunk rows.
 template <class SampleOp, class BinOp>
 static int s2sL_r2c(fxc_s2s_plan *p, int n, float *x, const SampleOp &sample, float2 *X,
                     long long Xd, const BinOp &bin, long long rows, hipStream_t st) {
   const int seg = p->cfg.seg;
   const LargeFft *f = nullptr;
   FXC_TRY(large_plan(n / 2, -1, &f));
-  if (f->pq) return half_r2c(f, x, seg, seg, X, Xd, rows, p->d_Lw, sample, bin, st);
+  if (half_pays(f, rows, true))
+    return half_r2c(f, x, seg, seg, X, Xd, rows, p->d_Lw, sample, bin, st);
   if (!std::is_same<SampleOp, PlainSample>::value) FXC_TRY(s2sL_apply(x, seg, seg, rows, sample, st));
   for (long long r = 0; r < rows; r += kLargeChunk)
-    FXC_TRY(large_r2c(n, x + r * seg, seg, seg, X + r * Xd, Xd, std::min(kLargeChunk, rows - r),
-                      p->d_Lw, 1.f, st));
+    FXC_TRY(four_step_r2c(f, x + r * seg, seg, seg, X + r * Xd, Xd, std::min(kLargeChunk, rows - r),
+                          p->d_Lw, 1.f, st));
   return s2sL_apply(X, Xd, n / 2 + 1, rows, bin, st);
 }
 
@@ -2125,11 +2127,12 @@ static int s2sL_c2r(fxc_s2s_plan *p, int n, float2 *X, long long Xd, const BinOp
   const int seg = p->cfg.seg;
   const LargeFft *f = nullptr;
   FXC_TRY(large_plan(n / 2, 1, &f));
-  if (f->pq) return half_c2r(f, X, Xd, x, seg, seg, rows, p->d_Lw, scale, bin, st);
+  if (half_pays(f, rows, true))
+    return half_c2r(f, X, Xd, x, seg, seg, rows, p->d_Lw, scale, bin, st);
   if (!std::is_same<BinOp, PlainBin>::value) FXC_TRY(s2sL_apply(X, Xd, n / 2 + 1, rows, bin, st));
   for (long long r = 0; r < rows; r += kLargeChunk)
-    FXC_TRY(large_c2r(n, X + r * Xd, Xd, x + r * seg, seg, seg, std::min(kLargeChunk, rows - r),
-                      p->d_Lw, scale, st));
+    FXC_TRY(four_step_c2r(f, X + r * Xd, Xd, x + r * seg, seg, seg,
+                          std::min(kLargeChunk, rows - r), p->d_Lw, scale, st));
   return FXC_OK;
 }
 

@@ -60,3 +60,55 @@ def test_real_halves(gpu, n, in_len, rows):
     for out_len in (n, in_len, n // 2 + 1):
         y = ops.fft_c2r(torch.from_numpy(z).to(gpu), n, out_len=out_len).cpu().numpy()
         assert rel_l2(y, ref[:, :out_len]) < 1e-6
+
+
+@pytest.mark.parametrize("halves", [0, 1])
+@pytest.mark.parametrize("n,in_len,rows", [(48000, 47999, 1), (50400, 50400, 5), (72576, 72000, 1), (74088, 72000, 17),
+                                           (75000, 70001, 2), (79380, 79380, 25)])
+def test_real_forms(gpu, monkeypatch, halves, n, in_len, rows):
+    """Lengths beyond one workgroup's LDS by two half-length LDS transforms and by the four steps
+    over memory, either of which a row count may take."""
+    import torch
+    from fastxc_amd import ops
+
+    monkeypatch.setenv("FXC_FFT_HALVES", str(halves))
+    rng = np.random.default_rng(n + halves)
+    x = rng.standard_normal((rows, in_len)).astype(np.float32)
+    X = ops.fft_r2c(torch.from_numpy(x).to(gpu), n=n).cpu().numpy()
+    want = np.fft.rfft(x.astype(np.float64), n=n)
+    assert rel_l2(X, want) < 1e-6
+    assert np.all(X[:, 0].imag == 0) and np.all(X[:, -1].imag == 0)
+    for out_len in (n, in_len):
+        y = ops.fft_c2r(torch.from_numpy(want.astype(np.complex64)).to(gpu), n, out_len=out_len).cpu().numpy()
+        assert rel_l2(y, (np.fft.irfft(want, n=n) * n)[:, :out_len]) < 1e-6
+
+
+def test_few_long_rows_take_the_faster_form(gpu, monkeypatch):
+    """One row of 74088 points is left to the four steps, which spread it over the chip: a call is
+    faster than with both halves in one workgroup."""
+    import time
+
+    import torch
+    from fastxc_amd import ops
+
+    x = torch.randn((1, 74088), device=gpu)
+
+    def best(halves):
+        if halves is None:
+            monkeypatch.delenv("FXC_FFT_HALVES", raising=False)
+        else:
+            monkeypatch.setenv("FXC_FFT_HALVES", halves)
+        t = []
+        for _ in range(40):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(10):
+                ops.fft_r2c(x)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    best("1")
+    forced, own = best("1"), best(None)
+    print(f"ten calls: halves {forced * 1e3:.3f} ms, own choice {own * 1e3:.3f} ms")
+    assert own < 0.94 * forced
