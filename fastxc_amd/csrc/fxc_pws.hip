@@ -8,7 +8,7 @@
 // and that is a real-to-real map.  Two rows therefore share one complex row,
 // z = s0 x_0 + i s1 x_1, whose spectrum is multiplied by -i sgn(k) in place, in
 // the forward transform's digit-reversed order, and transformed back by the
-// pass order that consumes it: one forward and one inverse transform per two
+// pass order that consumes it (s0, s1: pow2_scale): one forward and one inverse transform per two
 // rows, in one LDS row, with no spectrum in HBM.  Lengths of coprime axes
 // (2001 = 3 x 23 x 29) take both transforms without twiddles and their large
 // primes on the matrix instructions (fxc_pfa.hpp).  Rows of other lengths
@@ -33,15 +33,6 @@ constexpr int kPwsMaxLen = 8192;
 // How a length's Hilbert transforms run: mixed-radix passes, convolution
 // (Bluestein lengths), or axes of coprime radices without twiddles.
 enum PwsForm { kPwsMixed, kPwsConv, kPwsAxes };
-
-// Scale s0, s1 are powers of two that bring each row's largest |x| into
-// [1/2, 1), so both rows of a complex row carry the transform's rounding
-// relative to their own size and the unscaling is exact.
-__device__ __forceinline__ float pow2_scale(float mx) {
-  int e = 0;
-  if (mx > 0.f && isfinite(mx)) (void)frexpf(mx, &e);
-  return ldexpf(1.f, -e);
-}
 
 constexpr int pws_waves(int form, int per) { return per > 8 ? 2 : form == kPwsAxes ? 4 : 3; }
 
@@ -240,7 +231,7 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
           m0 = fmaxf(m0, red[0][2 * t][w]);
           m1 = fmaxf(m1, red[0][2 * t + 1][w]);
         }
-        const float u0 = 1.f / pow2_scale(m0), u1 = 1.f / pow2_scale(m1);
+        const float u0 = pow2_unscale(m0), u1 = pow2_unscale(m1);
         // mean and n/2 component of both rows
         float2 mean, nyq = make_float2(0.f, 0.f);
         if constexpr (kBlue) {

@@ -43,10 +43,8 @@ constexpr int kVoiceThreads = 512; // PWS and TF-PWS voice workgroups
 // (hilbertTransformKernel after R2C).  Output natural order, [rows][n].
 // Two real rows share one complex transform, z = s0 x0 + i s1 x1, whose
 // spectrum separates as s0 A0[k] = Z[k] + conj Z[n-k] and
-// s1 A1[k] = -i (Z[k] - conj Z[n-k]).  s0, s1 are powers of two that bring
-// each row's largest |x| into [1, 2), so both rows carry the transform's
-// rounding relative to their own size and the unscaling is exact.  per_wg
-// transforms (2 per_wg rows) per workgroup.  A workgroup whose rows hold a
+// s1 A1[k] = -i (Z[k] - conj Z[n-k]) (s0, s1: pow2_scale).  per_wg transforms
+// (2 per_wg rows) per workgroup.  A workgroup whose rows hold a
 // non-finite value transforms its rows one by one instead, so such a value
 // stays in its own row, as in a transform per row.
 constexpr int kAnalyticMaxPer = 3;
@@ -135,15 +133,11 @@ analytic_kernel(const float *__restrict__ x, long long rows, int per_wg, StackFf
     }
     return;
   }
-  // scales 2^-e with max |x| in [2^(e-1), 2^e); 1 for an all-zero row (or
-  // a non-finite maximum, which then propagates as in a single transform)
-  float sc[2 * kAnalyticMaxPer];
+  float sc[2 * kAnalyticMaxPer], un[2 * kAnalyticMaxPer];
 #pragma unroll
   for (int r = 0; r < 2 * kAnalyticMaxPer; ++r) {
-    const float mx = __uint_as_float(rmax[r]);
-    int e = 0;
-    if (mx > 0.f && isfinite(mx)) (void)frexpf(mx, &e);
-    sc[r] = ldexpf(1.f, -e);
+    sc[r] = pow2_scale(__uint_as_float(rmax[r]));
+    un[r] = pow2_unscale(__uint_as_float(rmax[r]));
   }
 #pragma unroll
   for (int t = 0; t < kAnalyticMaxPer; ++t) {
@@ -159,7 +153,7 @@ analytic_kernel(const float *__restrict__ x, long long rows, int per_wg, StackFf
 #pragma unroll
   for (int t = 0; t < kAnalyticMaxPer; ++t) {
     if (t >= nt) break;
-    const float u0 = 1.f / sc[2 * t], u1 = 1.f / sc[2 * t + 1];
+    const float u0 = un[2 * t], u1 = un[2 * t + 1];
     for (int k = tid; k < n; k += blockDim.x) {
       float2 a0 = make_float2(0.f, 0.f), a1 = make_float2(0.f, 0.f);
       if (k >= 1 && k < half) {

@@ -116,6 +116,22 @@ __device__ __forceinline__ void flat_rows(int i0, int step, int n, int (&t)[kB],
   }
 }
 
+// Scale of a row whose largest |x| is mx: a power of two that brings it into
+// [1/2, 1), so that rows which share one complex transform carry its rounding
+// relative to their own size and the unscaling is exact; 1 for an all-zero row
+// (or a non-finite maximum).
+__device__ __forceinline__ float pow2_scale(float mx) {
+  int e = 0;
+  if (mx > 0.f && isfinite(mx)) (void)frexpf(mx, &e);
+  return ldexpf(1.f, -e);
+}
+// Its inverse; 0 for an all-zero row, which then stays zero: what the transform
+// leaves in its part is the rounding of the row beside it, and a phase of that is
+// as large as any other.
+__device__ __forceinline__ float pow2_unscale(float mx) {
+  return mx == 0.f ? 0.f : 1.f / pow2_scale(mx);
+}
+
 // Loads of rows a kernel reads exactly once: nontemporal, so the twiddles
 // and tables every workgroup reads stay in L2.
 __device__ __forceinline__ float stream_load(const float *p) { return __builtin_nontemporal_load(p); }

@@ -303,3 +303,27 @@ def test_tfpws_coprime_lengths(gpu, N, counts):
             continue
         want = stack.tfpws(pre[g], w[g], lin[p], band=band, delta=1.0)
         assert rel_l2(out[p], want) < 2e-5
+
+
+@pytest.mark.parametrize("kind", ["pws", "tfpws"])
+@pytest.mark.parametrize("n", [2001, 2000, 512, 345, 401, 1006])
+def test_zero_rows_have_no_phase(gpu, kind, n):
+    """An all-zero group (a dead channel) shares a complex transform with the row beside it and
+    still adds nothing, whatever that row's size; the linear stack of a dead pair is zero."""
+    import torch
+    from fastxc_amd import ops
+
+    rng = np.random.default_rng(n)
+    off = np.array([0, 5, 9, 11])
+    x = _records(rng, off[-1], n)
+    x[2] *= np.float32(1e4)
+    x[[1, 3, 8, 9, 10]] = 0.0  # beside either neighbour; the third pair has no signal
+    w = np.concatenate([np.full(b - a, 1.0 / (b - a)) for a, b in zip(off, off[1:])]).astype(np.float32)
+    lin = np.stack([x[a:b].mean(axis=0) for a, b in zip(off, off[1:])])
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    got = getattr(ops, kind)(d(x), d(w), off, d(lin)).cpu().numpy()
+    for p in range(2):
+        g = slice(off[p], off[p + 1])
+        want = getattr(stack, kind)(x[g], w[g], lin[p])
+        assert rel_l2(got[p], want) < (1e-5 if kind == "pws" else 1e-4)
+    assert not got[2].any()
