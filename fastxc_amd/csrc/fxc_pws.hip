@@ -29,6 +29,7 @@
 namespace fxc {
 
 constexpr int kPwsMaxLen = 8192;
+constexpr float kSumScale = 0x1p-14f;  // of a row's sums (exact)
 
 // How a length's Hilbert transforms run: mixed-radix passes, convolution
 // (Bluestein lengths), or axes of coprime radices without twiddles.
@@ -123,9 +124,10 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
         mx.y = fmaxf(mx.y, fabsf(v.y));
         nonfinite |= !isfinite(v.x) || !isfinite(v.y);
         if constexpr (kBlue) {
-          const float s = (tid + k * kThreads) & 1 ? -1.f : 1.f;
-          sm.x += v.x;
-          sm.y += v.y;
+          // (kPwsMaxLen times any finite value stays finite)
+          const float s = (tid + k * kThreads) & 1 ? -kSumScale : kSumScale;
+          sm.x += v.x * kSumScale;
+          sm.y += v.y * kSumScale;
           sa.x += s * v.x;
           sa.y += s * v.y;
         }
@@ -243,8 +245,9 @@ pws_kernel(const float *__restrict__ x, const float *__restrict__ weights,
             b.x += alt[2 * t][w];
             b.y += alt[2 * t + 1][w];
           }
-          mean = make_float2(a.x * invn, a.y * invn);
-          if (even) nyq = make_float2(b.x * invn, b.y * invn);
+          constexpr float up = 1.f / kSumScale;
+          mean = make_float2(a.x * invn * up, a.y * invn * up);
+          if (even) nyq = make_float2(b.x * invn * up, b.y * invn * up);
         } else {
           mean = make_float2(dc[t].x * (u0 * invn), dc[t].y * (u1 * invn));
           if (even) nyq = make_float2(ny[t].x * (u0 * invn), ny[t].y * (u1 * invn));

@@ -119,11 +119,12 @@ __device__ __forceinline__ void flat_rows(int i0, int step, int n, int (&t)[kB],
 // Scale of a row whose largest |x| is mx: a power of two that brings it into
 // [1/2, 1), so that rows which share one complex transform carry its rounding
 // relative to their own size and the unscaling is exact; 1 for an all-zero row
-// (or a non-finite maximum).
+// (or a non-finite maximum).  The exponent stays within 126, where the scale and
+// its reciprocal are both normal: rows beyond are brought as near as that.
 __device__ __forceinline__ float pow2_scale(float mx) {
   int e = 0;
   if (mx > 0.f && isfinite(mx)) (void)frexpf(mx, &e);
-  return ldexpf(1.f, -e);
+  return ldexpf(1.f, -max(-126, min(126, e)));
 }
 // Its inverse; 0 for an all-zero row, which then stays zero: what the transform
 // leaves in its part is the rounding of the row beside it, and a phase of that is

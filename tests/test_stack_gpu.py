@@ -327,3 +327,34 @@ def test_zero_rows_have_no_phase(gpu, kind, n):
         want = getattr(stack, kind)(x[g], w[g], lin[p])
         assert rel_l2(got[p], want) < (1e-5 if kind == "pws" else 1e-4)
     assert not got[2].any()
+
+@pytest.mark.parametrize("kind", ["pws", "tfpws"])
+@pytest.mark.parametrize("n", [2001, 2000, 512, 345, 2003, 1006])
+@pytest.mark.parametrize("size", [1e-40, 3e-39, 1.2e38, 2e38])
+def test_stacks_with_rows_at_the_ends_of_the_range(gpu, kind, n, size):
+    """A finite row of subnormal size, or one (of constant envelope) whose square overflows, beside
+    ordinary rows: the stack stays finite, and is that with the row left at zero (a subnormal row
+    adds 1e-31 of the others; the phase of an overflowing one is zero) for every form of the
+    transform.  The time-frequency stack of the large row is not compared: its spectrum
+    overflows."""
+    import torch
+    from fastxc_amd import ops
+
+    if kind == "tfpws" and size > 1:
+        pytest.skip("the spectrum of such a row is not finite")
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((5, n)).astype(np.float32)
+    for r in (1, 4):
+        v = np.sin(2 * np.pi * (5 + r) * np.arange(n) / n) if size > 1 else x[r] / np.abs(x[r]).max()
+        x[r] = (v * size).astype(np.float32)
+    w = np.full(5, 0.2, np.float32)
+    lin = rng.standard_normal((1, n)).astype(np.float32)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    run = lambda a: getattr(ops, kind)(d(a), d(w), np.array([0, 5]), d(lin)).cpu().numpy()
+    got = run(x)
+    x[1] = x[4] = 0.0
+    want = run(x)
+    assert np.isfinite(got).all()
+    # the row beside it takes the rounding of a shared transform, about 1e-7 of its own size, which
+    # turns a phase by that over the envelope's relative size (0.02 and more): 5e-6, over 3 of 5 rows
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
