@@ -2538,23 +2538,31 @@ static bool xc_lag_r0_on() {
   return !off;
 }
 
+// Work rows of the four-step lag synthesis.
+static int xc_lag_workspace(fxc_xc_plan *p) {
+  if (p->d_lwork || !p->large_lag || p->half_lag) return FXC_OK;
+  return dmalloc((void **)&p->d_lwork, (size_t)kLagLargeChunk * p->nfft * sizeof(float2));
+}
+
 // task_scale (per task, may be null) multiplies the output scale of each row.
-// prod_src/prod_rec (one window, the compile-time lag plan only): xs are the
-// station spectra (rows of xpitch) and row r's stack is their product.
+// prod_src/prod_rec (one window; the compile-time lag plan, the half-length
+// and the four-step forms): xs are the station spectra (rows of xpitch) and row
+// r's stack is their product.
 static int xc_lags_rows(fxc_xc_plan *p, const float2 *xs, long long xpitch, long long nrows,
                         const int *row_out, float *d_cc, hipStream_t st,
                         const float *task_scale = nullptr, const int *prod_src = nullptr,
                         const int *prod_rec = nullptr) {
   if (nrows == 0) return FXC_OK;
   FXC_CHECK_ARG(!prod_src || p->large_lag || (p->d_fix_tw && xc_lag_r0_on()),
-                "xc: the one-window product form needs the compile-time or four-step lag");
+                "xc: the one-window product form needs the compile-time lag or a length beyond one "
+                "workgroup");
   const double weight0 = 1.0 / (double)((float)p->nfft * p->dt);
   if (p->large_lag && !p->half_lag) {
     // four-step inverse of the folded spectrum, kLagLargeChunk rows at a time
     const int M = p->nfft / 2;
     const LargeFft *lp = nullptr;
     FXC_TRY(large_plan(M, 1, &lp));
-    if (!p->d_lwork) FXC_TRY(dmalloc((void **)&p->d_lwork, (size_t)kLagLargeChunk * 2 * M * sizeof(float2)));
+    FXC_TRY(xc_lag_workspace(p));
     float2 *w0 = p->d_lwork, *w1 = p->d_lwork + (size_t)kLagLargeChunk * M;
     FXC_TRY(xc_mark(p, kTimeLag, true, st));
     for (long long r0 = 0; r0 < nrows; r0 += kLagLargeChunk) {
@@ -2670,7 +2678,7 @@ extern "C" int fxc_xc_lags(fxc_xc_plan *p, const float *d_xspec, long long nrows
 }
 
 // Full correlation: cc[task][0..2H] for every task set by fxc_xc_set_pairs.
-// One window at the compile-time lag length or a four-step one, every bin: a
+// One window at the compile-time lag length or one beyond one workgroup, every bin: a
 // pair's stack is the product conj(S[src]) S[rec] of its two spectra, formed
 // in FP32 as the lag synthesis reads them (the plan's operand form is not
 // used: there is no sum over windows to contract).
@@ -2690,6 +2698,7 @@ extern "C" int fxc_xc_correlate(fxc_xc_plan *p, const float *d_spec, float *d_cc
   long long maxrows = 0;
   FXC_TRY(fxc_xc_pairs_info(p, nullptr, nullptr, &maxrows));
   FXC_TRY(xc_ensure_workspace(p, (size_t)maxrows));
+  FXC_TRY(xc_lag_workspace(p));  // before the FP32 operand, which the call can do without
   FXC_TRY(xc_band_prepare(p, st));
   FXC_TRY(xc_prepare_spectra(p, (const float2 *)d_spec, st));
   const long long nc = (long long)p->chunk_tile_begin.size() - 1;
