@@ -1,6 +1,8 @@
 """Workgroup LDS FFT vs numpy (FP64), on the GPU; lengths whose transform
-exceeds one workgroup's LDS (complex 36000 and 37044, real 72000, 72576 and
-74088: the dt 0.05 s lengths) run the four-step transform over HBM."""
+exceeds one workgroup's LDS run in four steps over HBM (complex 36000 and
+37044; real lengths above about 80000, and shorter ones of few rows) or as two
+half-length LDS transforms (real 72000, 72576 and 74088: the dt 0.05 s
+lengths)."""
 import numpy as np
 import pytest
 
@@ -112,3 +114,24 @@ def test_few_long_rows_take_the_faster_form(gpu, monkeypatch):
     forced, own = best("1"), best(None)
     print(f"ten calls: halves {forced * 1e3:.3f} ms, own choice {own * 1e3:.3f} ms")
     assert own < 0.94 * forced
+
+
+@pytest.mark.parametrize("n,in_len,rows", [(81000, 81000, 2), (90000, 89999, 40), (92610, 90000, 3), (185220, 180000, 2)])
+def test_real_four_steps(gpu, n, in_len, rows):
+    """Real lengths beyond the two halves (50 Hz windows, two hours at 20 Hz): pack, columns, rows
+    and unfold over memory, and back, with zero padding and outputs cut short."""
+    import torch
+    from fastxc_amd import ops
+
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((rows, in_len)).astype(np.float32)
+    X = ops.fft_r2c(torch.from_numpy(x).to(gpu), n=n).cpu().numpy()
+    want = np.fft.rfft(x.astype(np.float64), n=n)
+    assert rel_l2(X, want) < 1e-6
+    assert np.all(X[:, 0].imag == 0) and np.all(X[:, -1].imag == 0)
+    z = (rng.standard_normal((rows, n // 2 + 1)) + 1j * rng.standard_normal((rows, n // 2 + 1)))
+    z = z.astype(np.complex64)
+    ref = np.fft.irfft(z.astype(np.complex128), n=n) * n
+    for out_len in (n, in_len, n // 2 + 1):
+        y = ops.fft_c2r(torch.from_numpy(z).to(gpu), n, out_len=out_len).cpu().numpy()
+        assert rel_l2(y, ref[:, :out_len]) < 1e-6

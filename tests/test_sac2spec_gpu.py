@@ -104,8 +104,9 @@ def test_production_lengths_one_station(gpu, tmp_path):
                                                         (1, 2, "0.1/2", 1), (0, 0, "0.1/2", 1)])
 def test_long_windows_dt005(gpu, tmp_path, whiten, normalize, bands, nch):
     """dt 0.05 s, one-hour windows: seg 72000, nfft_filter 72576, nfft_out
-    74088, whose transforms exceed one workgroup's LDS and run as four-step
-    transforms over HBM, against the FP64 oracle."""
+    74088, whose transforms exceed one workgroup's LDS, against the FP64 oracle
+    (few rows: four-step transforms over HBM; test_long_windows_forms has the
+    two halves)."""
     import torch
 
     path = str(tmp_path / "filter.txt")
@@ -253,3 +254,31 @@ def test_compensated_fp32_running_means(gpu, tmp_path, whiten, normalize):
     multi = _gpu_plan(plan, 3, whiten, normalize, 0)  # three channels: five-kernel path
     with pytest.raises(RuntimeError):
         multi.set_sums(True)
+
+
+@pytest.mark.parametrize("dt,halves", [(0.05, 1), (0.04, None)])
+@pytest.mark.parametrize("whiten,normalize,bands,nch", [
+    (2, 3, "0.1/2", 1), (3, 3, "0.1/2", 3), (3, 1, "0.1/0.5 0.5/2", 2), (1, 2, "0.1/2", 1), (2, 2, "0.1/2", 2),
+    (0, 3, "0.1/2", 2), (0, 1, "0.1/0.5 0.5/2", 1), (1, 0, "0.1/2", 3), (0, 0, "0.1/2", 1)])
+def test_long_windows_forms(gpu, tmp_path, monkeypatch, dt, halves, whiten, normalize, bands, nch):
+    """One-hour windows at 20 Hz with every transform as two halves in LDS, and at 25 Hz, where they
+    are too long for that and run in four steps over HBM with the normalisation, response, whitening
+    and output steps as passes of their own: every whitening order and normalisation against the
+    FP64 oracle."""
+    import torch
+
+    if halves is not None:
+        monkeypatch.setenv("FXC_FFT_HALVES", str(halves))
+    path = str(tmp_path / "filter.txt")
+    s2s.write_filter_file(path, dt, bands)
+    plan = s2s.plan_lengths(2 * 3600, dt, 3600, 3600, 100, s2s.read_filters(path))
+    assert plan.seg == (72000 if halves else 90000)
+    rng = np.random.default_rng(10 + 4 * whiten + normalize)
+    tr = _traces(rng, nch, plan.npts)
+    gp = _gpu_plan(plan, nch, whiten, normalize, 0)
+    out = gp.process(torch.from_numpy(tr).to(gpu), [0, 1]).cpu().numpy()
+    win = s2s.cut_windows(tr.astype(np.float64), plan, [0, 1])
+    want = s2s.process_batch(win.reshape(2, nch, plan.seg), plan, whiten, normalize, False).reshape(2, nch, -1)
+    err = rel_l2(out, want)
+    print(f"dt {dt} whiten={whiten} normalize={normalize} nch={nch} rel_l2={err:.3e}")
+    assert err < 1e-5

@@ -191,9 +191,9 @@ def test_one_window_product_form(gpu, precision):
 
 @pytest.mark.parametrize("precision", ["bf16x3", "fp32"])
 def test_one_window_product_form_dt005(gpu, precision):
-    """One window at nfft 74088 (dt 0.05 s): the four-step lag synthesis folds
-    the product conj(S[src]) S[rec] straight from the spectra; against FP64
-    and the PLAIN form, pairs in both orientations."""
+    """One window at nfft 74088 (dt 0.05 s): the lag synthesis of two half-length
+    transforms folds the product conj(S[src]) S[rec] straight from the spectra;
+    against FP64 and the PLAIN form, pairs in both orientations."""
     import torch
     from fastxc_amd.ops import XcPlan
 
@@ -246,7 +246,7 @@ def test_uneven_segments_with_gaps(gpu, precision):
 @pytest.mark.parametrize("precision", ["fp32", "bf16x3"])
 def test_long_nfft_dt005(gpu, precision):
     """nfft 74088 (dt 0.05 s, one-hour windows), 4001 lags: the lag synthesis
-    runs the four-step inverse transform; against FP64, lag order exact."""
+    runs two half-length transforms in LDS; against FP64, lag order exact."""
     import torch
     from fastxc_amd.ops import XcPlan
 
@@ -352,7 +352,7 @@ def test_fp32_matrix_tiles(gpu, nsta, nstep):
 def test_lag_halves(gpu, nfft, H):
     """Lag transforms of two half-length transforms: the shortest and longest lengths that take
     them, odd and even halves, no lag beside zero to every lag, odd row pitch; and the one-window
-    product form.  fp32 transforms of 2^16 points round to about log2(n) 2^-24 relative, 1e-6."""
+    product form.  80000 is just beyond them and takes the four steps over memory.  fp32 transforms of 2^16 points round to about log2(n) 2^-24 relative, 1e-6."""
     import torch
     from fastxc_amd.ops import XcPlan
 
@@ -459,3 +459,33 @@ def test_fp32_sparse_pairs_need_no_operand(gpu):
     held = free - torch.cuda.mem_get_info()[0]
     print(f"held {held} of {spec.numel() * 8} bytes of spectra")
     assert held < spec.numel() * 8 // 4
+
+
+@pytest.mark.parametrize("grid", [8, 256])
+@pytest.mark.parametrize("nstep", [1, 4, 8, 12, 16, 17, 20, 24, 28, 32, 36, 40, 41, 44, 48, 49, 52, 64])
+def test_fp32_every_depth(gpu, monkeypatch, grid, nstep):
+    """Every compiled depth of the FP32 matrix form (1 to 12 steps of 4 windows, and any depth
+    beyond), with its sources kept over runs of tiles and exchanged between them (8 workgroups, whose
+    runs are of 8 items) and with runs of one, tiles that list no pair of a receiver half or of a
+    source half, and a last bin chunk that is not full.  Bound as in test_fp32_matrix_tiles."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    monkeypatch.setenv("FXC_XC_F32", "matrix")
+    monkeypatch.setenv("FXC_XC_MFMA_GRID", str(grid))
+    nspec, nsta = 321, 110
+    rng = np.random.default_rng(nstep)
+    spec = (rng.standard_normal((nstep, nsta, nspec)) +
+            1j * rng.standard_normal((nstep, nsta, nspec))).astype(np.complex64)
+    src, rec = np.triu_indices(nsta, k=1)
+    keep = ~((rec >= 48) & (rec < 64)) & ~((src >= 64) & (src < 80))
+    src, rec = src[keep], rec[keep]
+    plan = XcPlan(nspec, nstep, 0.1, 20, "fp32")
+    plan.set_pairs(nsta, src, rec)
+    got = plan.cross_spectra(torch.from_numpy(spec).to(gpu)).cpu().numpy()
+    z = spec.astype(np.complex128)
+    for lo in range(0, len(src), 1000):
+        a, b = src[lo:lo + 1000], rec[lo:lo + 1000]
+        want = (z[:, a].conj() * z[:, b]).mean(axis=0)
+        bound = (np.abs(z[:, a]) * np.abs(z[:, b])).mean(axis=0) * (2 * nstep + 2) * 2.0 ** -24
+        assert (np.abs(got[lo:lo + 1000] - want) <= 2 * bound).all()
