@@ -122,15 +122,15 @@ __device__ __forceinline__ void flat_rows(int i0, int step, int n, int (&t)[kB],
 // (or a non-finite maximum).  The exponent stays within 126, where the scale and
 // its reciprocal are both normal: rows beyond are brought as near as that.
 __device__ __forceinline__ float pow2_scale(float mx) {
-  int e = 0;
-  if (mx > 0.f && isfinite(mx)) (void)frexpf(mx, &e);
-  return ldexpf(1.f, -max(-126, min(126, e)));
+  const unsigned e = __float_as_uint(mx) >> 23;  // mx >= 0: the exponent field
+  return mx == 0.f || e == 255 ? 1.f : __uint_as_float((253 - min(e, 252u)) << 23);
 }
 // Its inverse; 0 for an all-zero row, which then stays zero: what the transform
 // leaves in its part is the rounding of the row beside it, and a phase of that is
 // as large as any other.
 __device__ __forceinline__ float pow2_unscale(float mx) {
-  return mx == 0.f ? 0.f : 1.f / pow2_scale(mx);
+  const unsigned e = __float_as_uint(mx) >> 23;
+  return mx == 0.f ? 0.f : e == 255 ? 1.f : __uint_as_float((min(e, 252u) + 1) << 23);
 }
 
 // Loads of rows a kernel reads exactly once: nontemporal, so the twiddles
