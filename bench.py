@@ -314,7 +314,7 @@ def roofline(mode, args, npairs, default_workload):
     achieved = algorithmic bytes of the units one launch processes / the
     launch's average duration (HIP events on the launch stream)."""
     if mode["contract_ms"] >= mode["lag_ms"]:
-        name = {"fp32": "contract_fp32_kernel", "plain": "plain_accum_kernel"}.get(
+        name = {"fp32": "contract_f32_kernel", "plain": "plain_accum_kernel"}.get(
             mode["precision"], "contract_mfma_kernel")
         t = mode["contract_ms"] / max(mode["contract_launches_per_step"], 1)
         launches = max(mode["contract_launches_per_step"], 1)

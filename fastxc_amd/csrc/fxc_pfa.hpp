@@ -175,8 +175,11 @@ struct PfaTables {
   float2 *d_phase = nullptr;
 };
 // Whether n is a product of distinct radices among 2 or 4, 3, 5, 7, 23 and 29
-// (one axis each, small butterflies first).  Axes of 8, 9 and 16 would cost the
-// kernels' registers for lengths that hardly occur.
+// (one axis each, small butterflies first): few lengths, of the odd ones from 201
+// to 4001 these 12: 203, 345, 435, 483, 609, 667, 805, 1015, 2001, 2415, 3045,
+// 3335.  Axes of 8, 9, 16 and 25, and the primes 11 to 19 and 31, whose folded
+// form fits the matrix pass, are not tried; other lengths keep the kernels of
+// fxc_stack_fft.hpp's transforms.
 bool pfa_length(int n);
 int pfa_tables(int n, PfaTables *out, bool create = true);
 void pfa_release();

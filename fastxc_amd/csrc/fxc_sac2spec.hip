@@ -1510,7 +1510,7 @@ s2s_back_kernel(float2 *X, long long fpitch, int seg, int i1, int i2, int i3, in
 // LDS work of the transforms is what each kernel costs, and a runtime plan's
 // index arithmetic is most of that (29 against 12 us per transform of 18000
 // points).  14100 rows of three-channel frames: prefilter 3.54 -> 2.46 ms, row
-// 2.29 -> 1.70 ms, shared with the output transform 4.19 -> 2.53 ms.
+// 2.29 -> 1.76 ms, shared with the output transform 4.19 -> 2.65 ms.
 // ---------------------------------------------------------------------------
 template <class FPF>
 __global__ void __launch_bounds__(kS2sThreads)
@@ -1823,7 +1823,7 @@ extern "C" int fxc_s2s_plan_create(fxc_s2s_plan **out, const fxc_s2s_config *cfg
     const int need = std::max(std::max(need_f, need_s), std::max(need_o, need_so));
     large = need > kLdsComplexCapacity;
     if (large) {
-      // every transform of the plan runs as a four-step transform over HBM
+      // every transform of the plan is a long one (two halves in LDS or four steps over HBM)
       int a = 0, b = 0;
       for (int M : {Mf, Ms, Mo})
         FXC_CHECK_ARG(large_factor(M, &a, &b),

@@ -37,7 +37,7 @@ namespace fxc {
 
 constexpr int kStkThreads = 256;
 constexpr int kStkBatch = 4;       // transforms held in LDS at once (at most)
-constexpr int kVoiceThreads = 512; // PWS and TF-PWS voice workgroups
+constexpr int kVoiceThreads = 512; // TF-PWS voice workgroups
 
 // Analytic spectra of real rows: A[k] = 2 X[k] for 1 <= k < (n+1)/2, else 0
 // (hilbertTransformKernel after R2C).  Output natural order, [rows][n].

@@ -228,8 +228,8 @@ int tfpws_pfa_run(const StackFft &S, const float2 *Ag, const float2 *Alin, const
   FXC_TRY(pfa_tables(n, &a.t));
   long long most = 0;
   for (int i = 0; i < npairs; ++i) most = std::max(most, h_off[i + 1] - h_off[i]);
-  // a pair's groups and linear stack in one batch: up to 5 rows of 6 bins per
-  // thread (60 registers) stay held
+  // a pair's groups and linear stack in one batch: up to 5 rows of 4 bins per
+  // thread (40 registers) stay held; longer lengths read the rows again per voice
   const bool held = most < nrows && most <= nbatch && nrows <= kPfaMaxRows;
   if (n <= 1024) return pfa_launch<256, 4>(S, a, held, st);
   if (n <= 2048) return pfa_launch<512, 4>(S, a, held, st);

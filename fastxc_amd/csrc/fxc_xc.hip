@@ -1818,7 +1818,7 @@ struct fxc_xc_plan {
   // for the first band_zero_rows rows
   int band_c0 = 0, band_c1 = -1;
   size_t band_zero_rows = 0;
-  // nfft/2 beyond one workgroup's LDS: lag synthesis by the four-step
+  // nfft/2 beyond one workgroup's LDS: lag synthesis by half_lag, or the four-step
   // inverse transform (work buffer for kLagLargeChunk rows)
   bool large_lag = false;
   // (even nfft/2 whose half fits: two transforms in LDS, no work buffer)

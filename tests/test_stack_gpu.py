@@ -328,20 +328,17 @@ def test_zero_rows_have_no_phase(gpu, kind, n):
         assert rel_l2(got[p], want) < (1e-5 if kind == "pws" else 1e-4)
     assert not got[2].any()
 
-@pytest.mark.parametrize("kind", ["pws", "tfpws"])
 @pytest.mark.parametrize("n", [2001, 2000, 512, 345, 2003, 1006])
-@pytest.mark.parametrize("size", [1e-40, 3e-39, 1.2e38, 2e38])
-def test_stacks_with_rows_at_the_ends_of_the_range(gpu, kind, n, size):
+@pytest.mark.parametrize("kind,size", [("pws", 1e-40), ("pws", 3e-39), ("pws", 1.2e38), ("pws", 2e38),
+                                       ("tfpws", 1e-40), ("tfpws", 3e-39)])
+def test_stacks_with_rows_at_the_ends_of_the_range(gpu, kind, size, n):
     """A finite row of subnormal size, or one (of constant envelope) whose square overflows, beside
     ordinary rows: the stack stays finite, and is that with the row left at zero (a subnormal row
     adds 1e-31 of the others; the phase of an overflowing one is zero) for every form of the
-    transform.  The time-frequency stack of the large row is not compared: its spectrum
-    overflows."""
+    transform.  (A time-frequency stack's spectrum of the large row overflows.)"""
     import torch
     from fastxc_amd import ops
 
-    if kind == "tfpws" and size > 1:
-        pytest.skip("the spectrum of such a row is not finite")
     rng = np.random.default_rng(n)
     x = rng.standard_normal((5, n)).astype(np.float32)
     for r in (1, 4):
