@@ -257,10 +257,29 @@ __device__ __forceinline__ float2 tw_lookup(const float2 *tw, int e) {
 // 16, where the table's rounding would grow fifteenfold along a chain, they are
 // w^(4a + b) = (w^4)^a w^b from the table's w and w^4 (rms error of the powers
 // of radix 15 at 18000 points 9.6e-8 against 2.7e-7); larger radices read each
-// power.
-template <int R>
+// power.  kTwoReads: radices 4 to 9 form w^(3a + b) = (w^3)^a w^b from the table's
+// w and w^3, which halves the rounding of a transform of five such passes (18522
+// points 2.5e-7 against 1.4e-7).
+template <int R, bool kTwoReads>
 __device__ __forceinline__ void apply_twiddles(float2 *v, const float2 *tw, int e, int n) {
-  if constexpr (R <= 9) {
+  if constexpr (kTwoReads && R >= 4 && R <= 9) {
+    const float2 w1 = tw_lookup(tw, e);
+    int e3 = 2 * e;
+    if (e3 >= n) e3 -= n;
+    e3 += e;
+    if (e3 >= n) e3 -= n;
+    const float2 w3 = tw_lookup(tw, e3), w2 = cmul(w1, w1);
+    v[1] = cmul(v[1], w1);
+    v[2] = cmul(v[2], w2);
+    float2 wa = w3;
+#pragma unroll
+    for (int q = 3; q < R; q += 3) {
+      v[q] = cmul(v[q], wa);
+      if (q + 1 < R) v[q + 1] = cmul(v[q + 1], cmul(wa, w1));
+      if (q + 2 < R) v[q + 2] = cmul(v[q + 2], cmul(wa, w2));
+      if (q + 3 < R) wa = cmul(wa, w3);
+    }
+  } else if constexpr (R <= 9) {
     const float2 w = tw_lookup(tw, e);
     float2 wq = w;
     v[1] = cmul(v[1], w);
@@ -322,7 +341,7 @@ struct FlatWalk {
 };
 
 // One in-place DIF pass (butterfly, then twiddle) over ntrans transforms.
-template <int R>
+template <int R, bool kTwoReads = false>
 __device__ __forceinline__ void dif_pass(float2 *buf, int ntrans, const FftPlanDev &plan, int p,
                                          const float2 *tw, float sgn, int tid, int nthr) {
   const int n = plan.n;
@@ -371,7 +390,7 @@ __device__ __forceinline__ void dif_pass(float2 *buf, int ntrans, const FftPlanD
       });
     } else {
       dft<R>(v, sgn);
-      if (j > 0) apply_twiddles<R>(v, tw, j * tstep, n);
+      if (j > 0) apply_twiddles<R, kTwoReads>(v, tw, j * tstep, n);
       float2 *obase = base;
       if constexpr (R >= 12) {  // as above, for the large composite butterflies
         int off = t * n + blk * span + j;
@@ -383,6 +402,12 @@ __device__ __forceinline__ void dif_pass(float2 *buf, int ntrans, const FftPlanD
     }
   }
   __syncthreads();
+}
+
+template <int R>
+__device__ __forceinline__ void dif_pass_two(float2 *buf, int ntrans, const FftPlanDev &plan, int p,
+                                             const float2 *tw, float sgn, int tid, int nthr) {
+  dif_pass<R, true>(buf, ntrans, plan, p, tw, sgn, tid, nthr);
 }
 
 // One in-place DIT pass (twiddle, then butterfly): the exact inverse
@@ -407,7 +432,7 @@ __device__ __forceinline__ void dit_pass(float2 *buf, int ntrans, const FftPlanD
     float2 v[R];
 #pragma unroll
     for (int m = 0; m < R; ++m) v[m] = base[m * stride];
-    if (j > 0) apply_twiddles<R>(v, tw, j * tstep, n);
+    if (j > 0) apply_twiddles<R, false>(v, tw, j * tstep, n);
     if constexpr (kStreamRadix<R>) {
       int off = t * n + blk * span + j;  // see dif_pass
       asm volatile("" : "+v"(off));
@@ -491,22 +516,29 @@ __device__ __forceinline__ void lds_fft(float2 *buf, int ntrans, const FftPlanDe
 // span R = radix[P-1] contiguous values holds the input of an R-point DFT
 // whose output t is bin k = lower + (n/R) t, where the block starts at the
 // digit-reversed position of lower = k mod (n/R) (see last_pass_bin).
-template <unsigned kMask = kRadixSmooth>
+// kTwoReads: see apply_twiddles.
+template <unsigned kMask = kRadixSmooth, bool kTwoReads = false>
 __device__ __forceinline__ void lds_fft_head(float2 *buf, int ntrans, const FftPlanDev &plan,
                                     const float2 *tw, float sgn, int npass_run) {
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   for (int p = 0; p < npass_run; ++p) {
-    FXC_RADIX_SWITCH(dif_pass)
+    if constexpr (kTwoReads) {
+      FXC_RADIX_SWITCH(dif_pass_two)
+    } else {
+      FXC_RADIX_SWITCH(dif_pass)
+    }
   }
 }
 
 // Bin k of a transform whose last pass was left out (lds_fft_head with
 // npass_run = P-1): the direct R-point DFT of its block,
 //   Z[k] = sum_{m<R} buf[base + m] w_R^(m t),  w_R = w_n^(n/R),
-// with the powers w_R^(m t) re-read from the table every 8 terms.
+// with the powers w_R^(m t) re-read from the table every 8 terms, or (kRoots) from
+// roots[u] = w_R^u, u < R: the chain's rounding is that of a pass.
+template <bool kRoots = false>
 __device__ inline float2 last_pass_bin(const float2 *buf, const FftPlanDev &plan,
-                                       const float2 *tw, int k) {
+                                       const float2 *tw, int k, const float2 *roots = nullptr) {
   const int P = plan.npass;
   if (P == 0) return buf[0];
   const int R = plan.radix[P - 1];
@@ -520,7 +552,7 @@ __device__ inline float2 last_pass_bin(const float2 *buf, const FftPlanDev &plan
     base += (lower - q * r) * plan.stride[p];
     lower = q;
   }
-  const float2 wt = tw_lookup(tw, t * g);
+  const float2 wt = kRoots ? roots[t] : tw_lookup(tw, t * g);
   float2 z = buf[base];
   float2 wm = wt;
   int e = t;  // (m t) mod R for m = 1
@@ -530,7 +562,7 @@ __device__ inline float2 last_pass_bin(const float2 *buf, const FftPlanDev &plan
     z.y += v.x * wm.y + v.y * wm.x;
     e += t;
     if (e >= R) e -= R;
-    wm = ((m + 1) & 7) == 0 ? tw_lookup(tw, e * g) : cmul(wm, wt);
+    wm = kRoots ? roots[e] : ((m + 1) & 7) == 0 ? tw_lookup(tw, e * g) : cmul(wm, wt);
   }
   return z;
 }

@@ -1287,6 +1287,7 @@ contract_f32_kernel(const float2 *__restrict__ op, int nsta, int nspec, int step
 constexpr int kLagThreads = 1024;
 constexpr long long kLagLargeChunk = 2048;  // rows per four-step lag call
 constexpr int kLagMaxRadixDefault = 9;
+constexpr int kLagRoots = 16;  // LDS slots of the last pass' roots (two-half form)
 constexpr unsigned kRadixLag8 = (1u << 2) | (1u << 3) | (1u << 4) | (1u << 5) | (1u << 6) | (1u << 7) | (1u << 8);
 constexpr unsigned kRadixLag9 = kRadixLag8 | (1u << 9);
 constexpr int kLagRegs = (kLdsComplexCapacity + kLagThreads - 1) / kLagThreads;
@@ -1340,6 +1341,15 @@ lag_kernel(const float2 *__restrict__ xspec, long long xpitch, long long nrows,
   stage_real_tables(lds, plan, tw, fold);
   const float2 *twl = lds + M + 1;
   const float2 *fl = twl + tw_lds_count(M);
+  float2 *roots = lds + real_lds_count(M);  // kHalf: exp(2 pi i u / R) of the last pass
+  if constexpr (kHalf) {
+    const int R = plan.radix[plan.npass - 1];
+    if ((int)threadIdx.x < R) {  // read after the passes' barriers
+      double c, d;
+      sincospi(2.0 * threadIdx.x / R, &d, &c);
+      roots[threadIdx.x] = make_float2((float)c, (float)d);
+    }
+  }
   float2 pre[kLagRegs];
   auto prefetch = [&](long long r, int part) {
     if constexpr (kProd)
@@ -1384,7 +1394,7 @@ lag_kernel(const float2 *__restrict__ xspec, long long xpitch, long long nrows,
       __syncthreads();
       // all passes but the last; the last (largest radix, stride 1) is
       // evaluated only for the bins that hold kept lags
-      lds_fft_head<kRadixLag>(lds, 1, plan, twl, 1.f, plan.npass - 1);
+      lds_fft_head<kRadixLag, kHalf>(lds, 1, plan, twl, 1.f, plan.npass - 1);
       const int out_row = row_out ? row_out[row] : (int)row;
       float *y = cc + (size_t)out_row * (2 * half_cc + 1);
       const double wr = task_scale ? weight * (double)task_scale[out_row] : weight;
@@ -1392,7 +1402,7 @@ lag_kernel(const float2 *__restrict__ xspec, long long xpitch, long long nrows,
       const int n_lo = -((half_cc + 1) / 2), n_hi = half_cc / 2;
       for (int i = threadIdx.x; i <= n_hi - n_lo; i += blockDim.x) {
         const int n = n_lo + i;
-        float2 z = last_pass_bin(lds, plan, twl, n < 0 ? n + M : n);
+        float2 z = last_pass_bin<kHalf>(lds, plan, twl, n < 0 ? n + M : n, roots);
         const int m0 = 2 * n + half_cc;
         const bool in0 = m0 >= 0, in1 = m0 + 1 <= 2 * half_cc;
         if (kHalf && part == 0) {
@@ -1927,7 +1937,8 @@ extern "C" int fxc_xc_plan_create(fxc_xc_plan **out, int nspec, int nstep, float
   if (const char *env = getenv("FXC_XC_LAG_MAX_RADIX")) lag_max_radix = atoi(env) >= 9 ? 9 : 8;
   const bool large_lag = real_lds_count(nfft / 2) > kLdsComplexCapacity;
   // two transforms of nfft/4 in LDS, where that length fits and factors
-  bool half_lag = large_lag && nfft % 4 == 0 && real_lds_count(nfft / 4) <= kLdsComplexCapacity;
+  bool half_lag = large_lag && nfft % 4 == 0 &&
+                  real_lds_count(nfft / 4) + kLagRoots <= kLdsComplexCapacity;
   if (half_lag) {
     int radix[kMaxPasses], np = 0;
     half_lag = factor_radices(nfft / 4, radix, &np, lag_max_radix, true) && radix[np - 1] <= 9;
@@ -2589,7 +2600,8 @@ static int xc_lags_rows(fxc_xc_plan *p, const float2 *xs, long long xpitch, long
   const int nreal = p->half_lag ? p->nfft / 2 : p->nfft;  // real length of one LDS transform
   const RealFftPlan *rp = nullptr;
   FXC_TRY(plan_cache_real(nreal, 1, &rp, p->lag_max_radix, true));
-  const size_t lds = (size_t)real_lds_count(nreal / 2) * sizeof(float2);
+  const size_t lds =
+      (size_t)(real_lds_count(nreal / 2) + (p->half_lag ? kLagRoots : 0)) * sizeof(float2);
   const bool r9 = p->lag_max_radix >= 9;
   auto kern = r9 ? lag_kernel<kRadixLag9, false, false> : lag_kernel<kRadixLag8, false, false>;
   if (p->half_lag && prod_src)

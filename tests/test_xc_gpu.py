@@ -489,3 +489,24 @@ def test_fp32_every_depth(gpu, monkeypatch, grid, nstep):
         want = (z[:, a].conj() * z[:, b]).mean(axis=0)
         bound = (np.abs(z[:, a]) * np.abs(z[:, b])).mean(axis=0) * (2 * nstep + 2) * 2.0 ** -24
         assert (np.abs(got[lo:lo + 1000] - want) <= 2 * bound).all()
+
+
+@pytest.mark.parametrize("nfft", [72576, 72900, 73500, 74088, 75000])
+def test_long_lags_keep_their_precision(gpu, nfft):
+    """Lags of lengths beyond one workgroup (20 Hz windows with 25 to 110 s of lags): two half-length
+    transforms of five or six passes round to 1.8 to 2.0e-7 of white spectra's lags with powers of at
+    most three products of table values; powers chained from one value give 2.6 to 3.1e-7, the four
+    steps they replace 1.7 to 2.7e-7."""
+    import torch
+    from fastxc_amd.ops import XcPlan
+
+    H, dt = 2000, 0.05
+    g = torch.Generator(device=gpu)
+    g.manual_seed(nfft)
+    X = torch.randn((48, nfft // 2 + 1), generator=g, device=gpu, dtype=torch.complex64)
+    got = XcPlan(nfft // 2 + 1, 2, dt, H, "fp32").lags(X).double()
+    lag = torch.arange(-H, H + 1, device=gpu) % nfft
+    want = torch.fft.irfft(X.to(torch.complex128), n=nfft)[:, lag] / float(np.float32(dt))
+    err = float(torch.linalg.vector_norm(got - want) / torch.linalg.vector_norm(want))
+    print(f"nfft {nfft} rel_l2={err:.3e}")
+    assert err < 2.3e-7
