@@ -959,11 +959,11 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
 // Bound: fp32 matrix issue (8 x bins x windows x pairs flops at the ~147
 // TFLOP/s a large fp32 product reaches), then operand reads that miss an XCD's
 // L2 (600 stations x 47 windows: 3.7 MB per 16-bin chunk, 22 GB read per call)
-// and the 8-byte-per-bin result writes.  600 x 47 x 18523 bins: transpose 1.8
-// ms + contraction 14.7 ms (matrix pipe busy 65 %) against 33.7 ms for the
+// and the 8-byte-per-bin result writes.  600 x 47 x 18523 bins: transpose 2.0
+// ms + contraction 14.3 ms (13.7 with both products in one sum) against 33.7 ms for the
 // vector-ALU form it replaced, which issued the same flops at half the rate
 // and re-read station rows with 8 x 8 pairs per thread; 8 stations x 24
-// windows 17 + 27 us against 85 us.
+// windows 17 + 28 us against 85 us.
 // ---------------------------------------------------------------------------
 constexpr int kF32Group = 4;     // windows per matrix step
 constexpr int kF32TrThreads = 256;
@@ -1009,25 +1009,49 @@ f32_transpose_kernel(const float2 *__restrict__ spec, int nstep, int nsta, int n
   }
 }
 
+// Sums of one bin and phase: Re and Im of the blocks' pairs.  kTwo: the two
+// products of each part go into sums of their own, joined at the end, so that a
+// sum takes one rounding per window, as the vector form's does; with both in one
+// chain 24 windows are off by 1.31e-7 where the vector form is by 1.04e-7.
+template <bool kTwo>
+struct F32Sums {
+  f32x4_t re[2], im[2], re2[kTwo ? 2 : 1], im2[kTwo ? 2 : 1];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int si = 0; si < 2; ++si) {
+      re[si] = im[si] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kTwo) re2[si] = im2[si] = re[si];
+    }
+  }
+  __device__ __forceinline__ float2 value(int si, int r) const {
+    if constexpr (kTwo) return make_float2(re[si][r] + re2[si][r], im[si][r] + im2[si][r]);
+    return make_float2(re[si][r], im[si][r]);
+  }
+};
+
 // One matrix step (4 windows) of 32 source stations x 16 receivers (bit si of
 // kMask: source half si is listed).  The instructions of the two blocks are
 // interleaved, so that none waits for the accumulator of the one before it.
-template <int kMask>
-__device__ __forceinline__ void f32_step(const float2 (&s)[2], float2 r, f32x4_t (&cr)[2],
-                                         f32x4_t (&ci)[2]) {
+template <int kMask, bool kTwo>
+__device__ __forceinline__ void f32_step(const float2 (&s)[2], float2 r, F32Sums<kTwo> &c) {
 #pragma unroll
   for (int si = 0; si < 2; ++si)
     if ((kMask >> si) & 1) {
-      cr[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.x, cr[si], 0, 0, 0);
-      ci[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.y, ci[si], 0, 0, 0);
+      c.re[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.x, c.re[si], 0, 0, 0);
+      c.im[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].x, r.y, c.im[si], 0, 0, 0);
     }
 #pragma unroll
   for (int si = 0; si < 2; ++si)
     if ((kMask >> si) & 1) {
-      cr[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].y, r.y, cr[si], 0, 0, 0);
-      ci[si] = __builtin_amdgcn_mfma_f32_16x16x4f32(-s[si].y, r.x, ci[si], 0, 0, 0);
+      f32x4_t &re = kTwo ? c.re2[kTwo ? si : 0] : c.re[si], &im = kTwo ? c.im2[kTwo ? si : 0] : c.im[si];
+      re = __builtin_amdgcn_mfma_f32_16x16x4f32(s[si].y, r.y, re, 0, 0, 0);
+      im = __builtin_amdgcn_mfma_f32_16x16x4f32(-s[si].y, r.x, im, 0, 0, 0);
     }
 }
+
+// Depth to which the registers hold two sums; deeper ones leave the first half of
+// the windows' sum in LDS and add the second.
+constexpr int kF32TwoSums = 8;
 
 // Steps loaded ahead of their use (fewer where the sources fill the registers).
 constexpr int kF32Ahead = 6;
@@ -1052,18 +1076,32 @@ __device__ __forceinline__ void f32_bin(const float2 (&src)[kSteps > 0 ? kSteps 
                                         const float2 *__restrict__ sp, const unsigned (&so)[2],
                                         int steps, size_t step_elems, float scale, int b,
                                         int lane_r, int lane_g, float2 *stage) {
-  f32x4_t cr[2], ci[2];
+  constexpr bool kTwo = kSteps <= kF32TwoSums;
+  F32Sums<kTwo> c;
+  c.clear();
+  // pair (16 si + 4 lane_g + r, lane_r), whose low four bits are lane_r
+  float2 *o = stage + stage_index(4 * lane_g * 16 + lane_r, b);
+  auto each = [&](auto f) {
 #pragma unroll
-  for (int si = 0; si < 2; ++si) cr[si] = ci[si] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int si = 0; si < 2; ++si) {
+      if (!((kMask >> si) & 1)) continue;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) f(o[(16 * si + r) * 16 * kBinChunk], c.value(si, r));
+    }
+  };
   if constexpr (kSteps > 0) {
     constexpr int kD = f32_ahead(kSteps);
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
+      if (!kTwo && s == kSteps / 2) {  // the first half waits in its place
+        each([](float2 &p, float2 v) { p = v; });
+        c.clear();
+      }
       const float2 r = ring[s % kD];
       ring[s % kD] = s + kD < kSteps ? (cur.p + (s + kD) * step_elems)[cur.off]
                                      : (nxt.p + (s + kD - kSteps) * step_elems)[nxt.off];
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
-      f32_step<kMask>(src[s], r, cr, ci);
+      f32_step<kMask>(src[s], r, c);
     }
     // the next bin's step i sits at (kSteps + i) % kD
     float2 t[kD];
@@ -1089,19 +1127,14 @@ __device__ __forceinline__ void f32_bin(const float2 (&src)[kSteps > 0 ? kSteps 
         const float2 ai[2] = {a[i][0], a[i][1]}, ri = r[i];
         load(i, s0 + kD + i);
         __builtin_amdgcn_sched_barrier(0);
-        if (s0 + i < steps) f32_step<kMask>(ai, ri, cr, ci);
+        if (s0 + i < steps) f32_step<kMask>(ai, ri, c);
       }
     }
   }
-  // pair (16 si + 4 lane_g + r, lane_r), whose low four bits are lane_r
-  float2 *o = stage + stage_index(4 * lane_g * 16 + lane_r, b);
-#pragma unroll
-  for (int si = 0; si < 2; ++si) {
-    if (!((kMask >> si) & 1)) continue;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      o[(16 * si + r) * 16 * kBinChunk] = make_float2(cr[si][r] * scale, ci[si][r] * scale);
-  }
+  each([&](float2 &p, float2 v) {
+    if constexpr (!kTwo) v = cadd(v, p);
+    p = make_float2(v.x * scale, v.y * scale);
+  });
 }
 
 // Work items and order as contract_mfma_kernel: a 32 x 32 station tile x 16
