@@ -501,14 +501,19 @@ constexpr unsigned kRadixAll = kRadixSmooth | (1u << 23) | (1u << 29);
     default: break;                                                           \
   }
 
-// Natural-order input -> digit-reversed output (tw: LDS twiddle table).
-template <unsigned kMask = kRadixSmooth>
+// Natural-order input -> digit-reversed output (tw: LDS twiddle table;
+// kTwoReads: see apply_twiddles).
+template <unsigned kMask = kRadixSmooth, bool kTwoReads = false>
 __device__ __forceinline__ void lds_fft(float2 *buf, int ntrans, const FftPlanDev &plan, const float2 *tw,
                                float sgn) {
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   for (int p = 0; p < plan.npass; ++p) {
-    FXC_RADIX_SWITCH(dif_pass)
+    if constexpr (kTwoReads) {
+      FXC_RADIX_SWITCH(dif_pass_two)
+    } else {
+      FXC_RADIX_SWITCH(dif_pass)
+    }
   }
 }
 

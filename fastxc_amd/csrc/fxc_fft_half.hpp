@@ -70,7 +70,7 @@ half_r2c_kernel(const float *__restrict__ in, long long in_dist, int in_len, lon
                              a + 1 < in_len ? sample(row, a + 1, x[a + 1]) : 0.f);
       }
       __syncthreads();
-      lds_fft<kMask>(lds, 1, plan, twl, -1.f);
+      lds_fft<kMask, true>(lds, 1, plan, twl, -1.f);
       if (part == 0)
         for (int k = tid; k < Q; k += kHalfThreads) E[k] = lds[fft_pos(plan, k)];
     }
@@ -138,7 +138,7 @@ half_c2r_kernel(const float2 *__restrict__ in, long long in_dist, long long rows
         }
       }
       __syncthreads();
-      lds_fft<kMask>(lds, 1, plan, twl, 1.f);
+      lds_fft<kMask, true>(lds, 1, plan, twl, 1.f);
       if (part == 0)
         for (int n = tid; n < Q; n += kHalfThreads) F[n] = lds[fft_pos(plan, n)];
     }
