@@ -960,7 +960,7 @@ contract_mfma_kernel(const unsigned short *__restrict__ hi, const unsigned short
 // TFLOP/s a large fp32 product reaches), then operand reads that miss an XCD's
 // L2 (600 stations x 47 windows: 3.7 MB per 16-bin chunk, 22 GB read per call)
 // and the 8-byte-per-bin result writes.  600 x 47 x 18523 bins: transpose 2.0
-// ms + contraction 14.3 ms (13.7 with both products in one sum) against 33.7 ms for the
+// ms + contraction 14.2 ms (13.8 with both products in one sum) against 33.7 ms for the
 // vector-ALU form it replaced, which issued the same flops at half the rate
 // and re-read station rows with 8 x 8 pairs per thread; 8 stations x 24
 // windows 17 + 28 us against 85 us.
@@ -1093,15 +1093,20 @@ __device__ __forceinline__ void f32_bin(const float2 (&src)[kSteps > 0 ? kSteps 
     constexpr int kD = f32_ahead(kSteps);
 #pragma unroll
     for (int s = 0; s < kSteps; ++s) {
-      if (!kTwo && s == kSteps / 2) {  // the first half waits in its place
-        each([](float2 &p, float2 v) { p = v; });
-        c.clear();
-      }
       const float2 r = ring[s % kD];
       ring[s % kD] = s + kD < kSteps ? (cur.p + (s + kD) * step_elems)[cur.off]
                                      : (nxt.p + (s + kD - kSteps) * step_elems)[nxt.off];
       __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
-      f32_step<kMask>(src[s], r, c);
+      if (!kTwo && s == kSteps / 2) {
+        // the first half waits in its place, written behind the second's first step
+        F32Sums<kTwo> d;
+        d.clear();
+        f32_step<kMask>(src[s], r, d);
+        each([](float2 &p, float2 v) { p = v; });
+        c = d;
+      } else {
+        f32_step<kMask>(src[s], r, c);
+      }
     }
     // the next bin's step i sits at (kSteps + i) % kD
     float2 t[kD];
